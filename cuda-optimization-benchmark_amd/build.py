@@ -51,6 +51,7 @@ KERNEL_SOURCES = [
     "reward_to_go.hip",
     "leaky.hip",
     "efficient_kan.hip",
+    "efficient_kan_direct.hip",
     "fp8_linear.hip",
     "quantize_e4m3.hip",
 ]

@@ -87,8 +87,9 @@ def load_counter(path: str | Path | None = None) -> Counter:
 EXPECTED_LAUNCHES = {
     "pow_abs_sqrt_mean": 1, "leaky": 1, "reward_to_go": 1, "ppo_clip": 1, "ppo_clip_entropy": 1,
     "ppo_clip_entropy_noalloc": 1,  # its first call on a device adds the scratch clear
-    "efficient_kan": 2,          # kan_pack + kan_fused (spline order 3)
-    "efficient_kan_rowwise": 1,  # kan_rowwise (other spline orders)
+    "efficient_kan": 2,          # kan_pack + kan_fused, or kan_direct + kan_direct_sum
+    "efficient_kan_one_chunk": 1,  # kan_direct alone: the features are not split
+    "efficient_kan_rowwise": 1,  # kan_rowwise (spline order 0 or above 4)
     "fp8_linear": 1,
     "quantize_e4m3": 2,          # qz_amax + qz_cast (unaligned, or more chunks than fit at once)
     "quantize_e4m3_fused": 1,    # qz_fused (aligned, every chunk resident at once)
@@ -97,8 +98,8 @@ EXPECTED_LAUNCHES = {
 
 def workloads():
     """(name, entry point, expectation key, make_args) for every hidden and public case of
-    the six ops, the entropy variant of ppo_clip (allocating and not), the row-wise
-    efficient_kan path and the quantiser (aligned and unaligned)."""
+    the six ops, the entropy variant of ppo_clip (allocating and not), efficient_kan's
+    other spline orders and the quantiser (aligned and unaligned)."""
     import torch
     from cob_amd import capi, inputs, tasks
 
@@ -131,19 +132,19 @@ def workloads():
     for op in tasks.OPS:
         for case in tasks.all_cases(op):
             key = op
-            if op == "efficient_kan" and case.get("spline_order", 3) != 3:
-                key = "efficient_kan_rowwise"
+            if op == "efficient_kan" and case["B"] <= 16 and case["I"] <= 16:
+                key = "efficient_kan_one_chunk"
             out.append((f"{op}/{case['name']}", op, key, drop_in(op, case)))
             if op == "ppo_clip":
                 out.append((f"ppo_clip_entropy/{case['name']}", "ppo_clip_entropy", "ppo_clip_entropy",
                             drop_in(op, case, entropy=True)))
                 out.append((f"ppo_clip_entropy_noalloc/{case['name']}", "ppo_clip_entropy_noalloc",
                             "ppo_clip_entropy_noalloc", drop_in(op, case, entropy=True)))
-    for order in (1, 2):
+    for order in (1, 2, 5):
         case = dict(name=f"B64_I40_O24_order{order}", seed=70 + order, small=True, timed=False,
                     B=64, I=40, O=24, spline_order=order)
-        out.append((f"efficient_kan/{case['name']}", "efficient_kan", "efficient_kan_rowwise",
-                    drop_in("efficient_kan", case)))
+        out.append((f"efficient_kan/{case['name']}", "efficient_kan",
+                    "efficient_kan_rowwise" if order > 4 else "efficient_kan", drop_in("efficient_kan", case)))
     out.append(("quantize_e4m3/aligned_n1000003", "quantize_e4m3", "quantize_e4m3_fused", quant(1_000_003, 0)))
     # 4096 x 4096, the fused path's whole resident capacity: still one launch.
     out.append(("quantize_e4m3/aligned_n16777216", "quantize_e4m3", "quantize_e4m3_fused", quant(1 << 24, 0)))

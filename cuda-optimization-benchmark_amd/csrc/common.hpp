@@ -156,6 +156,11 @@ enum WorkspaceSlot : int {
 // caller's launches.
 hipError_t workspace(WorkspaceSlot slot, size_t bytes, hipStream_t stream, void** out);
 
+// workspace(), except that a region too small is left as it is (possibly empty) while `stream`
+// is capturing, where nothing may be allocated; *have is the region's size.  For callers that
+// can do with less.
+hipError_t workspace_if_possible(WorkspaceSlot slot, size_t bytes, hipStream_t stream, void** out, size_t* have);
+
 // Number of compute units of the current device (cached per device).
 int device_cu_count();
 

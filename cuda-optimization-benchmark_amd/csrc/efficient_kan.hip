@@ -1,15 +1,27 @@
 // efficient_kan on gfx950: KANLinear forward.
 //
 // Drop-in signature tasks/efficient_kan/tests/task.json:3, replacing
-// reference/efficient_kan/solution.cu:177-288.  Fast path (efficient_kan.hpp): spline
-// order 3 with at most 16 knots per feature — kan_pack (column scales, the scaled fp16
-// hi/lo weights in the GEMM's K order, basis tables) and the warp-specialized fp16x3 MFMA
-// GEMM kan_fused.  Other shapes take the row-wise fp32 path below.
+// reference/efficient_kan/solution.cu:177-288.  Three paths:
+//  * fast (efficient_kan.hpp): spline order 3 with at most 16 knots per feature — kan_pack
+//    (column scales, the scaled fp16 hi/lo weights in the GEMM's K order, basis tables) and
+//    the warp-specialized fp16x3 MFMA GEMM kan_fused;
+//  * direct (efficient_kan_direct.hpp): spline orders 1 .. 4 in fp32 MFMAs on the weights as
+//    they lie — other orders and finer knot grids, and the batches too small to pay for the
+//    packing (direct_is_faster);
+//  * row-wise fp32, below, for the rest (order 0 or above 4, fewer than four bases).
 #include <algorithm>
+#include <cmath>
 
 #include "efficient_kan.hpp"
 
 namespace taskops {
+
+// efficient_kan_direct.hip
+bool kan_direct_fits(int order, int C, int B, int I, int O);
+hipError_t kan_direct_launch(const float* x, const float* grid, const float* wb, const float* ws, const float* sc,
+                             int order, int L, int C, int B, int I, int O, float* out, size_t min_workspace,
+                             hipStream_t stream);
+
 namespace {
 
 // Row-wise fp32 path for shapes outside the fast path: the expanded activation row is
@@ -72,42 +84,72 @@ bool fast_path_fits(int B, int I, int O, int Cp) {
          ngroups * (1 + Cp) * Opad * kChunk * 2 < lim;
 }
 
+// The fast path's launch shape and its workspace.
+struct FastPlan {
+  int ngroups, Opad, table_blocks, tiles, nsplit, gper;
+  size_t half_bytes, table_bytes, counters_at, partial_at, bytes;
+};
+
+FastPlan fast_plan(int Cp, int B, int I, int O, int L) {
+  using namespace kan;
+  FastPlan p;
+  p.ngroups = (I + kGroup - 1) / kGroup;
+  p.Opad = ((O + BN - 1) / BN) * BN;
+  const int nq = p.ngroups * (1 + Cp);
+  p.half_bytes = (size_t)nq * p.Opad * kChunk * sizeof(_Float16);
+  p.table_bytes = (size_t)p.ngroups * tbl_group_bytes(L);
+  // kan_pack: one workgroup per kPackThreads basis-table entries (L per feature), each
+  // writing one knot-row flag word, then one per column pair.
+  p.table_blocks = (p.ngroups * kGroup * L + kPackThreads - 1) / kPackThreads;
+  // Split-K when the output tiles leave CUs idle (one workgroup fills a CU's registers): up to
+  // CUs / tiles splits of the feature groups, none empty.
+  p.tiles = ((B + BM - 1) / BM) * (p.Opad / BN);
+  p.nsplit = 1;
+  p.gper = p.ngroups;
+  if (p.tiles * 2 <= device_cu_count() && p.ngroups > 1) {
+    const int want = std::min(p.ngroups, device_cu_count() / p.tiles);
+    p.gper = (p.ngroups + want - 1) / want;
+    p.nsplit = (p.ngroups + p.gper - 1) / p.gper;
+  }
+  const size_t partial_bytes = p.nsplit > 1 ? (size_t)p.nsplit * p.tiles * BM * BN * sizeof(float) : 0;
+  const size_t fixed =
+      2 * p.half_bytes + p.table_bytes + (size_t)p.Opad * sizeof(float) + (size_t)p.table_blocks * sizeof(int);
+  p.counters_at = (fixed + 255) / 256 * 256;
+  p.partial_at = p.counters_at + ((size_t)p.tiles * sizeof(unsigned) + 255) / 256 * 256;
+  p.bytes = p.partial_at + partial_bytes;
+  return p;
+}
+
+// The direct path costs what its fp32 MFMAs do, about 25 us per 1e9 terms (B I O (1 + C)); the
+// fast path has 16 times their rate, but packs the weights first and, where its 128 x 256
+// tiles leave CUs idle, splits and sums the features: the more splits, the later it wins.
+// Where both took the same time (one box, terms against the fast path's splits): 2 splits 3e8
+// .. 8e8 terms, 4 7e8 .. 9e8, 8 1.0e9 .. 1.6e9, 16 1.5e9, 32 2.5e9, near 2.5e8 splits^(2/3).
+// Either side of the line (us, direct against fast): I = O = 1024, G = 5, B = 8 15.6 / 71, B =
+// 128 41 / 72, B = 512 131 / 68; I = 256, O = 512, G = 8, B = 256 25 / 47, B = 4096 159 / 70.
+bool direct_is_faster(const FastPlan& plan, int B, int I, int O, int C) {
+  const double terms = (double)B * I * O * (1 + C), n = plan.nsplit;
+  return terms <= 2.5e8 * std::cbrt(n * n);
+}
+
 template <int kCp>
 hipError_t launch_fast(const float* x, const float* grid, const float* wb, const float* ws,
                        const float* sc, int C, int B, int I, int O, int L, float* out,
                        hipStream_t stream) {
   using namespace kan;
-  const int ngroups = (I + kGroup - 1) / kGroup;
-  const int Opad = ((O + BN - 1) / BN) * BN;
-  const int nq = ngroups * (1 + kCp);
-  const size_t half_bytes = (size_t)nq * Opad * kChunk * sizeof(_Float16);
-  const size_t table_bytes = (size_t)ngroups * tbl_group_bytes(L);
-  // kan_pack: one workgroup per kPackThreads basis-table entries (L per feature), each
-  // writing one knot-row flag word, then one per column pair.
-  const int table_blocks = (ngroups * kGroup * L + kPackThreads - 1) / kPackThreads;
-  // Split-K when the output tiles leave CUs idle (one workgroup fills a CU's registers): up to
-  // CUs / tiles splits of the feature groups, none empty.
-  const int tiles = ((B + BM - 1) / BM) * (Opad / BN);
-  int nsplit = 1, gper = ngroups;
-  if (tiles * 2 <= device_cu_count() && ngroups > 1) {
-    const int want = std::min(ngroups, device_cu_count() / tiles);
-    gper = (ngroups + want - 1) / want;
-    nsplit = (ngroups + gper - 1) / gper;
-  }
-  const size_t partial_bytes = nsplit > 1 ? (size_t)nsplit * tiles * BM * BN * sizeof(float) : 0;
-  const size_t fixed = 2 * half_bytes + table_bytes + (size_t)Opad * sizeof(float) + (size_t)table_blocks * sizeof(int);
-  const size_t counters_at = (fixed + 255) / 256 * 256;
-  const size_t partial_at = counters_at + ((size_t)tiles * sizeof(unsigned) + 255) / 256 * 256;
+  const FastPlan plan = fast_plan(kCp, B, I, O, L);
+  const int ngroups = plan.ngroups, Opad = plan.Opad, table_blocks = plan.table_blocks, tiles = plan.tiles,
+            nsplit = plan.nsplit, gper = plan.gper;
   void* wsp = nullptr;
-  hipError_t e = workspace(kSlotKan, partial_at + partial_bytes, stream, &wsp);
+  hipError_t e = workspace(kSlotKan, plan.bytes, stream, &wsp);
   if (e != hipSuccess) return e;
   auto* bhi = static_cast<_Float16*>(wsp);
-  auto* blo = reinterpret_cast<_Float16*>(static_cast<char*>(wsp) + half_bytes);
-  auto* tables = reinterpret_cast<float*>(static_cast<char*>(wsp) + 2 * half_bytes);
-  auto* colscale = reinterpret_cast<float*>(static_cast<char*>(wsp) + 2 * half_bytes + table_bytes);
+  auto* blo = reinterpret_cast<_Float16*>(static_cast<char*>(wsp) + plan.half_bytes);
+  auto* tables = reinterpret_cast<float*>(static_cast<char*>(wsp) + 2 * plan.half_bytes);
+  auto* colscale = reinterpret_cast<float*>(static_cast<char*>(wsp) + 2 * plan.half_bytes + plan.table_bytes);
   auto* uflags = reinterpret_cast<int*>(colscale + Opad);
-  auto* counters = reinterpret_cast<unsigned*>(static_cast<char*>(wsp) + counters_at);
-  auto* partial = reinterpret_cast<float*>(static_cast<char*>(wsp) + partial_at);
+  auto* counters = reinterpret_cast<unsigned*>(static_cast<char*>(wsp) + plan.counters_at);
+  auto* partial = reinterpret_cast<float*>(static_cast<char*>(wsp) + plan.partial_at);
   // One launch finds the column scales, packs the weights and builds the basis tables and
   // their uniform-grid flags.
   const bool vecw = C % 4 == 0 && (reinterpret_cast<uintptr_t>(ws) & 15) == 0;
@@ -146,8 +188,23 @@ extern "C" hipError_t taskops_efficient_kan(const float* x, const float* grid,
   if (B == 0 || O == 0) return hipSuccess;
   const int C = grid_size + spline_order;
   const int Cp = kan::padded_bases(C);
-  if (spline_order == kan::kOrder && I > 0 && L <= kan::kMaxKnots && (Cp == 8 || Cp == 16) &&
-      fast_path_fits(B, I, O, Cp)) {
+  const bool fast = spline_order == kan::kOrder && I > 0 && L <= kan::kMaxKnots && (Cp == 8 || Cp == 16) &&
+                    fast_path_fits(B, I, O, Cp);
+  if (kan_direct_fits(spline_order, C, B, I, O)) {
+    size_t keep = 0;
+    bool direct = !fast;
+    if (fast) {
+      const FastPlan plan = fast_plan(Cp, B, I, O, L);
+      direct = direct_is_faster(plan, B, I, O, C);
+      // The workspace still grows to what the fast path asks for at this shape, so that a
+      // capture of another shape after this call finds as much room as the fast path leaves.
+      keep = plan.bytes;
+    }
+    if (direct)
+      return kan_direct_launch(x, grid, base_weight, spline_weight, spline_scaler, spline_order, L, C, B, I, O, out,
+                               keep, stream);
+  }
+  if (fast) {
     if (Cp == 8)
       return launch_fast<8>(x, grid, base_weight, spline_weight, spline_scaler, C, B, I, O, L, out, stream);
     return launch_fast<16>(x, grid, base_weight, spline_weight, spline_scaler, C, B, I, O, L, out, stream);

@@ -1,0 +1,96 @@
+// Host side of efficient_kan's direct fp32 path (efficient_kan_direct.hpp).
+#include <algorithm>
+
+#include "efficient_kan_direct.hpp"
+
+namespace taskops {
+namespace {
+
+using namespace kan_direct;
+
+// Row blocks of 16 per workgroup: as few as hold the batch, so small batches do no MFMAs
+// for missing rows, up to 4, which read each weight once per 64 rows.
+int row_blocks(int B) { return B <= 16 ? 1 : (B <= 32 ? 2 : 4); }
+
+template <int kNQ, int kR>
+hipError_t launch(const float* x, const float* grid, const float* wb, const float* ws, const float* sc, int order,
+                  int L, int C, int B, int I, int O, float* out, size_t min_workspace, hipStream_t stream) {
+  const int mtiles = (B + 16 * kR - 1) / (16 * kR), ctiles = (O + kCols - 1) / kCols;
+  const int nchunks = (I + chunk_features<kNQ, kR>() - 1) / chunk_features<kNQ, kR>();
+  const size_t lds = (size_t)lds_bytes<kNQ, kR>(C);
+  // Workgroups the chip holds at once, at most four per CU: the features are split until the
+  // grid has that many, in one round.  At 1, 2 and 4 per CU B = 8, I = O = 1024 took 19.7,
+  // 17.5 and 17.5 us (its LDS allows two); B = 4096, I = 256, O = 512 took 200 us at 3 and
+  // 178 at 4.
+  const int per_cu = std::max(1, std::min<int>(4, (int)(device_lds_per_cu() / lds)));
+  const int64_t tiles = (int64_t)mtiles * ctiles, want = (int64_t)per_cu * device_cu_count() / tiles;
+  int nsplit = (int)std::min<int64_t>(nchunks, std::max<int64_t>(want, 1));
+  const size_t n = (size_t)B * O;
+  void* partial = nullptr;
+  if (nsplit > 1 || min_workspace > 0) {
+    size_t have = 0;
+    const hipError_t e =
+        workspace_if_possible(kSlotKan, std::max(min_workspace, nsplit * n * sizeof(float)), stream, &partial, &have);
+    if (e != hipSuccess) return e;
+    // A capture that cannot allocate splits less: the sums only change their grouping.
+    nsplit = (int)std::min<size_t>(nsplit, std::max<size_t>(have / (n * sizeof(float)), 1));
+  }
+  const int cper = (nchunks + nsplit - 1) / nsplit;
+  nsplit = (nchunks + cper - 1) / cper;
+  const int64_t pairs = (int64_t)ctiles * nsplit, span = std::min<int64_t>(8, pairs), pairs8 = (pairs + span - 1) / span * span;
+  hipLaunchKernelGGL((kan_direct::kan_direct<kNQ, kR>), dim3((unsigned)(pairs8 * mtiles)), dim3(kThreads), lds, stream,
+                     x, grid, wb, ws, sc, order, L, C, B, I, O, mtiles, ctiles, nsplit, cper,
+                     nsplit > 1 ? static_cast<float*>(partial) : out);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || nsplit == 1) return e;
+  const unsigned blocks = (unsigned)std::min<size_t>((n + kThreads - 1) / kThreads, 4096);
+  hipLaunchKernelGGL(kan_direct_sum, dim3(blocks), dim3(kThreads), 0, stream, static_cast<const float*>(partial),
+                     (int64_t)n, nsplit, out);
+  return hipGetLastError();
+}
+
+template <int kNQ>
+hipError_t launch_rows(const float* x, const float* grid, const float* wb, const float* ws, const float* sc, int order,
+                       int L, int C, int B, int I, int O, float* out, size_t min_workspace, hipStream_t stream) {
+  switch (row_blocks(B)) {
+    case 1: return launch<kNQ, 1>(x, grid, wb, ws, sc, order, L, C, B, I, O, out, min_workspace, stream);
+    case 2: return launch<kNQ, 2>(x, grid, wb, ws, sc, order, L, C, B, I, O, out, min_workspace, stream);
+    default: return launch<kNQ, 4>(x, grid, wb, ws, sc, order, L, C, B, I, O, out, min_workspace, stream);
+  }
+}
+
+}  // namespace
+
+// Orders 1 .. 4 (the triangular scheme's instantiations), four or more bases (a feature's
+// bases are read 16 bytes at a time), 32-bit offsets for one workgroup's rows and columns,
+// and a grid one launch covers (2^32 - 1 work-items; the split never takes the grid past
+// three workgroups per CU).
+bool kan_direct_fits(int order, int C, int B, int I, int O) {
+  const int64_t lim = 0x7fffffff;
+  if (order < 1 || order > 4 || C < 4 || I < 1) return false;
+  if ((int64_t)kCols * I * C * 4 > lim || (int64_t)64 * I * 4 > lim) return false;
+  const int rows = 16 * row_blocks(B);
+  const int64_t tiles = (((int64_t)O + kCols - 1) / kCols + 7) / 8 * 8 * (((int64_t)B + rows - 1) / rows);
+  return tiles <= (int64_t)0xffffffff / kThreads;
+}
+
+hipError_t kan_direct_launch(const float* x, const float* grid, const float* wb, const float* ws, const float* sc,
+                             int order, int L, int C, int B, int I, int O, float* out, size_t min_workspace,
+                             hipStream_t stream) {
+#define TASKOPS_KAN_NQ(q) \
+  case q: return launch_rows<q>(x, grid, wb, ws, sc, order, L, C, B, I, O, out, min_workspace, stream)
+  switch ((C + 3) / 4) {
+    TASKOPS_KAN_NQ(1);
+    TASKOPS_KAN_NQ(2);
+    TASKOPS_KAN_NQ(3);
+    TASKOPS_KAN_NQ(4);
+    TASKOPS_KAN_NQ(5);
+    TASKOPS_KAN_NQ(6);
+    TASKOPS_KAN_NQ(7);
+    TASKOPS_KAN_NQ(8);
+    default: return hipErrorInvalidValue;
+  }
+#undef TASKOPS_KAN_NQ
+}
+
+}  // namespace taskops

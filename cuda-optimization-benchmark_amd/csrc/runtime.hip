@@ -31,39 +31,79 @@ __global__ void zero_fill(uint4* p, size_t n16) {
 
 }  // namespace
 
-hipError_t workspace(WorkspaceSlot slot, size_t bytes, hipStream_t stream, void** out) {
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
+namespace {
+
+// The current device, when `stream` (NULL = the default stream) belongs to it.  The workspace
+// is the current device's; kernels run on the stream's device.  A stream of another device is
+// refused rather than handed memory it cannot use.
+hipError_t stream_device(hipStream_t stream, int* dev) {
+  hipError_t e = hipGetDevice(dev);
   if (e != hipSuccess) return e;
-  if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
-  // The workspace is the current device's; kernels run on the stream's device.  A stream of
-  // another device is refused rather than handed memory it cannot use.
+  if (*dev < 0 || *dev >= kMaxDevices) return hipErrorInvalidDevice;
   if (stream != nullptr) {
     hipDevice_t sdev = 0;
     e = hipStreamGetDevice(stream, &sdev);
     if (e != hipSuccess) return e;
-    if (sdev != dev) return hipErrorInvalidValue;
+    if (sdev != *dev) return hipErrorInvalidValue;
   }
+  return hipSuccess;
+}
+
+// Makes region r at least `bytes` large (g_mu held).
+hipError_t grow(Region& r, size_t bytes, hipStream_t stream) {
+  const size_t want = ((bytes < 4096 ? 4096 : bytes) + 15) / 16 * 16;
+  void* p = nullptr;
+  hipError_t e = hipMalloc(&p, want);
+  if (e != hipSuccess) return e;
+  const size_t n16 = want / 16;
+  const unsigned blocks = (unsigned)(n16 / 256 < 4096 ? (n16 + 255) / 256 : 4096);
+  hipLaunchKernelGGL(zero_fill, dim3(blocks), dim3(256), 0, stream, static_cast<uint4*>(p), n16);
+  e = hipGetLastError();
+  if (e != hipSuccess) {
+    (void)hipFree(p);
+    return e;
+  }
+  if (r.ptr) g_retired.push_back(r.ptr);
+  r.ptr = p;
+  r.bytes = want;
+  return hipSuccess;
+}
+
+}  // namespace
+
+hipError_t workspace(WorkspaceSlot slot, size_t bytes, hipStream_t stream, void** out) {
+  int dev = 0;
+  hipError_t e = stream_device(stream, &dev);
+  if (e != hipSuccess) return e;
   std::lock_guard<std::mutex> lock(g_mu);
   Region& r = g_regions[dev][slot];
   if (r.bytes < bytes) {
-    const size_t want = ((bytes < 4096 ? 4096 : bytes) + 15) / 16 * 16;
-    void* p = nullptr;
-    e = hipMalloc(&p, want);
+    e = grow(r, bytes, stream);
     if (e != hipSuccess) return e;
-    const size_t n16 = want / 16;
-    const unsigned blocks = (unsigned)(n16 / 256 < 4096 ? (n16 + 255) / 256 : 4096);
-    hipLaunchKernelGGL(zero_fill, dim3(blocks), dim3(256), 0, stream, static_cast<uint4*>(p), n16);
-    e = hipGetLastError();
-    if (e != hipSuccess) {
-      (void)hipFree(p);
-      return e;
-    }
-    if (r.ptr) g_retired.push_back(r.ptr);
-    r.ptr = p;
-    r.bytes = want;
   }
   *out = r.ptr;
+  return hipSuccess;
+}
+
+hipError_t workspace_if_possible(WorkspaceSlot slot, size_t bytes, hipStream_t stream, void** out, size_t* have) {
+  int dev = 0;
+  hipError_t e = stream_device(stream, &dev);
+  if (e != hipSuccess) return e;
+  std::lock_guard<std::mutex> lock(g_mu);
+  Region& r = g_regions[dev][slot];
+  if (r.bytes < bytes) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    // The default stream cannot capture; asking about it while another stream captures is an
+    // error, and then nothing may be allocated either.
+    e = hipStreamIsCapturing(stream, &status);
+    if (e != hipSuccess) (void)hipGetLastError();
+    if (e == hipSuccess && status == hipStreamCaptureStatusNone) {
+      e = grow(r, bytes, stream);
+      if (e != hipSuccess) return e;
+    }
+  }
+  *out = r.ptr;
+  *have = r.bytes;
   return hipSuccess;
 }
 

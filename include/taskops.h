@@ -115,8 +115,9 @@ hipError_t taskops_ppo_clip_entropy_noalloc(int32_t B, int32_t T, int32_t H,
  * 5e-7 h use the cardinal cubic pieces (about 1e-6 of a basis value from the exact bases),
  * all other rows exact per-interval cubics.  It also needs x, out, its packed weights and
  * two output columns' I x 16 spline slots each under 2 GiB (spline_weight as a whole may be
- * larger).  Other orders, knot counts and sizes take an fp32 row-wise path without these
- * limits.
+ * larger).  Spline orders 1 to 4 otherwise (finer knot rows, other orders), and batches too
+ * small to pay for that path's weight packing, run on fp32 MFMAs, and the remaining orders and
+ * sizes row by row in fp32, both without these limits.
  * Replaces: reference/efficient_kan/solution.cu:177-288
  *           (tasks/efficient_kan/tests/task.json:3; op: reference.py:33-51). */
 hipError_t taskops_efficient_kan(const float* x, const float* grid, const float* base_weight,
