@@ -6,6 +6,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <mutex>
 
 #include "taskops.h"
 
@@ -160,6 +161,20 @@ hipError_t workspace(WorkspaceSlot slot, size_t bytes, hipStream_t stream, void*
 // is capturing, where nothing may be allocated; *have is the region's size.  For callers that
 // can do with less.
 hipError_t workspace_if_possible(WorkspaceSlot slot, size_t bytes, hipStream_t stream, void** out, size_t* have);
+
+// Scratch memory of one stream, for calls of two launches whose callers may be on several
+// streams and threads at once: launches on the stream use it one after another, and the lock
+// keeps other threads' calls from enqueuing between this call's launches.  ptr is null when
+// there is none, and the caller takes a path that needs none: while the stream is capturing
+// (a graph may be replayed beside other work), for hipStreamPerThread (one handle, many
+// streams), when kMaxScratchStreams other streams hold theirs, or when memory is short.
+// Not cleared.  Grown by doubling, kept until the process exits.
+struct StreamScratch {
+  StreamScratch(size_t bytes, hipStream_t stream);
+  std::unique_lock<std::mutex> lock;
+  void* ptr = nullptr;
+};
+constexpr int kMaxScratchStreams = 8;
 
 // Number of compute units of the current device (cached per device).
 int device_cu_count();

@@ -19,7 +19,7 @@ namespace taskops {
 // efficient_kan_direct.hip
 bool kan_direct_fits(int order, int C, int B, int I, int O);
 hipError_t kan_direct_launch(const float* x, const float* grid, const float* wb, const float* ws, const float* sc,
-                             int order, int L, int C, int B, int I, int O, float* out, size_t min_workspace,
+                             int order, int L, int C, int B, int I, int O, float* out, size_t shared_bytes,
                              hipStream_t stream);
 
 namespace {

@@ -1,5 +1,6 @@
 // Host side of efficient_kan's direct fp32 path (efficient_kan_direct.hpp).
 #include <algorithm>
+#include <optional>
 
 #include "efficient_kan_direct.hpp"
 
@@ -14,7 +15,7 @@ int row_blocks(int B) { return B <= 16 ? 1 : (B <= 32 ? 2 : 4); }
 
 template <int kNQ, int kR>
 hipError_t launch(const float* x, const float* grid, const float* wb, const float* ws, const float* sc, int order,
-                  int L, int C, int B, int I, int O, float* out, size_t min_workspace, hipStream_t stream) {
+                  int L, int C, int B, int I, int O, float* out, size_t shared_bytes, hipStream_t stream) {
   const int mtiles = (B + 16 * kR - 1) / (16 * kR), ctiles = (O + kCols - 1) / kCols;
   const int nchunks = (I + chunk_features<kNQ, kR>() - 1) / chunk_features<kNQ, kR>();
   const size_t lds = (size_t)lds_bytes<kNQ, kR>(C);
@@ -25,16 +26,19 @@ hipError_t launch(const float* x, const float* grid, const float* wb, const floa
   const int per_cu = std::max(1, std::min<int>(4, (int)(device_lds_per_cu() / lds)));
   const int64_t tiles = (int64_t)mtiles * ctiles, want = (int64_t)per_cu * device_cu_count() / tiles;
   int nsplit = (int)std::min<int64_t>(nchunks, std::max<int64_t>(want, 1));
-  const size_t n = (size_t)B * O;
+  const size_t n = (size_t)B * O, bytes = nsplit * n * sizeof(float);
   void* partial = nullptr;
-  if (nsplit > 1 || min_workspace > 0) {
+  std::optional<StreamScratch> scratch;
+  if (shared_bytes > 0) {
     size_t have = 0;
-    const hipError_t e =
-        workspace_if_possible(kSlotKan, std::max(min_workspace, nsplit * n * sizeof(float)), stream, &partial, &have);
+    const hipError_t e = workspace_if_possible(kSlotKan, std::max(shared_bytes, bytes), stream, &partial, &have);
     if (e != hipSuccess) return e;
-    // A capture that cannot allocate splits less: the sums only change their grouping.
-    nsplit = (int)std::min<size_t>(nsplit, std::max<size_t>(have / (n * sizeof(float)), 1));
+    nsplit = (int)std::min<size_t>(nsplit, have / (n * sizeof(float)));
+  } else if (nsplit > 1) {
+    scratch.emplace(bytes, stream);
+    partial = scratch->ptr;
   }
+  if (partial == nullptr || nsplit < 1) nsplit = 1;
   const int cper = (nchunks + nsplit - 1) / nsplit;
   nsplit = (nchunks + cper - 1) / cper;
   const int64_t pairs = (int64_t)ctiles * nsplit, span = std::min<int64_t>(8, pairs), pairs8 = (pairs + span - 1) / span * span;
@@ -51,11 +55,11 @@ hipError_t launch(const float* x, const float* grid, const float* wb, const floa
 
 template <int kNQ>
 hipError_t launch_rows(const float* x, const float* grid, const float* wb, const float* ws, const float* sc, int order,
-                       int L, int C, int B, int I, int O, float* out, size_t min_workspace, hipStream_t stream) {
+                       int L, int C, int B, int I, int O, float* out, size_t shared_bytes, hipStream_t stream) {
   switch (row_blocks(B)) {
-    case 1: return launch<kNQ, 1>(x, grid, wb, ws, sc, order, L, C, B, I, O, out, min_workspace, stream);
-    case 2: return launch<kNQ, 2>(x, grid, wb, ws, sc, order, L, C, B, I, O, out, min_workspace, stream);
-    default: return launch<kNQ, 4>(x, grid, wb, ws, sc, order, L, C, B, I, O, out, min_workspace, stream);
+    case 1: return launch<kNQ, 1>(x, grid, wb, ws, sc, order, L, C, B, I, O, out, shared_bytes, stream);
+    case 2: return launch<kNQ, 2>(x, grid, wb, ws, sc, order, L, C, B, I, O, out, shared_bytes, stream);
+    default: return launch<kNQ, 4>(x, grid, wb, ws, sc, order, L, C, B, I, O, out, shared_bytes, stream);
   }
 }
 
@@ -74,11 +78,14 @@ bool kan_direct_fits(int order, int C, int B, int I, int O) {
   return tiles <= (int64_t)0xffffffff / kThreads;
 }
 
+// shared_bytes: 0 for calls with no workspace of their own (the splits' sums then go to the
+// stream's scratch memory, and stay unsplit where there is none); else the size to which the
+// shared workspace is grown, which holds them.
 hipError_t kan_direct_launch(const float* x, const float* grid, const float* wb, const float* ws, const float* sc,
-                             int order, int L, int C, int B, int I, int O, float* out, size_t min_workspace,
+                             int order, int L, int C, int B, int I, int O, float* out, size_t shared_bytes,
                              hipStream_t stream) {
 #define TASKOPS_KAN_NQ(q) \
-  case q: return launch_rows<q>(x, grid, wb, ws, sc, order, L, C, B, I, O, out, min_workspace, stream)
+  case q: return launch_rows<q>(x, grid, wb, ws, sc, order, L, C, B, I, O, out, shared_bytes, stream)
   switch ((C + 3) / 4) {
     TASKOPS_KAN_NQ(1);
     TASKOPS_KAN_NQ(2);

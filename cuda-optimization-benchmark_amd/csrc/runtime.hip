@@ -14,7 +14,15 @@ struct Region {
   size_t bytes = 0;
 };
 
+struct StreamRegion {
+  hipStream_t stream = nullptr;
+  void* ptr = nullptr;
+  size_t bytes = 0;
+};
+
 std::mutex g_mu;
+std::mutex g_scratch_mu;
+StreamRegion g_scratch[kMaxDevices][kMaxScratchStreams];
 Region g_regions[kMaxDevices][kNumSlots];
 // Buffers replaced by a larger one stay allocated until exit: a kernel enqueued before
 // the replacement may still be using them, and freeing would need a host sync.
@@ -105,6 +113,39 @@ hipError_t workspace_if_possible(WorkspaceSlot slot, size_t bytes, hipStream_t s
   *out = r.ptr;
   *have = r.bytes;
   return hipSuccess;
+}
+
+StreamScratch::StreamScratch(size_t bytes, hipStream_t stream) {
+  int dev = 0;
+  if (stream == hipStreamPerThread || stream_device(stream, &dev) != hipSuccess) return;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  if (status != hipStreamCaptureStatusNone) return;
+  lock = std::unique_lock<std::mutex>(g_scratch_mu);
+  StreamRegion* r = nullptr;
+  for (StreamRegion& s : g_scratch[dev])
+    if (s.ptr != nullptr && s.stream == stream) r = &s;
+  for (StreamRegion& s : g_scratch[dev])
+    if (r == nullptr && s.ptr == nullptr) r = &s;
+  if (r == nullptr) return;
+  if (r->bytes < bytes) {
+    size_t want = r->bytes > 0 ? 2 * r->bytes : (size_t)1 << 18;
+    while (want < bytes) want *= 2;
+    void* p = nullptr;
+    if (hipMalloc(&p, want) != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
+    if (r->ptr != nullptr) {
+      std::lock_guard<std::mutex> retire(g_mu);
+      g_retired.push_back(r->ptr);
+    }
+    *r = StreamRegion{stream, p, want};
+  }
+  ptr = r->ptr;
 }
 
 int device_cu_count() {

@@ -19,7 +19,11 @@
  * results or derived weight contents between calls.  Calls are asynchronous: no host synchronisation and no
  * device-to-host copy happens inside a call.  Calls that share a device and overlap in
  * time on different streams race on that workspace (as the reference's statics do);
- * calls on one stream are safe.
+ * calls on one stream are safe.  reward_to_go, leaky and fp8_linear, and efficient_kan where
+ * it does not pack weights (other spline orders than 3, more than 16 knots), hold no such
+ * shared memory and may overlap: what scratch they use belongs to the stream (up to 8 streams'
+ * per device are kept, at most a few tens of MB each; other streams, hipStreamPerThread and
+ * captures run without).
  *
  * Raw-bit types are used at the boundary for the two non-C element types:
  *   e4m3 (OCP FP8, 1 byte)  -> uint8_t   (the reference uses __nv_fp8_e4m3)
