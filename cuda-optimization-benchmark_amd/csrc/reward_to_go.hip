@@ -9,13 +9,20 @@
 // of one 8-step-per-lane chunk (whose 16-byte accesses cover every other 16 bytes per
 // instruction, and which slows to 39 us with non-temporal stores).  Shorter rows use fewer
 // waves and chunks per wave, so no wave idles.
+#include <cmath>
+
 #include "reward_to_go.hpp"
 
 namespace taskops {
 namespace {
 
 constexpr int kPerLane = 4;
-constexpr int kNonTemporal = 5;  // non-temporal loads (bit 0) and stores (policy 2 in bits 1-2)
+// Cache policies (kNT of the kernel): aligned rows, non-temporal loads (bit 0) and stores
+// (policy 2 in bits 1-2).  Unaligned rows share the lines at their ends with the next load, so
+// theirs are ordinary loads: B = 4096, T = 4095 31.3 us against 34.0 with non-temporal ones
+// (39.4 with ordinary stores too; 65.1 element by element, which such rows took before).
+template <RtgAccess kAccess>
+constexpr int policy() { return kAccess == kUnaligned ? 4 : 5; }
 
 // Rows of 4 waves x 4 chunks (T > 2048) run with at most this many workgroups per CU,
 // held there by the LDS each one reserves (the kernel's own LDS is a few bytes).  At the
@@ -31,20 +38,71 @@ size_t occupancy_lds(int per_cu) { return (size_t)device_lds_per_cu() / (per_cu 
 // so rows go out in launches of at most kRowsPerLaunch (one launch for every B up to it).
 constexpr int kRowsPerLaunch = 1 << 23;
 
-template <int kWaves, int kSeg>
-void launch(const float* reward, const uint8_t* done, double g, int B, int T, float* out,
-            bool vec, hipStream_t stream) {
+template <int kWaves, int kSeg, RtgAccess kAccess>
+void launch(const float* reward, const uint8_t* done, double g, int B, int T, float* out, hipStream_t stream) {
   const size_t lds = (kWaves == 4 && kSeg == 4) ? occupancy_lds(kLongRowWorkgroupsPerCU) : 0;
   for (int b0 = 0; b0 < B; b0 += kRowsPerLaunch) {
     const int nb = B - b0 < kRowsPerLaunch ? B - b0 : kRowsPerLaunch;
-    const size_t off = (size_t)b0 * (size_t)T;  // T % 4 == 0 on the vector path: alignment kept
-    if (vec)
-      hipLaunchKernelGGL((reward_to_go_kernel<kWaves, kPerLane, kSeg, true, kNonTemporal>), dim3(nb),
-                         dim3(kWaves * kWave), lds, stream, reward + off, done + off, g, nb, T, out + off);
-    else
-      hipLaunchKernelGGL((reward_to_go_kernel<kWaves, kPerLane, kSeg, false, kNonTemporal>), dim3(nb),
-                         dim3(kWaves * kWave), lds, stream, reward + off, done + off, g, nb, T, out + off);
+    const size_t off = (size_t)b0 * (size_t)T;  // T % 4 == 0 on the aligned path: alignment kept
+    hipLaunchKernelGGL((reward_to_go_kernel<kWaves, kPerLane, kSeg, kAccess, policy<kAccess>()>), dim3(nb),
+                       dim3(kWaves * kWave), lds, stream, reward + off, done + off, g, nb, T, out + off, 1, 0,
+                       static_cast<RtgMap*>(nullptr));
   }
+}
+
+// Few long rows.  A workgroup walks its row one segment of 4096 steps after another, about 2.2
+// us each, so such rows are split into parts over workgroups: one launch composes each part's
+// map, a second scans each part from the maps after it, reading the rewards again (from the
+// caches).  Whole row against split, us per call: 16 x 65536 33-39 / 8.5, 1 x 131072 71 / 7.9,
+// 6 x 18592 12.4 / 7.8, 33 x 109969 75.6 / 13.6, 128 x 131072 82.7 / 38.9, 256 x 65536 46.2 / 39.1.
+// Rows of at most 12288 steps (three segments) or more than 256 of them keep the whole-row
+// form: 1 x 8000 5.7 / 8.0, 229 x 9751 11.5 / 11.6, 256 x 16384 13.3 / 13.3, 512 x 8192 9.5 / 13.3.
+constexpr int kSplitMaxRows = 256, kSplitMinChunks = 48;
+// Up to this many chunks in all, parts of 4 chunks (up to 1024 workgroups), else of 16: 64 x
+// 16384 8.5 against 8.7 us, 33 x 109969 17.8 against 13.6.
+constexpr int kSmallPartChunks = 4096;
+
+template <int kSeg, RtgAccess kAccess>
+hipError_t launch_split(const float* reward, const uint8_t* done, double g, int B, int T, float* out, int nparts,
+                        int cpart, RtgMap* maps, hipStream_t stream) {
+  constexpr int kWaves = 4;
+  // Ordinary loads in the first pass, so that the second finds the rewards in the caches.
+  hipLaunchKernelGGL((reward_to_go_kernel<kWaves, kPerLane, kSeg, kAccess, 0, kMaps>), dim3(B * nparts),
+                     dim3(kWaves * kWave), 0, stream, reward, done, g, B, T, out, nparts, cpart, maps);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((reward_to_go_kernel<kWaves, kPerLane, kSeg, kAccess, policy<kAccess>(), kApply>), dim3(B * nparts),
+                     dim3(kWaves * kWave), 0, stream, reward, done, g, B, T, out, nparts, cpart, maps);
+  return hipGetLastError();
+}
+
+template <RtgAccess kAccess>
+hipError_t run(const float* reward, const uint8_t* done, double g, int B, int T, float* out, hipStream_t stream) {
+  const int nchunks = (int)(((int64_t)T + kWave * kPerLane - 1) / (kWave * kPerLane));  // chunks of 256 steps
+  if constexpr (kAccess != kElements) {
+    // |g| <= 1: a part's a = g^steps cannot overflow (inf * 0 would make the carry NaN).
+    if (B <= kSplitMaxRows && nchunks > kSplitMinChunks && std::fabs(g) <= 1.0) {
+      const bool big = (int64_t)B * nchunks > kSmallPartChunks;
+      const int cpart = big ? 16 : 4, nparts = (nchunks + cpart - 1) / cpart;
+      StreamScratch scratch((size_t)B * nparts * sizeof(RtgMap), stream);
+      if (scratch.ptr != nullptr) {
+        auto* maps = static_cast<RtgMap*>(scratch.ptr);
+        return big ? launch_split<4, kAccess>(reward, done, g, B, T, out, nparts, cpart, maps, stream)
+                   : launch_split<1, kAccess>(reward, done, g, B, T, out, nparts, cpart, maps, stream);
+      }
+    }
+  }
+  if (nchunks <= 1)
+    launch<1, 1, kAccess>(reward, done, g, B, T, out, stream);
+  else if (nchunks <= 2)
+    launch<2, 1, kAccess>(reward, done, g, B, T, out, stream);
+  else if (nchunks <= 4)
+    launch<4, 1, kAccess>(reward, done, g, B, T, out, stream);
+  else if (nchunks <= 8)
+    launch<4, 2, kAccess>(reward, done, g, B, T, out, stream);
+  else
+    launch<4, 4, kAccess>(reward, done, g, B, T, out, stream);
+  return hipGetLastError();
 }
 
 }  // namespace
@@ -57,21 +115,12 @@ extern "C" hipError_t taskops_reward_to_go(const float* reward, const bool* done
                                            hipStream_t stream) {
   if (B <= 0 || T <= 0) return hipSuccess;  // nothing to write
   const uint8_t* d = reinterpret_cast<const uint8_t*>(done);
-  // The vector path's buffer stores address a row in 32-bit bytes (store_row16).
-  const bool vec = (T % 4) == 0 && T < (1 << 30) &&
-                   ((reinterpret_cast<uintptr_t>(reward) | reinterpret_cast<uintptr_t>(output)) & 15) == 0 &&
-                   (reinterpret_cast<uintptr_t>(d) & 3) == 0;
-  const int nchunks = (T + kWave * kPerLane - 1) / (kWave * kPerLane);  // chunks of 256 steps
   const double g = (double)gamma;
-  if (nchunks <= 1)
-    launch<1, 1>(reward, d, g, B, T, output, vec, stream);
-  else if (nchunks <= 2)
-    launch<2, 1>(reward, d, g, B, T, output, vec, stream);
-  else if (nchunks <= 4)
-    launch<4, 1>(reward, d, g, B, T, output, vec, stream);
-  else if (nchunks <= 8)
-    launch<4, 2>(reward, d, g, B, T, output, vec, stream);
-  else
-    launch<4, 4>(reward, d, g, B, T, output, vec, stream);
-  return hipGetLastError();
+  // The 16-byte paths' buffer stores address a row in 32-bit bytes (store_row16).
+  if (T >= (1 << 30)) return run<kElements>(reward, d, g, B, T, output, stream);
+  const bool aligned = (T % 4) == 0 &&
+                       ((reinterpret_cast<uintptr_t>(reward) | reinterpret_cast<uintptr_t>(output)) & 15) == 0 &&
+                       (reinterpret_cast<uintptr_t>(d) & 3) == 0;
+  if (aligned) return run<kAligned>(reward, d, g, B, T, output, stream);
+  return run<kUnaligned>(reward, d, g, B, T, output, stream);
 }

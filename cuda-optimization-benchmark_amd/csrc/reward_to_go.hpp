@@ -39,6 +39,10 @@ namespace taskops {
 namespace rtg_detail {
 using f32x4 = float __attribute__((ext_vector_type(4)));
 
+// The same accesses at a float's and a byte's alignment.
+typedef f32x4 __attribute__((aligned(4))) f32x4u;
+typedef unsigned __attribute__((aligned(1))) u32u;
+
 // A wave-uniform double moved to scalar registers (it is the same in every lane).
 __device__ __forceinline__ double uniform(double v) {
   const long long b = __double_as_longlong(v);
@@ -71,12 +75,56 @@ __device__ __forceinline__ void store_row16(float* row_base, int T, int t, f32x4
 }
 }  // namespace rtg_detail
 
+// How a lane reads its 4 steps: kAligned, T % 4 == 0 and 16-byte rewards and outputs, 4-byte
+// done words at aligned addresses; kUnaligned, the same loads and stores at any row start (a
+// float's alignment for the 16-byte accesses, a byte's for the done word, which gfx950's
+// memory pipeline takes), the row's last steps one by one; kElements, one by one throughout.
+enum RtgAccess : int { kElements = 0, kAligned = 1, kUnaligned = 2 };
+
+// What a workgroup does with its span of the row: kWhole, the whole row; for a row split over
+// workgroups, kMaps writes its part's composed map and kApply, in a second launch, composes
+// the maps of the parts after its own and scans its part from that value.
+enum RtgMode : int { kWhole = 0, kMaps = 1, kApply = 2 };
+
+// A part's map v -> r + a v.
+struct RtgMap {
+  double r, a;
+};
+
+namespace rtg_detail {
+// The maps first .. n - 1 of a row's parts composed and applied to 0, the same in every lane:
+// lane l of each batch of 64 takes one part, a suffix scan composes the batch, and batches are
+// composed from the row's end, always in this order, so the bits do not depend on timing.
+__device__ __forceinline__ double compose_after(const RtgMap* __restrict__ maps, int first, int n, int lane) {
+  double v = 0.0;
+  for (int p0 = first + (n - 1 - first) / kWave * kWave; p0 >= first && first < n; p0 -= kWave) {
+    double r = 0.0, a = 1.0;
+    if (p0 + lane < n) {
+      r = maps[p0 + lane].r;
+      a = maps[p0 + lane].a;
+    }
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {  // (r, a): the map of lanes lane .. lane + 2 off - 1
+      const double rn = __shfl_down(r, off, kWave), an = __shfl_down(a, off, kWave);
+      if (lane + off < kWave) {
+        r = fma(a, rn, r);
+        a *= an;
+      }
+    }
+    v = fma(uniform(__shfl(a, 0, kWave)), v, uniform(__shfl(r, 0, kWave)));
+  }
+  return v;
+}
+}  // namespace rtg_detail
+
 // kNT: bit 0 = non-temporal loads; bits 1-2 = the cache policy of buffer output stores
-// (store_row16), 0 = plain stores.
-template <int kWaves, int kPerLane, int kSeg, bool kVec, int kNT>
+// (store_row16), 0 = plain stores.  Split rows (kMode != kWhole): workgroup (row, part) =
+// (blockIdx.x / nparts, blockIdx.x % nparts) owns chunks part * cpart .. + cpart - 1 and
+// maps[row * nparts + part].
+template <int kWaves, int kPerLane, int kSeg, RtgAccess kAccess, int kNT, RtgMode kMode = kWhole>
 __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
     const float* __restrict__ reward, const uint8_t* __restrict__ done, double g, int B, int T,
-    float* __restrict__ out) {
+    float* __restrict__ out, int nparts = 1, int cpart = 0, RtgMap* __restrict__ maps = nullptr) {
   using namespace rtg_detail;
   static_assert(kPerLane == 4, "a lane owns one 16-byte reward vector per chunk");
   constexpr int kChunk = kWave * kPerLane;
@@ -106,13 +154,18 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
     }
   }
   const float gf = (float)g;
-  const size_t base = (size_t)blockIdx.x * (size_t)T;
+  const int row = kMode == kWhole ? (int)blockIdx.x : (int)blockIdx.x / nparts;
+  const int part = kMode == kWhole ? 0 : (int)blockIdx.x % nparts;
+  const int first = kMode == kWhole ? 0 : part * cpart;  // this workgroup's chunks
+  const int end = kMode == kWhole ? nchunks : min(nchunks, first + cpart);
+  const size_t base = (size_t)row * (size_t)T;
   const float* rr = reward + base;
   const uint8_t* dd = done + base;
   float* oo = out + base;
-  double carry = 0.0;
-  for (int hi = nchunks; hi > 0; hi -= kWaves * kSeg) {
-    const int lo = hi > kWaves * kSeg ? hi - kWaves * kSeg : 0;
+  double carry = 0.0, span = 1.0;  // span: kMaps, the a of the part's chunks so far
+  if constexpr (kMode == kApply) carry = compose_after(maps + (size_t)row * nparts, part + 1, nparts, lane);
+  for (int hi = end; hi > first; hi -= kWaves * kSeg) {
+    const int lo = hi - first > kWaves * kSeg ? hi - kWaves * kSeg : first;
     const int c0 = lo + wave * kSeg;
     float r[kSeg][4];
     unsigned dn[kSeg];
@@ -123,7 +176,7 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e) r[c][e] = 0.0f;
       if (c0 + c >= hi) continue;
-      if constexpr (kVec) {
+      if constexpr (kAccess == kAligned) {
         if (t < T) {
           const f32x4* src = reinterpret_cast<const f32x4*>(rr + t);
           const f32x4 v = (kNT & 1) ? __builtin_nontemporal_load(src) : *src;
@@ -133,6 +186,14 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
           r[c][3] = v.w;
           dn[c] = *reinterpret_cast<const unsigned*>(dd + t);
         }
+      } else if (kAccess == kUnaligned && (c0 + c + 1) * kChunk <= T) {  // uniform: a whole chunk
+        const f32x4u* src = reinterpret_cast<const f32x4u*>(rr + t);
+        const f32x4u v = (kNT & 1) ? __builtin_nontemporal_load(src) : *src;
+        r[c][0] = v.x;
+        r[c][1] = v.y;
+        r[c][2] = v.z;
+        r[c][3] = v.w;
+        dn[c] = *reinterpret_cast<const u32u*>(dd + t);
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -201,6 +262,15 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
       x = fma(span_a[v], x, span_r[v]);
     }
     const double next_carry = x;
+    if constexpr (kMode == kMaps) {
+      double a = 1.0;
+#pragma unroll
+      for (int v = 0; v < kWaves; ++v) a *= span_a[v];
+      span *= a;
+      carry = next_carry;
+      __syncthreads();
+      continue;
+    }
 
 #pragma unroll
     for (int c = kSeg - 1; c >= 0; --c) {
@@ -223,13 +293,17 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
       o[3] = (float)fma(coef(dn[c], 3, g), vin, (double)r[c][3]);
 #pragma unroll
       for (int e = 2; e >= 0; --e) o[e] = fmaf(coef32(dn[c], e, gf), o[e + 1], r[c][e]);
-      if constexpr (kVec) {
-        if (t < T) {
+      if constexpr (kAccess != kElements) {
+        if (kAccess == kAligned ? t < T : t + 4 <= T) {
           const f32x4 w = {o[0], o[1], o[2], o[3]};
           if constexpr (((kNT >> 1) & 3) != 0)
             store_row16<(kNT >> 1) & 3>(oo, T, t, w);
           else
-            *reinterpret_cast<f32x4*>(oo + t) = w;
+            *reinterpret_cast<f32x4u*>(oo + t) = w;
+        } else if (kAccess == kUnaligned) {
+#pragma unroll
+          for (int e = 0; e < 3; ++e)
+            if (t + e < T) oo[t + e] = o[e];
         }
       } else {
 #pragma unroll
@@ -240,6 +314,8 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
     carry = next_carry;
     __syncthreads();  // span_* are rewritten by the next segment
   }
+  if constexpr (kMode == kMaps)
+    if (threadIdx.x == 0) maps[(size_t)row * nparts + part] = RtgMap{carry, span};
 }
 
 }  // namespace taskops
