@@ -53,6 +53,7 @@ KERNEL_SOURCES = [
     "efficient_kan.hip",
     "efficient_kan_direct.hip",
     "fp8_linear.hip",
+    "fp8_linear_mid.hip",
     "quantize_e4m3.hip",
 ]
 

@@ -1,10 +1,9 @@
 // fp8_linear on gfx950: output = bf16((x/sx) @ (w/sw)^T + bias), OCP e4m3 inputs.
 //
 // Drop-in signature tasks/fp8_linear/tests/task.json:3, replacing
-// reference/fp8_linear/solution.cu:276-321.  Kernels are in fp8_linear.hpp: the skinny
-// split-K kernel for M <= 64, the wide (direct-to-LDS, 128-byte rows) kernel when
-// K % 16 == 0 and the operands are 16-byte aligned (in its 128-row form when 256x256
-// tiles would fill at most half the CUs), and the register-staged tiled kernel otherwise.
+// reference/fp8_linear/solution.cu:276-321.  Kernels are in fp8_linear.hpp (skinny, wide and its
+// 128-row form) and fp8_linear_mid.hpp (64 to 128-row tiles, any K and alignment); the rules
+// below choose.
 #include "fp8_linear.hpp"
 
 using namespace taskops;
@@ -25,6 +24,37 @@ bool offsets_fit(int64_t M, int64_t K, int64_t N) {
   return (int64_t)BM * K <= lim && (int64_t)BM * N * 2 <= lim;
 }
 
+// The middle kernel's tile for a call, or -1 for the skinny and wide kernels.
+//
+// M > 64: the smallest tile that gives each CU at most one workgroup, since the work of one
+// step is bound by its own LDS traffic and smaller tiles only spread it: us at 64x64 / 64x128 /
+// 128x128 / 128x256: M = 256, K = N = 4096 (256 tiles of 64x64) 9.2 / 13.5 / 16.8 / 24.0, M =
+// 512 14.7 / 14.0 / 17.1 / 24.0, M = 1024 27 / 26 / 19.0 / 24.3, M = 2048 51 / 51 / 36.9 / 29.8,
+// and from there on the wide kernel's forms.  Where they do not apply (K % 16, alignment),
+// 128x128 tiles take the rest.
+//
+// M <= 64: the skinny kernel's time is its weight stream at a rate that falls with the row
+// blocks, a 64x64 tile's is its steps, so wide N favours the tiles: at K = N = 8192 M = 16 17.0
+// against 13.5 us, M = 32 23.5 / 14.4, M = 64 30.1 / 15.7; at 4096 6.2 / 8.5, 7.9 / 8.5, 9.4 /
+// 9.1; from 33 rows on the tiles were never slower.  With 8-byte rows both move less per load: M
+// = 64, K = N = 8184 45.5 / 26.4 but M = 16 and 4088 7.2 / 12.6, M = 64 14.0 / 14.6.  Other K
+// have no 8-byte loads for the skinny kernel: M = 16, K = 2047, N = 8000 41.2 / 10.4, M = 1, K =
+// 333, N = 300 5.2 / 4.6.
+int mid_tile(int64_t M, int64_t K, int64_t N, int vec) {
+  const int64_t cus = device_cu_count();
+  if (M <= kSkinnyMaxM) {
+    if (vec == 16 && 64 * K > (int64_t)0x7fffffff) return -1;  // a tile's rows in 32-bit offsets
+    const int rb = (int)(M + 15) / 16;
+    const bool tiles = vec == 1 || (vec == 16 ? (rb >= 3 || N >= (rb == 2 ? 5120 : 7168)) : (rb >= 3 && N > 4096));
+    return tiles ? kTile64x64 : -1;
+  }
+  auto tiles = [&](int rows, int cols) { return ((M + rows - 1) / rows) * ((N + cols - 1) / cols); };
+  if (tiles(64, 64) <= cus) return kTile64x64;
+  if (tiles(64, 128) <= cus) return kTile64x128;
+  if (vec != 16 || tiles(128, 128) <= cus) return kTile128x128;
+  return -1;
+}
+
 }  // namespace
 
 extern "C" hipError_t taskops_fp8_linear(int32_t M, int32_t K, int32_t N, const uint8_t* x_fp8,
@@ -36,6 +66,10 @@ extern "C" hipError_t taskops_fp8_linear(int32_t M, int32_t K, int32_t N, const 
   if (!offsets_fit(M, K, N)) return hipErrorInvalidValue;
   const float inv = (float)(1.0 / ((double)scale_x * (double)scale_w));
   const int vec = vec_width(x_fp8, w_fp8, K);
+  const int mid = mid_tile(M, K, N, vec);
+  if (mid >= 0)
+    return mid_launch(static_cast<MidTile>(mid), vec == 16, x_fp8, w_fp8, (int)M, (int)N, (int)K, inv, bias, output,
+                      stream);
   if (M <= kSkinnyMaxM) {
     const dim3 grid((N + 15) / 16);
     if (vec == 16) {
@@ -58,55 +92,42 @@ extern "C" hipError_t taskops_fp8_linear(int32_t M, int32_t K, int32_t N, const 
                              x_fp8, w_fp8, (int)M, (int)N, (int)K, inv, bias, output);
           break;
       }
-    } else if (vec == 8)
-      hipLaunchKernelGGL(fp8_gemm_skinny<8>, grid, dim3(kSkinnyThreads), 0, stream, x_fp8, w_fp8,
-                         (int)M, (int)N, (int)K, inv, bias, output);
-    else
-      hipLaunchKernelGGL(fp8_gemm_skinny<1>, grid, dim3(kSkinnyThreads), 0, stream, x_fp8, w_fp8,
-                         (int)M, (int)N, (int)K, inv, bias, output);
+    } else
+      hipLaunchKernelGGL(fp8_gemm_skinny, grid, dim3(kSkinnyThreads), 0, stream, x_fp8, w_fp8, (int)M, (int)N, (int)K,
+                         inv, bias, output);
     return hipGetLastError();
   }
   const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-  const size_t lds = 2 * kStageBytes;
-  if (vec == 16) {
-    const size_t wide_lds = kWideLdsBytes;
-    const uintptr_t o = reinterpret_cast<uintptr_t>(output);
-    if (2 * tiles <= device_cu_count()) {
-      // At most half a 256x256 tile per CU: 128x256 tiles, twice as many workgroups.
-      const dim3 hgrid(((M + kHalfRows - 1) / kHalfRows) * ((N + BN - 1) / BN));
-      const size_t half_lds = kHalfLaunchLdsBytes;
-      if (N % 8 == 0 && (o & 15) == 0)
-        hipLaunchKernelGGL(fp8_gemm_half<2>, hgrid, dim3(kThreads), half_lds, stream, x_fp8, w_fp8, (int)M,
-                           (int)N, (int)K, inv, bias, output);
-      else if (N % 4 == 0 && (o & 7) == 0)
-        hipLaunchKernelGGL(fp8_gemm_half<1>, hgrid, dim3(kThreads), half_lds, stream, x_fp8, w_fp8, (int)M,
-                           (int)N, (int)K, inv, bias, output);
-      else
-        hipLaunchKernelGGL(fp8_gemm_half<0>, hgrid, dim3(kThreads), half_lds, stream, x_fp8, w_fp8, (int)M,
-                           (int)N, (int)K, inv, bias, output);
-      return hipGetLastError();
-    }
-    // K % 128 == 0: copies without per-lane bounds tests (copy_offset; the 128x256 form
-    // measured no faster with them dropped).
-    if (N % 8 == 0 && (o & 15) == 0 && K % WBK == 0)
-      hipLaunchKernelGGL((fp8_gemm_wide<2, true>), dim3(tiles), dim3(kThreads), wide_lds, stream, x_fp8, w_fp8,
-                         (int)M, (int)N, (int)K, inv, bias, output);
-    else if (N % 8 == 0 && (o & 15) == 0)
-      hipLaunchKernelGGL(fp8_gemm_wide<2>, dim3(tiles), dim3(kThreads), wide_lds, stream, x_fp8, w_fp8,
-                         (int)M, (int)N, (int)K, inv, bias, output);
+  const size_t wide_lds = kWideLdsBytes;
+  const uintptr_t o = reinterpret_cast<uintptr_t>(output);
+  if (2 * tiles <= device_cu_count()) {
+    // At most half a 256x256 tile per CU: 128x256 tiles, twice as many workgroups.
+    const dim3 hgrid(((M + kHalfRows - 1) / kHalfRows) * ((N + BN - 1) / BN));
+    const size_t half_lds = kHalfLaunchLdsBytes;
+    if (N % 8 == 0 && (o & 15) == 0)
+      hipLaunchKernelGGL(fp8_gemm_half<2>, hgrid, dim3(kThreads), half_lds, stream, x_fp8, w_fp8, (int)M,
+                         (int)N, (int)K, inv, bias, output);
     else if (N % 4 == 0 && (o & 7) == 0)
-      hipLaunchKernelGGL(fp8_gemm_wide<1>, dim3(tiles), dim3(kThreads), wide_lds, stream, x_fp8, w_fp8,
-                         (int)M, (int)N, (int)K, inv, bias, output);
+      hipLaunchKernelGGL(fp8_gemm_half<1>, hgrid, dim3(kThreads), half_lds, stream, x_fp8, w_fp8, (int)M,
+                         (int)N, (int)K, inv, bias, output);
     else
-      hipLaunchKernelGGL(fp8_gemm_wide<0>, dim3(tiles), dim3(kThreads), wide_lds, stream, x_fp8, w_fp8,
-                         (int)M, (int)N, (int)K, inv, bias, output);
+      hipLaunchKernelGGL(fp8_gemm_half<0>, hgrid, dim3(kThreads), half_lds, stream, x_fp8, w_fp8, (int)M,
+                         (int)N, (int)K, inv, bias, output);
     return hipGetLastError();
   }
-  if (vec == 8)
-    hipLaunchKernelGGL(fp8_gemm_tiled<8>, dim3(tiles), dim3(kThreads), lds, stream, x_fp8, w_fp8,
+  // K % 128 == 0: copies without per-lane bounds tests (copy_offset; the 128x256 form
+  // measured no faster with them dropped).
+  if (N % 8 == 0 && (o & 15) == 0 && K % WBK == 0)
+    hipLaunchKernelGGL((fp8_gemm_wide<2, true>), dim3(tiles), dim3(kThreads), wide_lds, stream, x_fp8, w_fp8,
+                       (int)M, (int)N, (int)K, inv, bias, output);
+  else if (N % 8 == 0 && (o & 15) == 0)
+    hipLaunchKernelGGL(fp8_gemm_wide<2>, dim3(tiles), dim3(kThreads), wide_lds, stream, x_fp8, w_fp8,
+                       (int)M, (int)N, (int)K, inv, bias, output);
+  else if (N % 4 == 0 && (o & 7) == 0)
+    hipLaunchKernelGGL(fp8_gemm_wide<1>, dim3(tiles), dim3(kThreads), wide_lds, stream, x_fp8, w_fp8,
                        (int)M, (int)N, (int)K, inv, bias, output);
   else
-    hipLaunchKernelGGL(fp8_gemm_tiled<1>, dim3(tiles), dim3(kThreads), lds, stream, x_fp8, w_fp8,
+    hipLaunchKernelGGL(fp8_gemm_wide<0>, dim3(tiles), dim3(kThreads), wide_lds, stream, x_fp8, w_fp8,
                        (int)M, (int)N, (int)K, inv, bias, output);
   return hipGetLastError();
 }

@@ -12,21 +12,16 @@
 // The product is accumulated in fp32 and the epilogue applies 1/(sx*sw), adds the bf16
 // bias and rounds to bf16 (nearest-even) once.
 //
-// Three kernels, one launch per call:
-//  * wide (M > 64, K % 16 == 0, 16-byte aligned operands): the main path, described at
-//    fp8_gemm_wide below — direct-to-LDS copies of whole 128-byte row segments into two
-//    64 KiB stages, 32x32x64 MFMAs with fragments read a half-step ahead.  Grids of at
-//    most half a 256x256 tile per CU take its 128x256-tile form, fp8_gemm_half.
-//  * tiled (M > 64, other K or alignment): 256x256 output tile per workgroup of 4 waves (one per SIMD, each
-//    128x128 = 8x8 MFMA blocks whose 256 fp32 accumulators sit in AGPRs), K in steps of
-//    128 staged through LDS (2 stages x 64 KiB, 16-byte
-//    chunks XOR-swizzled by row so a wave's fragment reads spread over the banks).  The
-//    next K-step's global loads are in flight while the current one feeds the MFMAs.
-//    Workgroups are mapped so that each XCD's 32 concurrent tiles form a 4x8 block of
-//    the output and share A/B panels in that XCD's L2.
-//  * skinny (M <= 64): the weight-streaming case.  A workgroup owns 16 output columns
-//    and all M rows; its 8 waves split K, read W straight from global memory into MFMA
-//    fragments, and reduce their partial tiles through LDS in a fixed order.
+// Three families, one launch per call (fp8_linear.hip chooses):
+//  * wide (K % 16 == 0, 16-byte aligned operands): the large-matrix path, described at
+//    fp8_gemm_wide below — direct-to-LDS copies of whole 128-byte row segments, 32x32x64 MFMAs
+//    with fragments read a half-step ahead.  Grids of at most half a 256x256 tile per CU take
+//    its 128x256-tile form, fp8_gemm_half.
+//  * mid (fp8_linear_mid.hpp): tiles of 64x64 to 128x128 for grids that even the 128x256 form
+//    leaves mostly idle, and for other K and alignments.
+//  * skinny (small M): the weight-streaming case.  A workgroup owns 16 output columns and all M
+//    rows; its 8 waves split K, read W into MFMA fragments, and reduce their partial tiles
+//    through LDS in a fixed order.
 #pragma once
 
 #include "common.hpp"
@@ -74,51 +69,25 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, si
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, n, kRawBufferFlags);
 }
 
-// 16 bytes of a K-contiguous row starting at column k, zero past K.  `off` is the byte
-// offset of (row, k) in the descriptor, or kOutOfRange for rows past the matrix.
-// kVec 16: K % 16 == 0, a chunk is wholly inside or outside K; 8: K % 8 == 0, two
-// independent halves; 1: any K, byte by byte.
-template <int kVec>
-__device__ __forceinline__ i32x4 load16(__amdgpu_buffer_rsrc_t r, unsigned off, int k, int K) {
-  if constexpr (kVec == 16) {
-    const unsigned o = k < K ? off : kOutOfRange;
-    return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, 0));
-  } else if constexpr (kVec == 8) {
-    const unsigned o0 = k < K ? off : kOutOfRange;
-    const unsigned o1 = k + 8 < K ? off + 8 : kOutOfRange;
-    const i32x2 lo = __builtin_bit_cast(i32x2, __builtin_amdgcn_raw_buffer_load_b64(r, o0, 0, 0));
-    const i32x2 hi = __builtin_bit_cast(i32x2, __builtin_amdgcn_raw_buffer_load_b64(r, o1, 0, 0));
-    return i32x4{lo.x, lo.y, hi.x, hi.y};
-  } else {
-    unsigned w[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const unsigned o = (k + i < K && off != kOutOfRange) ? off + i : kOutOfRange;
-      w[i / 4] |= (unsigned)__builtin_amdgcn_raw_buffer_load_b8(r, o, 0, 0) << (8 * (i % 4));
-    }
-    return i32x4{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
-  }
+// 16 bytes of a K-contiguous row starting at column k, zero past K (K % 8 == 0 and rows 8-byte
+// aligned: two independent halves).  `off` is the byte offset of (row, k) in the descriptor,
+// or kOutOfRange for rows past the matrix.
+__device__ __forceinline__ i32x4 load8x2(__amdgpu_buffer_rsrc_t r, unsigned off, int k, int K) {
+  const unsigned o0 = k < K ? off : kOutOfRange;
+  const unsigned o1 = k + 8 < K ? off + 8 : kOutOfRange;
+  const i32x2 lo = __builtin_bit_cast(i32x2, __builtin_amdgcn_raw_buffer_load_b64(r, o0, 0, 0));
+  const i32x2 hi = __builtin_bit_cast(i32x2, __builtin_amdgcn_raw_buffer_load_b64(r, o1, 0, 0));
+  return i32x4{lo.x, lo.y, hi.x, hi.y};
 }
 
 __device__ __forceinline__ i32x8 join(i32x4 a, i32x4 b) {
   return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-// ---------------------------------------------------------------------------------------
-// Tiled kernel
-// ---------------------------------------------------------------------------------------
-constexpr int BM = 256, BN = 256, BK = 128;
+constexpr int BM = 256, BN = 256;
 constexpr int kThreads = 256;
 constexpr int kWavesN = 2;                       // waves arranged 2 (M) x 2 (N)
-constexpr int WM = 128, WN = 128;                // wave tile
-constexpr int kMI = WM / 16, kNJ = WN / 16;      // 16x16 MFMA blocks per wave tile
-constexpr int kStageBytes = (BM + BN) * BK;  // 64 KiB: A tile then B tile
-constexpr int kChunksPerRow = BK / 16;       // 8
-constexpr int kLoadsPerThread = BM * kChunksPerRow / kThreads;  // 16-byte chunks per operand
-
-__device__ __forceinline__ int swizzle(int row, int chunk) {
-  return row * BK + ((chunk ^ (row & 7)) << 4);
-}
+constexpr int WM = 128, WN = 128;                // wave tile of the 256x256 form
 
 // Output tile of workgroup `b` (a bijection onto the tm x tn tiles for any tile counts).
 // Workgroups are dispatched to the 8 XCDs round-robin (b % 8), so when the tile count is
@@ -136,108 +105,6 @@ __device__ __forceinline__ void tile_of(int b, int tm, int tn, int& mt, int& nt)
   const int r = v % per_group;
   mt = first_m + r % rows;
   nt = r / rows;
-}
-
-template <int kVec>
-__global__ __launch_bounds__(kThreads) void fp8_gemm_tiled(
-    const uint8_t* __restrict__ x, const uint8_t* __restrict__ w, int M, int N, int K,
-    float inv_scale, const uint16_t* __restrict__ bias, uint16_t* __restrict__ out) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
-  int mt, nt;
-  tile_of(blockIdx.x, tm, tn, mt, nt);
-  const int m0 = mt * BM, n0 = nt * BN;
-  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int wm = wave / kWavesN, wn = wave % kWavesN;  // wave tile origin (wm*WM, wn*WN)
-  const int rows_a = min(BM, M - m0), rows_b = min(BN, N - n0);
-  const __amdgpu_buffer_rsrc_t xa = make_rsrc(x + (size_t)m0 * K, (size_t)rows_a * K);
-  const __amdgpu_buffer_rsrc_t wb = make_rsrc(w + (size_t)n0 * K, (size_t)rows_b * K);
-
-  i32x4 ra[kLoadsPerThread], rb[kLoadsPerThread];
-  auto gload = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < kLoadsPerThread; ++i) {
-      const int q = tid + kThreads * i;
-      const int row = q / kChunksPerRow, chunk = q % kChunksPerRow;
-      const int gk = k0 + chunk * 16;
-      const unsigned off = (unsigned)(row * K + gk);
-      ra[i] = load16<kVec>(xa, row < rows_a ? off : kOutOfRange, gk, K);
-      rb[i] = load16<kVec>(wb, row < rows_b ? off : kOutOfRange, gk, K);
-    }
-  };
-  auto swrite = [&](int stage) {
-    uint8_t* As = smem + stage * kStageBytes;
-    uint8_t* Bs = As + BM * BK;
-#pragma unroll
-    for (int i = 0; i < kLoadsPerThread; ++i) {
-      const int q = tid + kThreads * i;
-      const int row = q / kChunksPerRow, chunk = q % kChunksPerRow;
-      *reinterpret_cast<i32x4*>(As + swizzle(row, chunk)) = ra[i];
-      *reinterpret_cast<i32x4*>(Bs + swizzle(row, chunk)) = rb[i];
-    }
-  };
-
-  f32x4 acc[kMI][kNJ];
-#pragma unroll
-  for (int i = 0; i < kMI; ++i)
-#pragma unroll
-    for (int j = 0; j < kNJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int nk = (K + BK - 1) / BK;
-  gload(0);
-  swrite(0);
-  __syncthreads();
-  const int fr = lane % 16, fg = lane / 16;  // fragment row and k-group of this lane
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < nk) gload((kt + 1) * BK);
-    const uint8_t* As = smem + cur * kStageBytes;
-    const uint8_t* Bs = As + BM * BK;
-    i32x8 bf[kNJ];
-#pragma unroll
-    for (int j = 0; j < kNJ; ++j) {
-      const int row = wn * WN + j * 16 + fr;
-      bf[j] = join(*reinterpret_cast<const i32x4*>(Bs + swizzle(row, 2 * fg)),
-                   *reinterpret_cast<const i32x4*>(Bs + swizzle(row, 2 * fg + 1)));
-    }
-#pragma unroll
-    for (int i = 0; i < kMI; ++i) {
-      const int row = wm * WM + i * 16 + fr;
-      const i32x8 af = join(*reinterpret_cast<const i32x4*>(As + swizzle(row, 2 * fg)),
-                            *reinterpret_cast<const i32x4*>(As + swizzle(row, 2 * fg + 1)));
-#pragma unroll
-      for (int j = 0; j < kNJ; ++j) acc[i][j] = mfma_e4m3(af, bf[j], acc[i][j]);
-    }
-    if (kt + 1 < nk) swrite(cur ^ 1);
-    __syncthreads();
-  }
-
-  // Epilogue: lane holds rows 4*fg..4*fg+3 of column fr in every 16x16 block.  Stores go
-  // through a descriptor covering this tile's rows; columns past N get an out-of-range
-  // offset and are dropped.
-  // All bias loads are issued before the first store: vmcnt also counts stores, so a load
-  // between stores would wait for every earlier store to complete.
-  const __amdgpu_buffer_rsrc_t ob = make_rsrc(out + (size_t)m0 * N, (size_t)rows_a * N * 2);
-  float bvs[kNJ];
-#pragma unroll
-  for (int j = 0; j < kNJ; ++j) {
-    const int gn = n0 + wn * WN + j * 16 + fr;
-    bvs[j] = gn < N ? bf16_to_f32(bias[gn]) : 0.0f;
-  }
-#pragma unroll
-  for (int j = 0; j < kNJ; ++j) {
-    const int gn = n0 + wn * WN + j * 16 + fr;
-    const float bv = bvs[j];
-#pragma unroll
-    for (int i = 0; i < kMI; ++i) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = wm * WM + i * 16 + 4 * fg + r;
-        const unsigned off = gn < N ? (unsigned)(row * N + gn) * 2u : kOutOfRange;
-        __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16_rne(acc[i][j][r] * inv_scale + bv), ob, off, 0, 0);
-      }
-    }
-  }
 }
 
 constexpr int kSlotsPerInst = 64;  // a direct-to-LDS instruction writes 64 x 16 bytes
@@ -385,8 +252,7 @@ __device__ __forceinline__ unsigned short load_bias(const uint16_t* bias, int n0
 // barrier at its mid-step), and its w copies during the second half, into the slot step kt
 // left at this mid-step; one copy per two MFMAs throughout.  Row r's 16-byte chunk c sits
 // at chunk c ^ ((r >> 1) & 7), which spreads any 16 consecutive rows of one chunk over all
-// banks.  Accumulation order is k ascending in 64-wide MFMA steps, as in the tiled
-// kernel's 128-wide steps of two 64-wide halves.
+// banks.  Accumulation order is k ascending in 64-wide MFMA steps.
 // ---------------------------------------------------------------------------------------
 constexpr int WBK = 128;
 constexpr int kWideOperandBytes = BM * WBK;                          // 32 KiB per operand and step
@@ -719,8 +585,7 @@ __device__ __forceinline__ int skinny_block(int b, int nb) {
   return 4 * (x + 8 * (j / 4)) + j % 4;
 }
 
-template <int kVec>
-__global__ __launch_bounds__(kSkinnyThreads) void fp8_gemm_skinny(
+static __global__ __launch_bounds__(kSkinnyThreads) void fp8_gemm_skinny(
     const uint8_t* __restrict__ x, const uint8_t* __restrict__ w, int M, int N, int K,
     float inv_scale, const uint16_t* __restrict__ bias, uint16_t* __restrict__ out) {
   __shared__ float part[kSkinnyWaves][kSkinnyMaxM][16];
@@ -742,13 +607,13 @@ __global__ __launch_bounds__(kSkinnyThreads) void fp8_gemm_skinny(
   for (int s = s0; s < s1; ++s) {
     const int k = s * 128 + 32 * fg;
     const unsigned wo = woff == kOutOfRange ? kOutOfRange : woff + k;
-    const i32x8 bf = join(load16<kVec>(wb, wo, k, K), load16<kVec>(wb, wo + 16, k + 16, K));
+    const i32x8 bf = join(load8x2(wb, wo, k, K), load8x2(wb, wo + 16, k + 16, K));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (i < rblocks) {
         const int gm = i * 16 + fr;
         const unsigned xo = gm < M ? (unsigned)(gm * K + k) : kOutOfRange;
-        const i32x8 af = join(load16<kVec>(xa, xo, k, K), load16<kVec>(xa, xo + 16, k + 16, K));
+        const i32x8 af = join(load8x2(xa, xo, k, K), load8x2(xa, xo + 16, k + 16, K));
         acc[i] = mfma_e4m3(af, bf, acc[i]);
       }
     }
@@ -868,6 +733,11 @@ __global__ __launch_bounds__(kSkinnyThreads) void fp8_gemm_skinny_flat(
     out[(size_t)m * N + n] = f32_to_bf16_rne(s * inv_scale + bias_v);
   }
 }
+
+// The middle kernel's tiles (fp8_linear_mid.hip).
+enum MidTile : int { kTile64x64, kTile64x128, kTile128x128 };
+hipError_t mid_launch(MidTile tile, bool direct, const uint8_t* x, const uint8_t* w, int M, int N, int K, float inv,
+                      const uint16_t* bias, uint16_t* out, hipStream_t stream);
 
 inline int vec_width(const uint8_t* x, const uint8_t* w, int K) {
   const uintptr_t bits = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w);
