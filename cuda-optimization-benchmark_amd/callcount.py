@@ -91,8 +91,8 @@ EXPECTED_LAUNCHES = {
     "efficient_kan_one_chunk": 1,  # kan_direct alone: the features are not split
     "efficient_kan_rowwise": 1,  # kan_rowwise (spline order 0 or above 4)
     "fp8_linear": 1,
-    "quantize_e4m3": 2,          # qz_amax + qz_cast (unaligned, or more chunks than fit at once)
-    "quantize_e4m3_fused": 1,    # qz_fused (aligned, every chunk resident at once)
+    "quantize_e4m3": 2,          # qz_amax + qz_cast (unaligned, or more than 134 M elements)
+    "quantize_e4m3_fused": 1,    # qz_fused or qz_hold (aligned)
 }
 
 
@@ -146,9 +146,9 @@ def workloads():
         out.append((f"efficient_kan/{case['name']}", "efficient_kan",
                     "efficient_kan_rowwise" if order > 4 else "efficient_kan", drop_in("efficient_kan", case)))
     out.append(("quantize_e4m3/aligned_n1000003", "quantize_e4m3", "quantize_e4m3_fused", quant(1_000_003, 0)))
-    # 4096 x 4096, the fused path's whole resident capacity: still one launch.
+    # 4096 x 4096, qz_fused's whole resident capacity; then qz_hold, past what it holds.
     out.append(("quantize_e4m3/aligned_n16777216", "quantize_e4m3", "quantize_e4m3_fused", quant(1 << 24, 0)))
-    out.append(("quantize_e4m3/aligned_n67108864", "quantize_e4m3", "quantize_e4m3", quant(1 << 26, 0)))
+    out.append(("quantize_e4m3/aligned_n67108864", "quantize_e4m3", "quantize_e4m3_fused", quant(1 << 26, 0)))
     out.append(("quantize_e4m3/unaligned_n4099", "quantize_e4m3", "quantize_e4m3", quant(4099, 1)))
     return out
 

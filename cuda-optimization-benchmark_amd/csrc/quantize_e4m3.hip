@@ -11,9 +11,9 @@
 // as raw bits: for |x| the IEEE order is the unsigned-integer order and every NaN sorts
 // above inf, so an integer max propagates NaN.  Conversion is v_cvt_pk_fp8_f32.
 //
-// Two launches (unaligned operands, or more chunks than can be resident at once): qz_amax
-// writes one partial max per workgroup; qz_cast reduces those partials (a few KiB from L2),
-// derives the scale and converts, reading x a second time.
+// Two launches (unaligned operands, or the largest tensors): qz_amax writes one partial max per
+// workgroup; qz_cast reduces those partials (a few KiB from L2), derives the scale and converts,
+// reading x a second time.
 //
 // The kernels walk x in chunks of 16384 elements per 512-thread workgroup and step.  A
 // thread issues all 8 of its 16-byte loads of a chunk before it uses any (32 floats in
@@ -24,14 +24,14 @@
 // loads was 17.83-17.84 us per fused call against 17.58-17.61 (A/B on two boxes, same
 // bits); 512 x 16 and 1024 x 8 were in between, 1024 x 16 slower (22.4).
 //
-// One launch (qz_fused, when the grid fits the resident capacity): each workgroup keeps its
-// chunk in registers, the workgroups combine their maxima through a grid barrier, and each
-// converts the chunk it holds, so x is read once.  The barrier is a plain launch sized by
-// the occupancy API (a cooperative launch, which guarantees residency, costs about 100 us
-// per launch on this stack).  Residency is not guaranteed (another stream's kernels can
-// hold CUs), so the wait is bounded: a workgroup that times out reads all of x for the max
-// itself.  The max is exact and order-free, so both paths give identical bits, every wave
-// exits, and no result depends on the timing.
+// One launch (qz_fused while every chunk has a resident workgroup of its own, qz_hold beyond):
+// each workgroup keeps its chunks in registers (and LDS), the workgroups combine their maxima
+// through a grid barrier, and each converts the chunks it holds, so x is read once.  The
+// barrier is a plain launch sized by the occupancy API (a cooperative launch, which guarantees
+// residency, costs about 100 us per launch on this stack).  Residency is not guaranteed
+// (another stream's kernels can hold CUs), so the wait is bounded: a workgroup that times out
+// reads all of x for the max itself.  The max is exact and order-free, so both paths give
+// identical bits, every wave exits, and no result depends on the timing.
 #include "common.hpp"
 
 namespace taskops {
@@ -64,32 +64,40 @@ __device__ __forceinline__ unsigned block_max_u32(unsigned v, unsigned* lds) {
   return m;
 }
 
-// This thread's 64 elements of the chunk at `base` (x 16-byte aligned); elements at or
-// beyond n read as 0, which never raises the max.
+// Vectors k0 .. k0 + kN - 1 of this thread's part of the whole chunk at `base` (x 16-byte
+// aligned).  kNT: non-temporal.
+template <int kN, bool kNT>
+__device__ __forceinline__ void load_whole(const float* __restrict__ x, int64_t base, int k0, f32x4 (&v)[kN]) {
+  const f32x4* p = reinterpret_cast<const f32x4*>(x + base) + threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < kN; ++k)
+    v[k] = kNT ? __builtin_nontemporal_load(p + (k0 + k) * kThreads) : p[(k0 + k) * kThreads];
+}
+
+// Four elements at i; those at or beyond n read as 0, which never raises the max.
+__device__ __forceinline__ f32x4 load_tail4(const float* __restrict__ x, int64_t n, int64_t i) {
+  if (i + 4 <= n) return *reinterpret_cast<const f32x4*>(x + i);
+  f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (i < n) v.x = x[i];
+  if (i + 1 < n) v.y = x[i + 1];
+  if (i + 2 < n) v.z = x[i + 2];
+  return v;
+}
+
+// This thread's 32 elements of the chunk at `base`, whole or not.
 __device__ __forceinline__ void load_chunk(const float* __restrict__ x, int64_t n, int64_t base, f32x4 (&v)[kVecs]) {
   if (base + kChunk <= n) {
-    const f32x4* p = reinterpret_cast<const f32x4*>(x + base) + threadIdx.x;
-#pragma unroll
-    for (int k = 0; k < kVecs; ++k) v[k] = __builtin_nontemporal_load(p + k * kThreads);
+    load_whole<kVecs, true>(x, base, 0, v);
     return;
   }
 #pragma unroll
-  for (int k = 0; k < kVecs; ++k) {
-    const int64_t i = base + 4 * ((int64_t)k * kThreads + threadIdx.x);
-    if (i + 4 <= n) {
-      v[k] = *reinterpret_cast<const f32x4*>(x + i);
-    } else {
-      v[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      if (i < n) v[k].x = x[i];
-      if (i + 1 < n) v[k].y = x[i + 1];
-      if (i + 2 < n) v[k].z = x[i + 2];
-    }
-  }
+  for (int k = 0; k < kVecs; ++k) v[k] = load_tail4(x, n, base + 4 * ((int64_t)k * kThreads + threadIdx.x));
 }
 
-__device__ __forceinline__ unsigned chunk_max(const f32x4 (&v)[kVecs], unsigned m) {
+template <int kN>
+__device__ __forceinline__ unsigned chunk_max(const f32x4 (&v)[kN], unsigned m) {
 #pragma unroll
-  for (int k = 0; k < kVecs; ++k)
+  for (int k = 0; k < kN; ++k)
     m = max(max(m, max(abs_bits(v[k].x), abs_bits(v[k].y))), max(abs_bits(v[k].z), abs_bits(v[k].w)));
   return m;
 }
@@ -125,25 +133,31 @@ __device__ __forceinline__ float scale_from(unsigned m) {
 // stores are non-temporal (each instruction writes 256 contiguous bytes, whole lines), so
 // the codes do not sit dirty in the L2s for the end of the kernel to write back: 19.5-19.6
 // -> 17.6-17.7 us per call at 4096 x 4096 (A/B on one box, both orders, same bits).
+__device__ __forceinline__ void store_whole(uint8_t* __restrict__ q, int64_t base, const f32x4 (&v)[kVecs], float scale) {
+  unsigned* out = reinterpret_cast<unsigned*>(q + base) + threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < kVecs; ++k) __builtin_nontemporal_store(cvt4(v[k], scale), out + k * kThreads);
+}
+
+// The codes of four elements at i, those below n.
+__device__ __forceinline__ void store_tail4(uint8_t* __restrict__ q, int64_t n, int64_t i, f32x4 v, float scale) {
+  const unsigned w = cvt4(v, scale);
+  if (i + 4 <= n) {
+    *reinterpret_cast<unsigned*>(q + i) = w;
+  } else {
+    for (int c = 0; c < 3; ++c)
+      if (i + c < n) q[i + c] = (uint8_t)(w >> (8 * c));
+  }
+}
+
 __device__ __forceinline__ void store_chunk(uint8_t* __restrict__ q, int64_t n, int64_t base,
                                             const f32x4 (&v)[kVecs], float scale) {
   if (base + kChunk <= n) {
-    unsigned* out = reinterpret_cast<unsigned*>(q + base) + threadIdx.x;
-#pragma unroll
-    for (int k = 0; k < kVecs; ++k) __builtin_nontemporal_store(cvt4(v[k], scale), out + k * kThreads);
+    store_whole(q, base, v, scale);
     return;
   }
 #pragma unroll
-  for (int k = 0; k < kVecs; ++k) {
-    const int64_t i = base + 4 * ((int64_t)k * kThreads + threadIdx.x);
-    const unsigned w = cvt4(v[k], scale);
-    if (i + 4 <= n) {
-      *reinterpret_cast<unsigned*>(q + i) = w;
-    } else {
-      for (int c = 0; c < 3; ++c)
-        if (i + c < n) q[i + c] = (uint8_t)(w >> (8 * c));
-    }
-  }
+  for (int k = 0; k < kVecs; ++k) store_tail4(q, n, base + 4 * ((int64_t)k * kThreads + threadIdx.x), v[k], scale);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -253,24 +267,19 @@ __device__ __forceinline__ unsigned qz_add(unsigned* p) {
   return __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Requires x 16-byte and q 4-byte aligned and gridDim.x = ceil(n / kChunk).  Thread 0 of
-// each workgroup runs the barrier; every RMW's returned value is used before the next
-// one is issued, which orders them at the coherence point.  8 waves per SIMD (at most 64
-// VGPRs) make 4 workgroups per CU resident, 1024 on 256 CUs: a 4096 x 4096 operand's chunks.
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) void qz_fused(
-    const float* __restrict__ x, int64_t n, uint8_t* __restrict__ q, float* __restrict__ scale_out,
-    unsigned* __restrict__ bar, unsigned spin_limit) {
-  __shared__ unsigned lds[kThreads / kWave];
-  __shared__ unsigned gmax_s, fallback_s;
-  const int64_t base = (int64_t)blockIdx.x * kChunk;
-  f32x4 v[kVecs];
-  load_chunk(x, n, base, v);
-  // The parity is read behind the chunk's loads; it only has to be read before this
-  // workgroup arrives.
-  unsigned parity = 0u;
-  if (threadIdx.x == 0) parity = qz_load(qz_parity(bar));
-  const unsigned m = block_max_u32(chunk_max(v, 0u), lds);
+// The barrier's words in LDS.
+struct QzShared {
+  unsigned lds[kThreads / kWave];
+  unsigned gmax, fallback;
+};
 
+// The max bits of all of x, from this workgroup's `m` (called by every thread; parity: thread
+// 0's read of the parity word).  Thread 0 of each workgroup runs the barrier; every RMW's
+// returned value is used before the next one is issued, which orders them at the coherence
+// point.
+__device__ __forceinline__ unsigned qz_grid_max(unsigned m, unsigned parity, unsigned* bar, unsigned spin_limit,
+                                                const float* __restrict__ x, int64_t n, QzShared* sh) {
+  m = block_max_u32(m, sh->lds);
   if (threadIdx.x < kWave) {  // wave 0 runs the barrier; lane 0 makes the RMWs
     const int lane = threadIdx.x;
     parity = (unsigned)__shfl((int)parity, 0, kWave);
@@ -303,47 +312,153 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) v
     unsigned gm = 0u;
     if (done) gm = wave_max_u32((unsigned)lane < groups ? qz_load(qz_word(bar, set, kQzGroupMax, lane)) : 0u);
     if (lane == 0) {
-      fallback_s = done ? 0u : 1u;
-      gmax_s = gm;
+      sh->fallback = done ? 0u : 1u;
+      sh->gmax = gm;
     }
   }
   __syncthreads();
-  unsigned gm = gmax_s;
-  if (fallback_s) {  // the barrier did not complete in time: this workgroup finds the max itself
-    unsigned mm = 0u;    // (one 16-byte load at a time: the chunk in v stays in registers)
+  unsigned gm = sh->gmax;
+  if (sh->fallback) {  // the barrier did not complete in time: this workgroup finds the max itself
+    unsigned mm = 0u;    // (one 16-byte load at a time: the held chunks stay in registers)
     const int64_t n4 = n & ~(int64_t)3;
     for (int64_t i = 4 * (int64_t)threadIdx.x; i < n4; i += 4 * kThreads) {
       const f32x4 w = *reinterpret_cast<const f32x4*>(x + i);
       mm = max(max(mm, max(abs_bits(w.x), abs_bits(w.y))), max(abs_bits(w.z), abs_bits(w.w)));
     }
     if ((int64_t)threadIdx.x < n - n4) mm = max(mm, abs_bits(x[n4 + threadIdx.x]));
-    gm = block_max_u32(mm, lds);
+    gm = block_max_u32(mm, sh->lds);
   }
-  const float scale = scale_from(gm);
+  return gm;
+}
+
+// Requires x 16-byte and q 4-byte aligned and gridDim.x = ceil(n / kChunk).  8 waves per SIMD
+// (at most 64 VGPRs) make 4 workgroups per CU resident, 1024 on 256 CUs: a 4096 x 4096
+// operand's chunks.
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) void qz_fused(
+    const float* __restrict__ x, int64_t n, uint8_t* __restrict__ q, float* __restrict__ scale_out,
+    unsigned* __restrict__ bar, unsigned spin_limit) {
+  __shared__ QzShared sh;
+  const int64_t base = (int64_t)blockIdx.x * kChunk;
+  f32x4 v[kVecs];
+  load_chunk(x, n, base, v);
+  // The parity is read behind the chunk's loads; it only has to be read before this
+  // workgroup arrives.
+  unsigned parity = 0u;
+  if (threadIdx.x == 0) parity = qz_load(qz_parity(bar));
+  const float scale = scale_from(qz_grid_max(chunk_max(v, 0u), parity, bar, spin_limit, x, n, &sh));
   if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = scale;
   store_chunk(q, n, base, v, scale);
 }
 
-unsigned g_qz_spin_limit = kQzSpinDefault;
-int g_qz_capacity[64];  // resident qz_fused workgroups per device (0: not yet known, -1: none)
+// Larger tensors, one launch too: a workgroup holds up to four chunks, three in registers and
+// one in LDS, so 512 resident workgroups (4 waves per SIMD, at most 128 VGPRs, 2 per CU) hold
+// 2048 chunks, 33.5 M elements, and read them once.  The chunks are loaded one after another,
+// the LDS one in halves: with all of them in flight at once the reads themselves were slower
+// (42.1 us at 8192 x 4096).  Chunks past the held ones ("rest") are read before
+// them for the max and again after them for the codes, the last first, with ordinary loads, so
+// that what the Infinity Cache kept of them is found there.
+// Only whole chunks are held (with the element tests of a part chunk in every load the kernel
+// spilled registers, 40 us); the last workgroup reads the part chunk twice.
+// us per call against the two launches: 21 M elements 21.2 / 33.6, 33.5 M 31.3 / 48.9 (168 MB: the
+// floor is 33 at a copy's 5.1 TB/s), 41 M 39.4 / 59.9, 67 M 77.0 / 95.3, 98 M 118.9 / 139.8.
+constexpr int kHeldRegs = 3;
+constexpr int kHeld = kHeldRegs + 1;
+__device__ __forceinline__ void finish_loads(unsigned& m) {  // nothing loaded later starts before m is known
+  asm volatile("" : "+v"(m)::"memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void qz_hold(
+    const float* __restrict__ x, int64_t n, uint8_t* __restrict__ q, float* __restrict__ scale_out,
+    unsigned* __restrict__ bar, unsigned spin_limit) {
+  __shared__ QzShared sh;
+  extern __shared__ __attribute__((aligned(16))) f32x4 held[];  // [kVecs][kThreads]
+  const int64_t stride = (int64_t)gridDim.x * kChunk, first = (int64_t)blockIdx.x * kChunk;
+  const int64_t whole = n - n % kChunk;  // the last workgroup also takes the part chunk from here on
+  const bool tail = blockIdx.x == gridDim.x - 1;
+  unsigned m = 0u;
+  int64_t rest = first + kHeld * stride;
+  for (; rest < whole; rest += stride) {
+    f32x4 v[kVecs];
+    load_whole<kVecs, false>(x, rest, 0, v);
+    m = chunk_max(v, m);
+  }
+  if (tail)
+    for (int64_t i = whole + 4 * (int64_t)threadIdx.x; i < n; i += 4 * kThreads) {
+      const f32x4 v[1] = {load_tail4(x, n, i)};
+      m = chunk_max(v, m);
+    }
+  f32x4 r[kHeldRegs][kVecs];
+#pragma unroll
+  for (int c = 0; c < kHeldRegs; ++c) {
+    const int64_t base = first + (c + 1) * stride;
+    if (base < whole) {
+      load_whole<kVecs, true>(x, base, 0, r[c]);
+      m = chunk_max(r[c], m);
+    }
+    finish_loads(m);
+  }
+  if (first < whole) {
+#pragma unroll
+    for (int k0 = 0; k0 < kVecs; k0 += kVecs / 2) {
+      f32x4 v[kVecs / 2];
+      load_whole<kVecs / 2, true>(x, first, k0, v);
+      m = chunk_max(v, m);
+#pragma unroll
+      for (int k = 0; k < kVecs / 2; ++k) held[(k0 + k) * kThreads + threadIdx.x] = v[k];
+      finish_loads(m);
+    }
+  }
+  unsigned parity = 0u;
+  if (threadIdx.x == 0) parity = qz_load(qz_parity(bar));
+  const float scale = scale_from(qz_grid_max(m, parity, bar, spin_limit, x, n, &sh));
+  if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = scale;
+#pragma unroll
+  for (int c = 0; c < kHeldRegs; ++c) {
+    const int64_t base = first + (c + 1) * stride;
+    if (base < whole) store_whole(q, base, r[c], scale);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  f32x4 v[kVecs];
+  if (first < whole) {
+#pragma unroll
+    for (int k = 0; k < kVecs; ++k) v[k] = held[k * kThreads + threadIdx.x];
+    store_whole(q, first, v, scale);
+  }
+  if (tail)
+    for (int64_t i = whole + 4 * (int64_t)threadIdx.x; i < n; i += 4 * kThreads)
+      store_tail4(q, n, i, load_tail4(x, n, i), scale);
+  for (rest -= stride; rest >= first + kHeld * stride; rest -= stride) {
+    load_whole<kVecs, false>(x, rest, 0, v);
+    store_whole(q, rest, v, scale);
+  }
+}
+constexpr size_t kHeldLds = (size_t)kChunk * sizeof(float);
+// Up to this many chunks per resident workgroup (134 M elements, four times what is held):
+// 174.6 us against 190.7 there, 388.8 / 387.3 at twice that, where the two launches, which wait
+// for nothing, keep the call.
+constexpr int kHoldMost = 16;
 
-int fused_capacity() {
+
+unsigned g_qz_spin_limit = kQzSpinDefault;
+int g_qz_capacity[2][64];  // resident qz_fused, qz_hold workgroups per device (0: not yet known, -1: none)
+
+int resident(int which, const void* kernel, size_t lds) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  int cap = __atomic_load_n(&g_qz_capacity[dev], __ATOMIC_RELAXED);
+  int cap = __atomic_load_n(&g_qz_capacity[which][dev], __ATOMIC_RELAXED);
   if (cap != 0) return cap > 0 ? cap : 0;
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(qz_fused), kThreads, 0) !=
-          hipSuccess ||
-      per_cu <= 0) {
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kThreads, lds) != hipSuccess || per_cu <= 0) {
     (void)hipGetLastError();
     cap = -1;
   } else {
     cap = per_cu * device_cu_count();
   }
-  __atomic_store_n(&g_qz_capacity[dev], cap, __ATOMIC_RELAXED);
+  __atomic_store_n(&g_qz_capacity[which][dev], cap, __ATOMIC_RELAXED);
   return cap > 0 ? cap : 0;
 }
+int fused_capacity() { return resident(0, reinterpret_cast<const void*>(qz_fused), 0); }
+int hold_capacity() { return resident(1, reinterpret_cast<const void*>(qz_hold), kHeldLds); }
 
 // Workgroups for n elements at `per_block` elements per step: enough for one step each,
 // at most `per_cu` per CU and kMaxPartials.
@@ -374,6 +489,12 @@ extern "C" hipError_t taskops_quantize_e4m3(const float* x, int64_t n, uint8_t* 
   if (vx && vq && chunks <= fused_capacity()) {
     hipLaunchKernelGGL(qz_fused, dim3((unsigned)chunks), dim3(kThreads), 0, stream, x, n, q, scale,
                        partial + kMaxPartials, g_qz_spin_limit);
+    return hipGetLastError();
+  }
+  const int hold = vx && vq ? hold_capacity() : 0;
+  if (hold > 0 && chunks <= (int64_t)kHoldMost * hold) {
+    hipLaunchKernelGGL(qz_hold, dim3((unsigned)(chunks < hold ? chunks : hold)), dim3(kThreads), kHeldLds, stream, x, n, q,
+                       scale, partial + kMaxPartials, g_qz_spin_limit);
     return hipGetLastError();
   }
   if (vx && vq) {
