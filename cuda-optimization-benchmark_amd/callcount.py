@@ -88,7 +88,7 @@ EXPECTED_LAUNCHES = {
     "pow_abs_sqrt_mean": 1, "leaky": 1, "reward_to_go": 1, "ppo_clip": 1, "ppo_clip_entropy": 1,
     "ppo_clip_entropy_noalloc": 1,  # its first call on a device adds the scratch clear
     "efficient_kan": 2,          # kan_pack + kan_fused, or kan_direct + kan_direct_sum
-    "efficient_kan_one_chunk": 1,  # kan_direct alone: the features are not split
+    "efficient_kan_direct": 1,   # kan_direct alone: features unsplit, or summed by the last arrival
     "efficient_kan_rowwise": 1,  # kan_rowwise (spline order 0 or above 4)
     "fp8_linear": 1,
     "quantize_e4m3": 2,          # qz_amax + qz_cast (unaligned, or more than 134 M elements)
@@ -133,7 +133,7 @@ def workloads():
         for case in tasks.all_cases(op):
             key = op
             if op == "efficient_kan" and case["B"] <= 16 and case["I"] <= 16:
-                key = "efficient_kan_one_chunk"
+                key = "efficient_kan_direct"
             out.append((f"{op}/{case['name']}", op, key, drop_in(op, case)))
             if op == "ppo_clip":
                 out.append((f"ppo_clip_entropy/{case['name']}", "ppo_clip_entropy", "ppo_clip_entropy",
@@ -144,7 +144,7 @@ def workloads():
         case = dict(name=f"B64_I40_O24_order{order}", seed=70 + order, small=True, timed=False,
                     B=64, I=40, O=24, spline_order=order)
         out.append((f"efficient_kan/{case['name']}", "efficient_kan",
-                    "efficient_kan_rowwise" if order > 4 else "efficient_kan", drop_in("efficient_kan", case)))
+                    "efficient_kan_rowwise" if order > 4 else "efficient_kan_direct", drop_in("efficient_kan", case)))
     out.append(("quantize_e4m3/aligned_n1000003", "quantize_e4m3", "quantize_e4m3_fused", quant(1_000_003, 0)))
     # 4096 x 4096, qz_fused's whole resident capacity; then qz_hold, past what it holds.
     out.append(("quantize_e4m3/aligned_n16777216", "quantize_e4m3", "quantize_e4m3_fused", quant(1 << 24, 0)))

@@ -168,12 +168,15 @@ hipError_t workspace_if_possible(WorkspaceSlot slot, size_t bytes, hipStream_t s
 // there is none, and the caller takes a path that needs none: while the stream is capturing
 // (a graph may be replayed beside other work), for hipStreamPerThread (one handle, many
 // streams), when kMaxScratchStreams other streams hold theirs, or when memory is short.
-// Not cleared.  Grown by doubling, kept until the process exits.
+// Not cleared, except for kScratchCounters arrival counters, which start at zero and which
+// every launch leaves at zero.  Grown by doubling, kept until the process exits.
 struct StreamScratch {
   StreamScratch(size_t bytes, hipStream_t stream);
   std::unique_lock<std::mutex> lock;
+  unsigned* counters = nullptr;
   void* ptr = nullptr;
 };
+constexpr int kScratchCounters = 1024;
 constexpr int kMaxScratchStreams = 8;
 
 // Number of compute units of the current device (cached per device).

@@ -13,6 +13,13 @@ using namespace kan_direct;
 // for missing rows, up to 4, which read each weight once per 64 rows.
 int row_blocks(int B) { return B <= 16 ? 1 : (B <= 32 ? 2 : 4); }
 
+// Up to this many splits the tile's last arrival adds them; it reads them all by itself, so
+// beyond that a second launch, spread over the chip, is faster although it costs 2 to 4 us: us
+// with one launch / two at 2 splits (B = 70, I = 5, O = 30, G = 7) 6.7 / 8.6, 6 (B = 1024, I = 256,
+// O = 512, G = 16) 66.3 / 71.6, 10 (B = 1, I = 77, O = 301, G = 23) 12.9 / 13.5, 26 (B = 6, I = 208, O = 448,
+// G = 20) 11.1 / 10.4, 42 (B = 20, I = 333, O = 131, G = 10) 12.1 / 11.5.
+constexpr int kMaxArrivals = 16;
+
 template <int kNQ, int kR>
 hipError_t launch(const float* x, const float* grid, const float* wb, const float* ws, const float* sc, int order,
                   int L, int C, int B, int I, int O, float* out, size_t shared_bytes, hipStream_t stream) {
@@ -26,30 +33,34 @@ hipError_t launch(const float* x, const float* grid, const float* wb, const floa
   const int per_cu = std::max(1, std::min<int>(4, (int)(device_lds_per_cu() / lds)));
   const int64_t tiles = (int64_t)mtiles * ctiles, want = (int64_t)per_cu * device_cu_count() / tiles;
   int nsplit = (int)std::min<int64_t>(nchunks, std::max<int64_t>(want, 1));
-  const size_t n = (size_t)B * O, bytes = nsplit * n * sizeof(float);
-  void* partial = nullptr;
+  const size_t per_split = (size_t)tiles * 16 * kR * kCols * sizeof(float);
+  unsigned* counters = nullptr;
+  float* partial = nullptr;
   std::optional<StreamScratch> scratch;
   if (shared_bytes > 0) {
+    void* p = nullptr;
     size_t have = 0;
-    const hipError_t e = workspace_if_possible(kSlotKan, std::max(shared_bytes, bytes), stream, &partial, &have);
+    const hipError_t e = workspace_if_possible(kSlotKan, std::max(shared_bytes, nsplit * per_split), stream, &p, &have);
     if (e != hipSuccess) return e;
-    nsplit = (int)std::min<size_t>(nsplit, have / (n * sizeof(float)));
+    nsplit = (int)std::min<size_t>(nsplit, std::max<size_t>(have / per_split, 1));
+    partial = static_cast<float*>(p);
   } else if (nsplit > 1) {
-    scratch.emplace(bytes, stream);
-    partial = scratch->ptr;
+    scratch.emplace(nsplit * per_split, stream);
+    counters = scratch->counters;
+    partial = static_cast<float*>(scratch->ptr);
   }
-  if (partial == nullptr || nsplit < 1) nsplit = 1;
+  if (partial == nullptr) nsplit = 1;
   const int cper = (nchunks + nsplit - 1) / nsplit;
   nsplit = (nchunks + cper - 1) / cper;
-  const int64_t pairs = (int64_t)ctiles * nsplit, span = std::min<int64_t>(8, pairs), pairs8 = (pairs + span - 1) / span * span;
-  hipLaunchKernelGGL((kan_direct::kan_direct<kNQ, kR>), dim3((unsigned)(pairs8 * mtiles)), dim3(kThreads), lds, stream,
-                     x, grid, wb, ws, sc, order, L, C, B, I, O, mtiles, ctiles, nsplit, cper,
-                     nsplit > 1 ? static_cast<float*>(partial) : out);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || nsplit == 1) return e;
-  const unsigned blocks = (unsigned)std::min<size_t>((n + kThreads - 1) / kThreads, 4096);
-  hipLaunchKernelGGL(kan_direct_sum, dim3(blocks), dim3(kThreads), 0, stream, static_cast<const float*>(partial),
-                     (int64_t)n, nsplit, out);
+  if (nsplit > kMaxArrivals || tiles > kScratchCounters) counters = nullptr;
+  const int64_t pairs = (int64_t)ctiles * nsplit, span = std::min<int64_t>(8, pairs), padded = (pairs + span - 1) / span * span;
+  hipLaunchKernelGGL((kan_direct::kan_direct<kNQ, kR>), dim3((unsigned)(padded * mtiles)), dim3(kThreads), lds, stream,
+                     x, grid, wb, ws, sc, order, L, C, B, I, O, mtiles, ctiles, nsplit, cper, partial,
+                     counters, out);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || nsplit == 1 || counters != nullptr) return e;
+  hipLaunchKernelGGL(kan_direct_sum<kR>, dim3((unsigned)(tiles * 4 * kR)), dim3(kThreads), 0, stream,
+                     static_cast<const float*>(partial), B, O, mtiles, ctiles, nsplit, out);
   return hipGetLastError();
 }
 
@@ -80,7 +91,8 @@ bool kan_direct_fits(int order, int C, int B, int I, int O) {
 
 // shared_bytes: 0 for calls with no workspace of their own (the splits' sums then go to the
 // stream's scratch memory, and stay unsplit where there is none); else the size to which the
-// shared workspace is grown, which holds them.
+// shared workspace is grown, which holds them.  The arrival counters are the scratch memory's
+// alone: two streams' calls at once could leave shared ones wrong for every later call.
 hipError_t kan_direct_launch(const float* x, const float* grid, const float* wb, const float* ws, const float* sc,
                              int order, int L, int C, int B, int I, int O, float* out, size_t shared_bytes,
                              hipStream_t stream) {

@@ -1,4 +1,4 @@
-// efficient_kan on fp32 matrix cores, weights read where they lie: kan_direct and kan_direct_sum.
+// efficient_kan on fp32 matrix cores, weights read where they lie: kan_direct.
 //
 // Op: tasks/efficient_kan/reference.py:33-51, any spline order 1 .. 4 and any knot row of up
 // to 32 knots, all arithmetic fp32.
@@ -15,8 +15,8 @@
 //    scheme on the interval's own knots, written into a zeroed run of C slots in LDS.  Chunk
 //    c + 1 is expanded while chunk c feeds the MFMAs (two LDS stages, one barrier per chunk).
 //  * The features are split over workgroups until the chip is full; each split writes its
-//    fp32 tile and kan_direct_sum adds the splits in order, so the result does not depend on
-//    timing.
+//    fp32 tile, and the last to arrive (where there are counters, and few splits) or
+//    kan_direct_sum adds the splits in order, so the result does not depend on timing.
 // Each step's terms are summed from zero and then added to the running sum, so a long sum
 // rounds like one of its partial sums: 1.1e-7 .. 1.8e-7 (2-norm, against fp64) where the
 // row-wise kernel had 2.3e-7 .. 3.7e-7 and the fp16x3 path 2.2e-7 .. 3.6e-7.
@@ -24,7 +24,7 @@
 // Bound: for batches up to about 32 rows by the weight stream and two launches' latency (B = 8,
 // I = O = 1024, G = 5: 42 MB in 15.6 us, 71.4 with the fp16x3 path), above by the fp32 MFMAs
 // and the expansion beside them (fp32 MFMAs and VALU instructions do not overlap): B = 1024,
-// I = 256, O = 512, G = 16 takes 71.6 us, 35 of them MFMA time, against 11,050 for the row-wise
+// I = 256, O = 512, G = 16 takes 66.3 us, 35 of them MFMA time, against 11,050 for the row-wise
 // kernel; there the loads and LDS reads cost 3 us and the expansion about 14.
 #pragma once
 
@@ -41,6 +41,8 @@ constexpr int kCols = 16 * kWaves;     // output columns per workgroup, 16 per w
 constexpr int kMaxKnots = 32;
 constexpr int kRawBufferFlags = 0x00020000;
 constexpr unsigned kOutOfRange = 0x80000000u;
+constexpr int kSystemScope = 17;  // buffer cache policy sc0 | sc1
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 // Features per chunk: 16 kR rows x these features are the (row, feature) pairs the threads
 // expand, one each (half the threads idle for kR = 1 with many bases, whose staged weights
@@ -146,12 +148,14 @@ __device__ __forceinline__ void write_bases(float x, const float* kn, int L, int
 // kNQ: 16-byte groups of a feature's C bases, 4 (kNQ - 1) < C <= 4 kNQ.  The last group is
 // read at C - 4, inside the feature's own floats, so its first 4 kNQ - C ("dup") elements
 // repeat the group before it: they have no slot and no MFMA.  kR: row blocks of 16.
-// out: [nsplit][B][O] partial sums, or the output itself for one split.
+// nsplit > 1: partial holds a tile of sums per (split, row tile, column tile), counters (or
+// null) one arrival counter per tile, zero between launches.
 template <int kNQ, int kR>
 __global__ __launch_bounds__(kThreads) void kan_direct(
     const float* __restrict__ x, const float* __restrict__ grid, const float* __restrict__ wb,
     const float* __restrict__ ws, const float* __restrict__ sc, int order, int L, int C, int B, int I, int O,
-    int mtiles, int ctiles, int nsplit, int cper, float* __restrict__ out) {
+    int mtiles, int ctiles, int nsplit, int cper, float* __restrict__ partial, unsigned* __restrict__ counters,
+    float* __restrict__ out) {
   constexpr int kFeat = chunk_features<kNQ, kR>();
   constexpr int kPairs = pairs<kNQ, kR>(), kAct = act_floats<kNQ, kR>();
   constexpr bool kFlat = flat_loads<kR>();
@@ -394,33 +398,95 @@ __global__ __launch_bounds__(kThreads) void kan_direct(
     for (int s = 0; s < kSteps; ++s) step(c, s);
   }
 
-  float* dst = out + (size_t)split * B * O;
+  if (nsplit > 1) {
+    // Every split stores its tile, 16 bytes per lane and row block.  Without counters
+    // kan_direct_sum adds them.  With counters it then arrives on the tile's, and the last adds
+    // the splits' tiles in split order, so the result does not depend on which one that is.
+    // The stores and the loads are system-scope (sc0 sc1): they go through
+    // to the coherence point, a store's completion (vmcnt) means it got there, and the arrival
+    // follows every wave's wait for that.  So no L2 needs writing back or invalidating: with
+    // agent-scope fences, one per workgroup, the write-backs queued up (B = 64, I = O = 1024
+    // 55 us; a second launch for the sums 27.0).
+    constexpr int kTile = kRows * kCols;
+    const int tile = mt * ctiles + ct;
+    // Split by split, so that what the sum reads together lies together.
+    const int stride = mtiles * ctiles * kTile * 4;
+    const __amdgpu_buffer_rsrc_t rp =
+        make_rsrc(partial + (size_t)tile * kTile, (size_t)(nsplit - 1) * stride + kTile * 4);
+    unsigned at[kR];  // missing rows' sums go nowhere: past the descriptor
+#pragma unroll
+    for (int r = 0; r < kR; ++r)
+      at[r] = m0 + 16 * r + 4 * fq < B ? (unsigned)(((wave * kR + r) * kWave + lane) * 16) : kOutOfRange;
+    if (counters == nullptr) {
+#pragma unroll
+      for (int r = 0; r < kR; ++r)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, acc[r]), rp, at[r], split * stride, 0);
+      return;
+    }
+#pragma unroll
+    for (int r = 0; r < kR; ++r)
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, acc[r]), rp, at[r], split * stride, kSystemScope);
+    __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8));  // vmcnt(0): the stores are done
+    __syncthreads();  // every wave's; the LDS is free
+    unsigned* flag = reinterpret_cast<unsigned*>(smem);
+    if (tid == 0) {
+      const bool last =
+          __hip_atomic_fetch_add(counters + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)nsplit - 1;
+      if (last) __hip_atomic_store(counters + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *flag = last;
+    }
+    __syncthreads();
+    if (!*flag) return;
+    constexpr int kBatch = 16 / kR;  // splits whose loads are in flight together
+#pragma unroll
+    for (int r = 0; r < kR; ++r) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < nsplit; s += kBatch) {
+      f32x4 v[kBatch][kR];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u)  // past the last split: past the descriptor, zero
+#pragma unroll
+        for (int r = 0; r < kR; ++r)
+          v[u][r] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, at[r], (s + u) * stride, kSystemScope));
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u)
+#pragma unroll
+        for (int r = 0; r < kR; ++r) acc[r] += v[u][r];
+    }
+  }
   if (col < O) {
 #pragma unroll
     for (int r = 0; r < kR; ++r)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int row = m0 + 16 * r + 4 * fq + e;
-        if (row < B) dst[(size_t)row * O + col] = acc[r][e];
+        if (row < B) out[(size_t)row * O + col] = acc[r][e];
       }
   }
 }
 
-// out[e] = the nsplit partial sums of element e, added in split order.
+// The sums without counters: thread per element of a tile, as kan_direct stored it, the
+// splits added in the same order.  4 * kR workgroups per tile.
 constexpr int kSumBatch = 16;
-__global__ __launch_bounds__(kThreads) void kan_direct_sum(const float* __restrict__ partial, int64_t n, int nsplit,
-                                                           float* __restrict__ out) {
-  for (int64_t e = (int64_t)blockIdx.x * kThreads + threadIdx.x; e < n; e += (int64_t)gridDim.x * kThreads) {
-    float t = 0.0f;
-    for (int s = 0; s < nsplit; s += kSumBatch) {  // a batch of loads in flight, added in order
-      float v[kSumBatch];
+template <int kR>
+__global__ __launch_bounds__(kThreads) void kan_direct_sum(const float* __restrict__ partial, int B, int O, int mtiles,
+                                                           int ctiles, int nsplit, float* __restrict__ out) {
+  constexpr int kTile = 16 * kR * kCols;
+  const int tile = (int)blockIdx.x / (4 * kR), at = (int)blockIdx.x % (4 * kR) * kThreads + (int)threadIdx.x;
+  const int lane = at / 4 % kWave, r = at / 4 / kWave % kR, wave = at / 4 / kWave / kR;
+  const int col = tile % ctiles * kCols + 16 * wave + lane % 16;
+  const int row = tile / ctiles * 16 * kR + 16 * r + 4 * (lane / 16) + at % 4;
+  if (col >= O || row >= B) return;
+  const size_t stride = (size_t)mtiles * ctiles * kTile;
+  const float* from = partial + (size_t)tile * kTile + at;
+  float t = 0.f;
+  for (int s = 0; s < nsplit; s += kSumBatch) {  // a batch of loads in flight, added in order
+    float v[kSumBatch];
 #pragma unroll
-      for (int u = 0; u < kSumBatch; ++u) v[u] = s + u < nsplit ? partial[(size_t)(s + u) * n + e] : 0.0f;
+    for (int u = 0; u < kSumBatch; ++u) v[u] = s + u < nsplit ? from[(s + u) * stride] : 0.f;
 #pragma unroll
-      for (int u = 0; u < kSumBatch; ++u) t += v[u];
-    }
-    out[e] = t;
+    for (int u = 0; u < kSumBatch; ++u) t += v[u];
   }
+  out[(size_t)row * O + col] = t;
 }
 
 }  // namespace kan_direct

@@ -131,12 +131,18 @@ StreamScratch::StreamScratch(size_t bytes, hipStream_t stream) {
   for (StreamRegion& s : g_scratch[dev])
     if (r == nullptr && s.ptr == nullptr) r = &s;
   if (r == nullptr) return;
-  if (r->bytes < bytes) {
+  constexpr size_t kHead = kScratchCounters * sizeof(unsigned);
+  if (r->bytes < kHead + bytes) {
     size_t want = r->bytes > 0 ? 2 * r->bytes : (size_t)1 << 18;
-    while (want < bytes) want *= 2;
+    while (want < kHead + bytes) want *= 2;
     void* p = nullptr;
     if (hipMalloc(&p, want) != hipSuccess) {
       (void)hipGetLastError();
+      return;
+    }
+    hipLaunchKernelGGL(zero_fill, dim3(1), dim3(256), 0, stream, static_cast<uint4*>(p), kHead / 16);
+    if (hipGetLastError() != hipSuccess) {
+      (void)hipFree(p);
       return;
     }
     if (r->ptr != nullptr) {
@@ -145,7 +151,8 @@ StreamScratch::StreamScratch(size_t bytes, hipStream_t stream) {
     }
     *r = StreamRegion{stream, p, want};
   }
-  ptr = r->ptr;
+  counters = static_cast<unsigned*>(r->ptr);
+  ptr = static_cast<char*>(r->ptr) + kHead;
 }
 
 int device_cu_count() {
