@@ -443,10 +443,15 @@ __global__ __launch_bounds__(kThreads) void kan_direct(
     for (int s = 0; s < nsplit; s += kBatch) {
       f32x4 v[kBatch][kR];
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u)  // past the last split: past the descriptor, zero
+      for (int u = 0; u < kBatch; ++u) {
+        // Past the last split: the vector offset, the one the descriptor's bound is checked
+        // against, lies past the buffer and the load returns zero.
+        const bool live = s + u < nsplit;
 #pragma unroll
         for (int r = 0; r < kR; ++r)
-          v[u][r] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, at[r], (s + u) * stride, kSystemScope));
+          v[u][r] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                  rp, live ? at[r] : kOutOfRange, live ? (s + u) * stride : 0, kSystemScope));
+      }
 #pragma unroll
       for (int u = 0; u < kBatch; ++u)
 #pragma unroll

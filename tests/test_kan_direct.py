@@ -109,3 +109,18 @@ def test_direct_first_call_in_a_capture(lib):
     print("\n[kan_direct] first call under capture", flush=True)
     r = subprocess.run([sys.executable, "-c", CAPTURE.format(root=str(ROOT))], capture_output=True, text=True, timeout=110)
     assert r.returncode == 0 and "captured" in r.stdout, (r.stdout[-500:], r.stderr[-2000:])
+
+
+def test_direct_few_splits_after_many(lib):
+    """A call split in 2 (or 3) after one split in 16 on the same stream: the sum reads no more
+    than its own splits, whatever the earlier call left behind them in the stream's scratch."""
+    print("\n[kan_direct] few splits after many", flush=True)
+    many = inputs.make_inputs("efficient_kan", dict(name="d", seed=77, B=512, I=80, O=512, grid_size=12, spline_order=3))
+    many["base_weight"] = many["base_weight"] * 100.0
+    for B, I in [(70, 5), (70, 9), (20, 17), (3, 17)]:
+        few = inputs.make_inputs("efficient_kan", dict(name="d", seed=78, B=B, I=I, O=30, grid_size=12, spline_order=3))
+        want = exact.efficient_kan(few)["out"]
+        capi.run_op(lib, "efficient_kan", many)
+        got = capi.run_op(lib, "efficient_kan", few)["out"].cpu().numpy()
+        t = tally(got, want, tasks.load_task("efficient_kan")["tolerance"])
+        assert t["mismatched"] == 0, (B, I, t)
