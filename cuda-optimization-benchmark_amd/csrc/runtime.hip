@@ -57,6 +57,17 @@ hipError_t stream_device(hipStream_t stream, int* dev) {
   return hipSuccess;
 }
 
+// While this lives, the calling thread's HIP calls do not count against a capture that another
+// stream is making: in the default, global capture mode an allocation on any thread is refused
+// and that capture invalidated.  For allocations whose own stream is not capturing.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool on = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  ~RelaxedCapture() {
+    if (on) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+};
+
 // Makes region r at least `bytes` large (g_mu held).
 hipError_t grow(Region& r, size_t bytes, hipStream_t stream) {
   const size_t want = ((bytes < 4096 ? 4096 : bytes) + 15) / 16 * 16;
@@ -106,6 +117,7 @@ hipError_t workspace_if_possible(WorkspaceSlot slot, size_t bytes, hipStream_t s
     e = hipStreamIsCapturing(stream, &status);
     if (e != hipSuccess) (void)hipGetLastError();
     if (e == hipSuccess && status == hipStreamCaptureStatusNone) {
+      const RelaxedCapture relaxed;
       e = grow(r, bytes, stream);
       if (e != hipSuccess) return e;
     }
@@ -136,6 +148,7 @@ StreamScratch::StreamScratch(size_t bytes, hipStream_t stream) {
     size_t want = r->bytes > 0 ? 2 * r->bytes : (size_t)1 << 18;
     while (want < kHead + bytes) want *= 2;
     void* p = nullptr;
+    const RelaxedCapture relaxed;
     if (hipMalloc(&p, want) != hipSuccess) {
       (void)hipGetLastError();
       return;

@@ -87,3 +87,34 @@ def test_graph_of_several_ops(lib):
         for op, (_, outs) in bound.items():
             for n, t in outs.items():
                 assert torch.equal(t, want[op][n]), (op, n)
+
+
+@pytest.mark.parametrize("op,case", [
+    ("reward_to_go", dict(name="g", seed=7, B=4, T=40_000, gamma=0.99, done_p=0.01)),
+    ("efficient_kan", dict(name="g", seed=8, B=200, I=96, O=128, grid_size=12)),
+])
+def test_eager_first_call_beside_a_capture(lib, op, case):
+    """An eager call on a new stream, which allocates that stream's scratch memory, leaves a
+    capture that another stream is making whole: the graph replays, and the call's result is
+    the one a call outside any capture gives."""
+    print(f"\n[graph] {op} beside a capture", flush=True)
+    args, outs = _bind(op, inputs.make_inputs(op, case))
+    small, small_outs = _bind("leaky", inputs.make_inputs("leaky", SMALL["leaky"]))
+    torch.cuda.synchronize()
+    beside = torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        capi.call(lib, "leaky", small)
+        capi.call(lib, op, args, beside.cuda_stream)
+    torch.cuda.synchronize()
+    got = {n: t.clone() for n, t in outs.items()}
+    for t in small_outs.values():
+        t.fill_(9.0)
+    for _ in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        assert not bool((small_outs["spikes"] == 9.0).any())
+    capi.call(lib, op, args)
+    torch.cuda.synchronize()
+    for n, t in outs.items():
+        assert torch.equal(t, got[n]), n
