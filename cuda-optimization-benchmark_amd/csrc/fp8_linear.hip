@@ -33,19 +33,41 @@ bool offsets_fit(int64_t M, int64_t K, int64_t N) {
 // and from there on the wide kernel's forms.  Where they do not apply (K % 16, alignment),
 // 128x128 tiles take the rest.
 //
-// M <= 64: the skinny kernel's time is its weight stream at a rate that falls with the row
-// blocks, a 64x64 tile's is its steps, so wide N favours the tiles: at K = N = 8192 M = 16 17.0
-// against 13.5 us, M = 32 23.5 / 14.4, M = 64 30.1 / 15.7; at 4096 6.2 / 8.5, 7.9 / 8.5, 9.4 /
-// 9.1; from 33 rows on the tiles were never slower.  With 8-byte rows both move less per load: M
-// = 64, K = N = 8184 45.5 / 26.4 but M = 16 and 4088 7.2 / 12.6, M = 64 14.0 / 14.6.  Other K
-// have no 8-byte loads for the skinny kernel: M = 16, K = 2047, N = 8000 41.2 / 10.4, M = 1, K =
-// 333, N = 300 5.2 / 4.6.
+// M <= 64: the skinny kernel gives 16 columns to a workgroup and splits K over its waves; a tile
+// has four times the columns and walks K alone.  With more than one skinny workgroup per CU the
+// skinny kernel's time doubles and the tiles win; below that it depends on K.  us, skinny / tiles,
+// weights in the Infinity Cache and (in brackets) from memory:
+//  * 17 rows up, more than 16 columns per CU: M = 32, K = 4096, N = 5120 12.8 / 8.3 (13.2 / 11.9),
+//    M = 64 16.0 / 8.6 (16.6 / 12.9).  Up to 16 rows from N = 7168 on: M = 16, K = 1024, N = 8192 7.6 /
+//    4.1 (7.8 / 5.6), K = 4096 10.1 / 8.3 (10.3 / 11.3), K = 7168 15.9 / 11.8 (16.0 / 17.6), but K =
+//    14336 28.2 / 30.5 (28.3 / 30.5): half the CUs hold a tile and do not draw the memory's rate.
+//  * 33 to 48 rows at fewer columns: the skinny kernel's waves take 2048 of K a pass, so just beyond
+//    one pass the tiles win: M = 43, K = 2176, N = 1632 6.4 / 5.3 (10.1 / 6.3), M = 33, K = 3072, N = 1024
+//    7.7 / 6.2 (9.3 / 7.3), K = 4096 7.6 / 7.2 (9.8 / 8.6); at K = 2048 5.1 / 5.1 (5.4 / 6.0), 4.3 / 5.1
+//    with the weights in the L2s, and at N = 64, K = 4096 5.7 / 7.0.  Longer K from memory is too much for
+//    the few CUs that hold a tile: M = 39, K = 5536, N = 1568 (14.3 / 18.1), M = 48, K = 10352, N =
+//    1216 (26.6 / 36.6), although from the Infinity Cache the tiles would be faster.
+//  * 49 rows up at fewer columns: M = 64, K = 1024, N = 512 3.5 / 4.1, K = 2048, N = 4096 5.5 / 5.2 (6.0 /
+//    8.0), K = 7168, N = 1024 13.4 / 11.9 (13.7 / 19.3): the skinny kernel.
+//  * 33 rows up at less than two columns per CU, where the skinny kernel has few workgroups as well,
+//    and K past 4096: M = 54, K = 8000, N = 176 14.9 / 11.3, M = 64, K = 7168, N = 64 12.1 / 10.1.
+// With 8-byte rows both move less per load: M = 33, K = 4088, N = 4104 16.6 / 13.8 (18.1 / 18.5), K =
+// 1016 4.8 / 5.6 (4.9 / 5.8), N = 8200 6.1 / 5.7 (7.2 / 7.2); M = 64, K = 1016, N = 4104 6.2 / 5.6 (6.2 /
+// 6.0).  Other K have no 8-byte loads for the skinny kernel: M = 16, K = 1001, N = 1024 12.3 / 6.1.
 int mid_tile(int64_t M, int64_t K, int64_t N, int vec) {
   const int64_t cus = device_cu_count();
   if (M <= kSkinnyMaxM) {
     if (vec == 16 && 64 * K > (int64_t)0x7fffffff) return -1;  // a tile's rows in 32-bit offsets
     const int rb = (int)(M + 15) / 16;
-    const bool tiles = vec == 1 || (vec == 16 ? (rb >= 3 || N >= (rb == 2 ? 5120 : 7168)) : (rb >= 3 && N > 4096));
+    const bool wide = N > 16 * cus;  // more than one skinny workgroup per CU
+    bool tiles = vec == 1;
+    if (vec == 16) {
+      if (rb == 1) tiles = N >= 28 * cus && (K <= 8192 || N > 32 * cus);
+      else if (rb == 2) tiles = N >= 20 * cus;
+      else tiles = wide || (K > 4096 ? N < 2 * cus : rb == 3 && K > 2048 && N >= 2 * cus);
+    } else if (vec == 8) {
+      tiles = wide && (rb == 4 || (rb == 3 && (K > 2048 || N >= 32 * cus)));
+    }
     return tiles ? kTile64x64 : -1;
   }
   auto tiles = [&](int rows, int cols) { return ((M + rows - 1) / rows) * ((N + cols - 1) / cols); };

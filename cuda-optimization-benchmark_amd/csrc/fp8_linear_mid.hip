@@ -29,12 +29,18 @@ hipError_t launch_any(bool direct, const uint8_t* x, const uint8_t* w, int M, in
 }  // namespace
 
 // Ring depths: 64 x 64 tiles in four steps (two workgroups fit a CU), the larger ones as many
-// as one CU's LDS holds; 8 steps for 64 x 64 measured the same with one workgroup per CU and
-// slower with two (M = 512, K = N = 4096 16.8 against 14.7 us).
+// as one CU's LDS holds; 8 steps for 64 x 64 measured slower with two workgroups per CU (M = 512,
+// K = N = 4096 16.8 against 14.7 us).  Up to 32 rows with one workgroup per CU and a long K, where
+// the weights are the stream, 8 steps keep twice the bytes in flight: from memory M = 16, K = 4096,
+// N = 8192 12.6 -> 11.3 us, K = 7168 19.1 -> 17.6, the same from the Infinity Cache; K = 1024 4.1 ->
+// 4.7 there, and the same at 64 rows, so shorter K and more rows keep four.
 hipError_t mid_launch(MidTile tile, bool direct, const uint8_t* x, const uint8_t* w, int M, int N, int K, float inv,
                       const uint16_t* bias, uint16_t* out, hipStream_t stream) {
   switch (tile) {
-    case kTile64x64: return launch_any<1, 1, 4>(direct, x, w, M, N, K, inv, bias, out, stream);
+    case kTile64x64:
+      if (direct && M <= 32 && K >= 4096 && (N + 63) / 64 <= device_cu_count())
+        return launch<1, 1, 8, true>(x, w, M, N, K, inv, bias, out, stream);
+      return launch_any<1, 1, 4>(direct, x, w, M, N, K, inv, bias, out, stream);
     case kTile64x128: return launch_any<1, 2, 6>(direct, x, w, M, N, K, inv, bias, out, stream);
     default: return launch_any<2, 2, 4>(direct, x, w, M, N, K, inv, bias, out, stream);
   }

@@ -16,6 +16,10 @@ SHAPES = [
     # 64x64 tiles, direct copies: one tile and ragged ones, one step to more than the ring holds
     (65, 16, 64, 0, 0), (64, 128, 65, 0, 0), (128, 144, 63, 0, 0), (100, 512, 200, 0, 0), (127, 1040, 130, 0, 4),
     (33, 640, 72, 0, 1), (48, 656, 1, 0, 0), (16, 256, 8192, 0, 0), (32, 272, 5121, 0, 0),
+    # at most 64 rows: few columns and K past 2048, more than 16 columns per CU, and the ring of 8
+    # steps (up to 32 rows, K from 4096 on) with ragged tails
+    (33, 2064, 520, 0, 0), (48, 3088, 1000, 0, 1), (40, 4096, 515, 0, 0), (64, 4112, 70, 0, 0), (40, 144, 4100, 0, 0), (64, 528, 4225, 0, 0),
+    (16, 4096, 7168, 0, 0), (1, 4112, 7201, 0, 0), (17, 4224, 5125, 0, 0), (32, 4240, 5120, 0, 4),
     # 64x128 and 128x128 tiles, direct copies
     (513, 400, 4000, 0, 0), (400, 768, 4100, 0, 0), (1000, 912, 4100, 0, 0), (777, 1024, 4001, 0, 3),
     # 16-byte loads at any alignment: K below 16, on both sides of a load and of a step

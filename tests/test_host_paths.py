@@ -72,3 +72,30 @@ def test_allocating_leaves_another_streams_capture_alone(host, op, args):
 def test_a_capturing_stream_allocates_nothing(host, op, args):
     out = host([put("capturing", 4, 1), put("global_capture", 1), call(op, stream=4, **args)])[-1]
     assert out["rc"] == 0 and not any(line.startswith(("malloc", "capture_broken")) for line in out["log"]), out["log"]
+
+
+def fp8_kernel(host, *sizes, x=0):
+    steps = [call("fp8_linear", M=M, K=K, N=N, scale_x=1.0, scale_w=1.0, x_fp8=(1 << 40) + x) for M, K, N in sizes]
+    out = host(steps)
+    assert all(s["rc"] == 0 for s in out)
+    names = [kernels(s) for s in out]
+    assert all(len(n) == 1 for n in names)
+    return [n[0] for n in names]
+
+
+# Sides of fp8_linear's rule for at most 64 rows: the skinny kernel where its workgroups fit the
+# CUs once (it was up to 25% faster there than the tiles), the tiles beyond.
+FP8_SKINNY = [(33, 2048, 64), (33, 4096, 64), (40, 1024, 4096), (48, 2048, 2048), (64, 1024, 512), (64, 2048, 1024),
+              (64, 4096, 4096), (64, 8192, 512), (64, 7168, 4096), (56, 704, 1600), (63, 3136, 576), (16, 16384, 4096),
+              (32, 8192, 4096), (16, 16384, 8192), (8, 4096, 6144), (48, 8192, 520), (33, 4096, 448), (39, 5536, 1568),
+              (16, 4088, 8200), (33, 1016, 4104), (33, 2040, 8000), (48, 4088, 4096), (64, 4088, 1024)]
+FP8_TILES = [(33, 4096, 1024), (48, 2064, 512), (48, 8192, 64), (64, 7168, 504), (33, 256, 4112), (64, 256, 4112), (64, 8192, 5120), (17, 256, 5120),
+             (32, 16384, 5120), (1, 256, 7168), (16, 8192, 8192), (16, 16384, 16384), (33, 4088, 4104), (48, 1016, 8200),
+             (64, 1016, 4104), (1, 333, 300), (64, 4095, 64), (16, 63, 4096)]
+
+
+def test_fp8_small_m_routes(host):
+    for size, name in zip(FP8_SKINNY, fp8_kernel(host, *FP8_SKINNY)):
+        assert "fp8_gemm_skinny" in name, (size, name)
+    for size, name in zip(FP8_TILES, fp8_kernel(host, *FP8_TILES)):
+        assert "fp8_gemm_mid" in name, (size, name)
