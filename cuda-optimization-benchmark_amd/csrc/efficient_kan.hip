@@ -10,7 +10,6 @@
 //    packing (direct_is_faster);
 //  * row-wise fp32, below, for the rest (order 0 or above 4, fewer than four bases).
 #include <algorithm>
-#include <cmath>
 
 #include "efficient_kan.hpp"
 
@@ -18,6 +17,7 @@ namespace taskops {
 
 // efficient_kan_direct.hip
 bool kan_direct_fits(int order, int C, int B, int I, int O);
+double kan_direct_us(int C, int B, int I, int O);
 hipError_t kan_direct_launch(const float* x, const float* grid, const float* wb, const float* ws, const float* sc,
                              int order, int L, int C, int B, int I, int O, float* out, size_t shared_bytes,
                              hipStream_t stream);
@@ -120,16 +120,26 @@ FastPlan fast_plan(int Cp, int B, int I, int O, int L) {
   return p;
 }
 
-// The direct path costs what its fp32 MFMAs do, about 25 us per 1e9 terms (B I O (1 + C)); the
-// fast path has 16 times their rate, but packs the weights first and, where its 128 x 256
-// tiles leave CUs idle, splits and sums the features: the more splits, the later it wins.
-// Where both took the same time (one box, terms against the fast path's splits): 2 splits 3e8
-// .. 8e8 terms, 4 7e8 .. 9e8, 8 1.0e9 .. 1.6e9, 16 1.5e9, 32 2.5e9, near 2.5e8 splits^(2/3).
-// Either side of the line (us, direct against fast): I = O = 1024, G = 5, B = 8 15.6 / 71, B =
-// 128 41 / 72, B = 512 131 / 68; I = 256, O = 512, G = 8, B = 256 25 / 47, B = 4096 159 / 70.
-bool direct_is_faster(const FastPlan& plan, int B, int I, int O, int C) {
-  const double terms = (double)B * I * O * (1 + C), n = plan.nsplit;
-  return terms <= 2.5e8 * std::cbrt(n * n);
+// About how long the fast path takes, in us: two launches, the packing (by its padded weights),
+// the feature groups each CU walks, and with split-K the partial tiles, each written, arrived on
+// and read again.  Within 10% of 239 measured calls in 90% of them.
+double fast_us(const FastPlan& plan, int Cp) {
+  const int cus = device_cu_count(), rounds = (plan.tiles * plan.nsplit + cus - 1) / cus;
+  const double packed = 1e-6 * plan.Opad * plan.ngroups * kan::kGroup * (1 + Cp);
+  double us = 6.9 + (Cp == 16 ? 2.3 : 0.0) + 1.34 * packed + rounds * (6.9 + 0.774 * plan.gper * (1 + Cp));
+  if (plan.nsplit > 1) us += 1.1 * plan.nsplit + 17.0 * plan.tiles * plan.nsplit / cus;
+  return us;
+}
+
+// The direct path reads the weights where they lie but runs every term on fp32 MFMAs; the fast
+// path has 16 times their rate, but packs the weights first and pads to 128 x 256 tiles.  The
+// direct path has to be estimated 8% faster: then on 322 calls around the line none was more
+// than 11% slower than the fast path, and none lost more than 11% by being turned away (a line by
+// B I O (1 + C) and the splits alone had calls 34% slower: B = 1710, I = 1000, O = 100, G = 5 59.0 us
+// fast, 78.9 direct).  Either side of it (us, direct against fast): I = O = 1024, G = 5, B = 8 15.6 /
+// 71, B = 128 41 / 72, B = 512 131 / 68; I = 256, O = 512, G = 8, B = 256 25 / 47, B = 4096 159 / 70.
+bool direct_is_faster(const FastPlan& plan, int Cp, int B, int I, int O, int C) {
+  return 1.08 * kan_direct_us(C, B, I, O) < fast_us(plan, Cp);
 }
 
 template <int kCp>
@@ -195,7 +205,7 @@ extern "C" hipError_t taskops_efficient_kan(const float* x, const float* grid,
     bool direct = !fast;
     if (fast) {
       const FastPlan plan = fast_plan(Cp, B, I, O, L);
-      direct = direct_is_faster(plan, B, I, O, C);
+      direct = direct_is_faster(plan, Cp, B, I, O, C);
       // The workspace still grows to what the fast path asks for at this shape, so that a
       // capture of another shape after this call finds as much room as the fast path leaves.
       keep = plan.bytes;

@@ -20,20 +20,41 @@ int row_blocks(int B) { return B <= 16 ? 1 : (B <= 32 ? 2 : 4); }
 // G = 20) 11.1 / 10.4, 42 (B = 20, I = 333, O = 131, G = 10) 12.1 / 11.5.
 constexpr int kMaxArrivals = 16;
 
+// A call's launch: workgroups the chip holds at once, at most four per CU: the features are
+// split until the grid has that many, in one round.  At 1, 2 and 4 per CU B = 8, I = O = 1024 took
+// 19.7, 17.5 and 17.5 us (its LDS allows two); B = 4096, I = 256, O = 512 took 200 us at 3 and 178 at
+// 4.  nsplit splits of at most cper chunks each, none empty.
+struct Plan {
+  size_t lds;
+  int mtiles, ctiles, nchunks, per_cu, nsplit, cper, features;
+  void split(int n) {
+    cper = (nchunks + n - 1) / n;
+    nsplit = (nchunks + cper - 1) / cper;
+  }
+};
+
+template <int kNQ, int kR>
+Plan make_plan(int C, int B, int I, int O) {
+  Plan p;
+  p.features = chunk_features<kNQ, kR>();
+  p.mtiles = (B + 16 * kR - 1) / (16 * kR);
+  p.ctiles = (O + kCols - 1) / kCols;
+  p.nchunks = (I + p.features - 1) / p.features;
+  p.lds = (size_t)lds_bytes<kNQ, kR>(C);
+  p.per_cu = std::max(1, std::min<int>(4, (int)(device_lds_per_cu() / p.lds)));
+  const int64_t want = (int64_t)p.per_cu * device_cu_count() / ((int64_t)p.mtiles * p.ctiles);
+  p.split((int)std::min<int64_t>(p.nchunks, std::max<int64_t>(want, 1)));
+  return p;
+}
+
 template <int kNQ, int kR>
 hipError_t launch(const float* x, const float* grid, const float* wb, const float* ws, const float* sc, int order,
                   int L, int C, int B, int I, int O, float* out, size_t shared_bytes, hipStream_t stream) {
-  const int mtiles = (B + 16 * kR - 1) / (16 * kR), ctiles = (O + kCols - 1) / kCols;
-  const int nchunks = (I + chunk_features<kNQ, kR>() - 1) / chunk_features<kNQ, kR>();
-  const size_t lds = (size_t)lds_bytes<kNQ, kR>(C);
-  // Workgroups the chip holds at once, at most four per CU: the features are split until the
-  // grid has that many, in one round.  At 1, 2 and 4 per CU B = 8, I = O = 1024 took 19.7,
-  // 17.5 and 17.5 us (its LDS allows two); B = 4096, I = 256, O = 512 took 200 us at 3 and
-  // 178 at 4.
-  const int per_cu = std::max(1, std::min<int>(4, (int)(device_lds_per_cu() / lds)));
-  const int64_t tiles = (int64_t)mtiles * ctiles, want = (int64_t)per_cu * device_cu_count() / tiles;
-  int nsplit = (int)std::min<int64_t>(nchunks, std::max<int64_t>(want, 1));
+  Plan plan = make_plan<kNQ, kR>(C, B, I, O);
+  const int mtiles = plan.mtiles, ctiles = plan.ctiles;
+  const int64_t tiles = (int64_t)mtiles * ctiles;
   const size_t per_split = (size_t)tiles * 16 * kR * kCols * sizeof(float);
+  int nsplit = plan.nsplit;
   unsigned* counters = nullptr;
   float* partial = nullptr;
   std::optional<StreamScratch> scratch;
@@ -50,12 +71,12 @@ hipError_t launch(const float* x, const float* grid, const float* wb, const floa
     partial = static_cast<float*>(scratch->ptr);
   }
   if (partial == nullptr) nsplit = 1;
-  const int cper = (nchunks + nsplit - 1) / nsplit;
-  nsplit = (nchunks + cper - 1) / cper;
+  plan.split(nsplit);
+  nsplit = plan.nsplit;
   if (nsplit > kMaxArrivals || tiles > kScratchCounters) counters = nullptr;
   const int64_t pairs = (int64_t)ctiles * nsplit, span = std::min<int64_t>(8, pairs), padded = (pairs + span - 1) / span * span;
-  hipLaunchKernelGGL((kan_direct::kan_direct<kNQ, kR>), dim3((unsigned)(padded * mtiles)), dim3(kThreads), lds, stream,
-                     x, grid, wb, ws, sc, order, L, C, B, I, O, mtiles, ctiles, nsplit, cper, partial,
+  hipLaunchKernelGGL((kan_direct::kan_direct<kNQ, kR>), dim3((unsigned)(padded * mtiles)), dim3(kThreads), plan.lds, stream,
+                     x, grid, wb, ws, sc, order, L, C, B, I, O, mtiles, ctiles, nsplit, plan.cper, partial,
                      counters, out);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || nsplit == 1 || counters != nullptr) return e;
@@ -87,6 +108,28 @@ bool kan_direct_fits(int order, int C, int B, int I, int O) {
   const int rows = 16 * row_blocks(B);
   const int64_t tiles = (((int64_t)O + kCols - 1) / kCols + 7) / 8 * 8 * (((int64_t)B + rows - 1) / rows);
   return tiles <= (int64_t)0xffffffff / kThreads;
+}
+
+namespace {
+template <int kNQ>
+Plan plan_rows(int C, int B, int I, int O) {
+  switch (row_blocks(B)) {
+    case 1: return make_plan<kNQ, 1>(C, B, I, O);
+    case 2: return make_plan<kNQ, 2>(C, B, I, O);
+    default: return make_plan<kNQ, 4>(C, B, I, O);
+  }
+}
+}  // namespace
+
+// About how long a call takes, in us, for the choice between the two paths (C at most 12 there):
+// each CU's share of (16-row block, feature) pairs, with the padding of the tiles, the splits and
+// the last round, at 25 ns for the expansion and 3.7 ns a term.  Within 15% of 239 measured calls
+// of 15 to 100 us in 90% of them.
+double kan_direct_us(int C, int B, int I, int O) {
+  const Plan p = C <= 4 ? plan_rows<1>(C, B, I, O) : (C <= 8 ? plan_rows<2>(C, B, I, O) : plan_rows<3>(C, B, I, O));
+  const int64_t groups = (int64_t)p.mtiles * p.ctiles * p.nsplit, round = (int64_t)p.per_cu * device_cu_count();
+  const double pairs = (double)((groups + round - 1) / round) * p.per_cu * p.cper * p.features * row_blocks(B);
+  return 14.0 + pairs * (0.025 + 0.0037 * (1 + C));
 }
 
 // shared_bytes: 0 for calls with no workspace of their own (the splits' sums then go to the

@@ -99,3 +99,26 @@ def test_fp8_small_m_routes(host):
         assert "fp8_gemm_skinny" in name, (size, name)
     for size, name in zip(FP8_TILES, fp8_kernel(host, *FP8_TILES)):
         assert "fp8_gemm_mid" in name, (size, name)
+
+
+def kan_kernel(host, *shapes, order=3):
+    """"direct", "fast" (kan_fused) or "rowwise" for (B, I, O, G[, order]) on a fresh library."""
+    steps = [call("efficient_kan", B=s[0], I=s[1], O=s[2], grid_size=s[3], spline_order=s[4] if len(s) > 4 else order)
+             for s in shapes]
+    out = host(steps)
+    assert all(s["rc"] == 0 for s in out)
+    known = {"kan_directI": "direct", "kan_fused": "fast", "kan_rowwise": "rowwise"}
+    return [next(v for k, v in known.items() if any(k in n for n in kernels(s))) for s in out]
+
+
+# Both sides of efficient_kan's choice between the direct and the fast path, at shapes where one
+# of them was measured at least 10% faster.
+KAN_DIRECT = [(8, 1024, 1024, 5), (128, 1024, 1024, 5), (256, 256, 512, 8), (6889, 128, 64, 5), (4096, 512, 64, 3),
+              (341, 65, 1606, 5), (1024, 1024, 1024, 16), (16, 8, 8, 5), (1852, 64, 512, 8, 2)]
+KAN_FAST = [(1710, 1000, 100, 5), (1499, 1000, 100, 5), (6561, 32, 128, 5), (2823, 32, 320, 3), (2114, 256, 256, 3),
+            (716, 1856, 192, 5), (512, 1024, 1024, 5), (4096, 256, 512, 8), (8192, 1024, 1024, 5)]
+
+
+def test_kan_routes(host):
+    assert kan_kernel(host, *KAN_DIRECT) == ["direct"] * len(KAN_DIRECT)
+    assert kan_kernel(host, *KAN_FAST) == ["fast"] * len(KAN_FAST)
