@@ -133,13 +133,13 @@ double fast_us(const FastPlan& plan, int Cp) {
 
 // The direct path reads the weights where they lie but runs every term on fp32 MFMAs; the fast
 // path has 16 times their rate, but packs the weights first and pads to 128 x 256 tiles.  The
-// direct path has to be estimated 8% faster: then on 322 calls around the line none was more
-// than 11% slower than the fast path, and none lost more than 11% by being turned away (a line by
-// B I O (1 + C) and the splits alone had calls 34% slower: B = 1710, I = 1000, O = 100, G = 5 59.0 us
-// fast, 78.9 direct).  Either side of it (us, direct against fast): I = O = 1024, G = 5, B = 8 15.6 /
-// 71, B = 128 41 / 72, B = 512 131 / 68; I = 256, O = 512, G = 8, B = 256 25 / 47, B = 4096 159 / 70.
+// direct path has to be estimated 4% faster: then of 400 calls around the line none was more
+// than 13% slower than the fast path, 5 more than 5%, and 6 lost more than 5% by being turned away
+// (a line by B I O (1 + C) and the splits alone had calls 34% slower: B = 1710, I = 1000, O = 100, G = 5
+// 59.0 us fast, 78.9 direct).  Either side of it (us, direct against fast): I = O = 1024, G = 5, B = 8
+// 15.6 / 71, B = 128 41 / 72, B = 512 131 / 68; I = 256, O = 512, G = 8, B = 256 25 / 47, B = 4096 159 / 70.
 bool direct_is_faster(const FastPlan& plan, int Cp, int B, int I, int O, int C) {
-  return 1.08 * kan_direct_us(C, B, I, O) < fast_us(plan, Cp);
+  return 1.04 * kan_direct_us(C, B, I, O) < fast_us(plan, Cp);
 }
 
 template <int kCp>

@@ -122,14 +122,12 @@ Plan plan_rows(int C, int B, int I, int O) {
 }  // namespace
 
 // About how long a call takes, in us, for the choice between the two paths (C at most 12 there):
-// each CU's share of (16-row block, feature) pairs, with the padding of the tiles, the splits and
-// the last round, at 25 ns for the expansion and 3.7 ns a term.  Within 15% of 239 measured calls
-// of 15 to 100 us in 90% of them.
+// each CU's share of (16-row block, feature) pairs, padding of the tiles and splits included, at
+// 27 ns for the expansion and 4 ns a term.  Within 10% of 80% of 370 measured calls of 15 to 100 us.
 double kan_direct_us(int C, int B, int I, int O) {
   const Plan p = C <= 4 ? plan_rows<1>(C, B, I, O) : (C <= 8 ? plan_rows<2>(C, B, I, O) : plan_rows<3>(C, B, I, O));
-  const int64_t groups = (int64_t)p.mtiles * p.ctiles * p.nsplit, round = (int64_t)p.per_cu * device_cu_count();
-  const double pairs = (double)((groups + round - 1) / round) * p.per_cu * p.cper * p.features * row_blocks(B);
-  return 14.0 + pairs * (0.025 + 0.0037 * (1 + C));
+  const double pairs = (double)p.mtiles * p.ctiles * p.nsplit * p.cper * p.features * row_blocks(B) / device_cu_count();
+  return 14.3 + pairs * (0.027 + 0.004 * (1 + C));
 }
 
 // shared_bytes: 0 for calls with no workspace of their own (the splits' sums then go to the
