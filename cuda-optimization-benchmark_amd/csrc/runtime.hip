@@ -18,11 +18,13 @@ struct StreamRegion {
   hipStream_t stream = nullptr;
   void* ptr = nullptr;
   size_t bytes = 0;
+  uint64_t used = 0;  // g_scratch_uses at the last use
 };
 
 std::mutex g_mu;
 std::mutex g_scratch_mu;
 StreamRegion g_scratch[kMaxDevices][kMaxScratchStreams];
+uint64_t g_scratch_uses = 0;
 Region g_regions[kMaxDevices][kNumSlots];
 // Buffers replaced by a larger one stay allocated until exit: a kernel enqueued before
 // the replacement may still be using them, and freeing would need a host sync.
@@ -127,9 +129,40 @@ hipError_t workspace_if_possible(WorkspaceSlot slot, size_t bytes, hipStream_t s
   return hipSuccess;
 }
 
+namespace {
+
+// Whether a region's stream has completed everything enqueued on it, or no longer exists.  A
+// capturing stream is not asked, which would end its capture.
+bool at_rest(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  hipError_t e = hipStreamIsCapturing(stream, &status);
+  if (e == hipSuccess && status == hipStreamCaptureStatusNone) e = hipStreamQuery(stream);
+  else if (e == hipSuccess) e = hipErrorNotReady;
+  if (e == hipSuccess) return true;
+  (void)hipGetLastError();
+  return e == hipErrorContextIsDestroyed || e == hipErrorInvalidHandle;
+}
+
+// The region of `stream`: its own, an unused one, or one whose stream is at rest; null when every
+// other stream with a region has work in flight (g_scratch_mu held).
+StreamRegion* region_for(hipStream_t stream, int dev) {
+  for (StreamRegion& s : g_scratch[dev])
+    if (s.ptr != nullptr && s.stream == stream) return &s;
+  for (StreamRegion& s : g_scratch[dev])
+    if (s.ptr == nullptr) return &s;
+  StreamRegion* r = nullptr;
+  const RelaxedCapture relaxed;
+  for (StreamRegion& s : g_scratch[dev])
+    if ((r == nullptr || s.used < r->used) && at_rest(s.stream)) r = &s;
+  return r;
+}
+
+}  // namespace
+
 StreamScratch::StreamScratch(size_t bytes, hipStream_t stream) {
+  constexpr size_t kHead = kScratchCounters * sizeof(unsigned);
   int dev = 0;
-  if (stream == hipStreamPerThread || stream_device(stream, &dev) != hipSuccess) return;
+  if (bytes > kMaxScratchBytes - kHead || stream == hipStreamPerThread || stream_device(stream, &dev) != hipSuccess) return;
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
     (void)hipGetLastError();
@@ -137,13 +170,8 @@ StreamScratch::StreamScratch(size_t bytes, hipStream_t stream) {
   }
   if (status != hipStreamCaptureStatusNone) return;
   lock = std::unique_lock<std::mutex>(g_scratch_mu);
-  StreamRegion* r = nullptr;
-  for (StreamRegion& s : g_scratch[dev])
-    if (s.ptr != nullptr && s.stream == stream) r = &s;
-  for (StreamRegion& s : g_scratch[dev])
-    if (r == nullptr && s.ptr == nullptr) r = &s;
+  StreamRegion* r = region_for(stream, dev);
   if (r == nullptr) return;
-  constexpr size_t kHead = kScratchCounters * sizeof(unsigned);
   if (r->bytes < kHead + bytes) {
     size_t want = r->bytes > 0 ? 2 * r->bytes : (size_t)1 << 18;
     while (want < kHead + bytes) want *= 2;
@@ -162,8 +190,11 @@ StreamScratch::StreamScratch(size_t bytes, hipStream_t stream) {
       std::lock_guard<std::mutex> retire(g_mu);
       g_retired.push_back(r->ptr);
     }
-    *r = StreamRegion{stream, p, want};
+    r->ptr = p;
+    r->bytes = want;
   }
+  r->stream = stream;
+  r->used = ++g_scratch_uses;
   counters = static_cast<unsigned*>(r->ptr);
   ptr = static_cast<char*>(r->ptr) + kHead;
 }

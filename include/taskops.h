@@ -21,9 +21,11 @@
  * time on different streams race on that workspace (as the reference's statics do);
  * calls on one stream are safe.  reward_to_go, leaky and fp8_linear, and efficient_kan where
  * it does not pack weights (other spline orders than 3, more than 16 knots), hold no such
- * shared memory and may overlap: what scratch they use belongs to the stream (up to 8 streams'
- * per device are kept, at most a few tens of MB each; other streams, hipStreamPerThread and
- * captures run without).
+ * shared memory and may overlap: what scratch they use belongs to the stream.  Up to 8 streams
+ * per device have some at a time, at most 64 MB each; a stream whose work has completed gives
+ * its own to another that needs it.  Further busy streams, hipStreamPerThread, captures and
+ * calls that would need more run without.  Destroy a stream only once the calls on it have
+ * completed.
  *
  * Raw-bit types are used at the boundary for the two non-C element types:
  *   e4m3 (OCP FP8, 1 byte)  -> uint8_t   (the reference uses __nv_fp8_e4m3)

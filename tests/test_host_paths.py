@@ -122,3 +122,49 @@ KAN_FAST = [(1710, 1000, 100, 5), (1499, 1000, 100, 5), (6561, 32, 128, 5), (282
 def test_kan_routes(host):
     assert kan_kernel(host, *KAN_DIRECT) == ["direct"] * len(KAN_DIRECT)
     assert kan_kernel(host, *KAN_FAST) == ["fast"] * len(KAN_FAST)
+
+
+def split(step):
+    """Whether a FEW_LONG_ROWS call ran split over workgroups (two launches)."""
+    assert step["rc"] == 0
+    return len([k for k in kernels(step) if "reward_to_go" in k]) == 2
+
+
+def test_streams_at_rest_give_their_scratch_back(host):
+    """Ten streams one after another, each idle when the next one calls: all of them split."""
+    out = host([call("reward_to_go", stream=s, **FEW_LONG_ROWS) for s in range(3, 13)])
+    assert all(split(s) for s in out)
+    assert sum(line.startswith("malloc") for s in out for line in s["log"]) == 8
+
+
+def test_destroyed_streams_give_their_scratch_back(host):
+    first = [call("reward_to_go", stream=s, **FEW_LONG_ROWS) for s in range(3, 11)]
+    busy = [put("stream_state", s, 1) for s in range(3, 11)]
+    out = host(first + busy + [call("reward_to_go", stream=20, **FEW_LONG_ROWS), put("stream_state", 6, 2),
+                               call("reward_to_go", stream=20, **FEW_LONG_ROWS)])
+    assert not split(out[16]) and split(out[18])
+
+
+def test_busy_and_capturing_streams_keep_their_scratch(host):
+    """No region is taken from a stream with work in flight or one that captures, whose capture
+    stays whole; the owners still have theirs afterwards."""
+    first = [call("reward_to_go", stream=s, **FEW_LONG_ROWS) for s in range(3, 11)]
+    busy = [put("stream_state", s, 1) for s in range(3, 10)] + [put("capturing", 10, 1), put("global_capture", 1)]
+    out = host(first + busy + [call("reward_to_go", stream=20, **FEW_LONG_ROWS), call("reward_to_go", stream=5, **FEW_LONG_ROWS)])
+    assert not split(out[-2]) and split(out[-1])
+    assert not any(line.startswith("capture_broken") for line in out[-2]["log"]), out[-2]["log"]
+
+
+def test_the_least_recently_used_scratch_goes_first(host):
+    order = [3, 4, 5, 6, 7, 8, 9, 10, 3, 4]  # 5 is the oldest use
+    steps = [call("reward_to_go", stream=s, **FEW_LONG_ROWS) for s in order]
+    steps += [put("stream_state", s, 1) for s in range(3, 11)] + [put("stream_state", 5, 0), put("stream_state", 9, 0)]
+    out = host(steps + [call("reward_to_go", stream=20, **FEW_LONG_ROWS), call("reward_to_go", stream=9, **FEW_LONG_ROWS),
+                        put("stream_state", 9, 1), put("stream_state", 20, 1), call("reward_to_go", stream=5, **FEW_LONG_ROWS)])
+    assert split(out[-5]) and split(out[-4]) and not split(out[-1])
+
+
+def test_scratch_is_bounded(host):
+    """Maps for 2^31 steps, more than a region may hold: unsplit, and nothing is allocated."""
+    out = host([call("reward_to_go", stream=3, gamma=0.99, B=256, T=1 << 27)])[0]
+    assert not split(out) and not any(line.startswith("malloc") for line in out["log"])

@@ -124,3 +124,25 @@ def test_direct_few_splits_after_many(lib):
         got = capi.run_op(lib, "efficient_kan", few)["out"].cpu().numpy()
         t = tally(got, want, tasks.load_task("efficient_kan")["tolerance"])
         assert t["mismatched"] == 0, (B, I, t)
+
+
+def test_direct_on_many_streams(lib):
+    """Ten streams at once, more than hold scratch memory, in 2 to 16 splits (arrival counters)
+    and more (a second launch): every call's result is its own, also when repeated."""
+    print("\n[kan_direct] ten streams", flush=True)
+    streams = [torch.cuda.Stream() for _ in range(10)]
+    args = []
+    for k in range(10):
+        B, I, O = [(70, 9, 30), (300, 40, 128), (20, 333, 131), (512, 60, 256), (5, 208, 448)][k % 5]
+        inp = inputs.make_inputs("efficient_kan", dict(name="d", seed=60 + k, B=B, I=I, O=O, grid_size=12, spline_order=3))
+        a = capi.device_args("efficient_kan", inp)
+        a["out"] = torch.zeros(B, O, device="cuda")
+        args.append((inp, a))
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for s, (_, a) in zip(streams, args):
+            capi.call(lib, "efficient_kan", a, s.cuda_stream)
+    torch.cuda.synchronize()
+    for inp, a in args:
+        t = tally(a["out"].cpu().numpy(), exact.efficient_kan(inp)["out"], tasks.load_task("efficient_kan")["tolerance"])
+        assert t["mismatched"] == 0, t

@@ -2,6 +2,8 @@
 chunk edges, odd row lengths, offset pointers, streams and captures, against the fp64 oracle
 at the task tolerance (atol = rtol = 1e-5; the fp32 steps from fp64 carries measure at most
 0.25 of it at these discounts)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -81,6 +83,28 @@ def test_split_on_many_streams(lib):
     for inp, a in args:
         t = tally(a["output"].cpu(), exact.reward_to_go(inp)["output"], TOL)
         assert t["mismatched"] == 0, t
+
+
+def test_split_on_streams_that_come_and_go(lib):
+    """Twelve streams one after another, each destroyed once its call has completed."""
+    print("\n[rtg] streams that come and go", flush=True)
+    with open("/proc/self/maps") as f:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+    inp = _case(4, 50_000)
+    a = capi.device_args("reward_to_go", inp)
+    out = a["output"] = torch.zeros(4, 50_000, device="cuda")
+    torch.cuda.synchronize()
+    want = exact.reward_to_go(inp)["output"]
+    for _ in range(12):
+        s = ctypes.c_void_p()
+        assert hip.hipStreamCreate(ctypes.byref(s)) == 0
+        out.zero_()
+        torch.cuda.synchronize()
+        for _ in range(2):
+            capi.call(lib, "reward_to_go", a, s.value)
+        assert hip.hipStreamSynchronize(s) == 0
+        assert hip.hipStreamDestroy(s) == 0
+        assert tally(out.cpu(), want, TOL)["mismatched"] == 0
 
 
 def test_split_under_capture(lib):
