@@ -164,23 +164,33 @@ hipError_t workspace_if_possible(WorkspaceSlot slot, size_t bytes, hipStream_t s
 
 // Scratch memory of one stream, for calls of two launches whose callers may be on several
 // streams and threads at once: launches on the stream use it one after another, and the lock
-// keeps other threads' calls from enqueuing between this call's launches.  A stream that finds
-// every region taken gets the least recently used one whose stream has nothing left to run or
-// has been destroyed (whose work has then completed: taskops.h asks callers for that).  An event
-// behind each use would say the same without asking, but costs the next launch 2 to 4 us (16 x
-// 65536 reward_to_go 8.1 -> 11.9, with the event on the kernel's own packet 10.9).
+// keeps other threads' calls from enqueuing between this call's launches.
+// A region goes by its stream's handle; streams are only destroyed once their calls have
+// completed (taskops.h), so a handle that a new stream was given brings an idle region with it.
+// As soon as a second stream has a region, every use ends with an event (`done`) on its last
+// launch, and a stream that finds all regions taken gets the least recently used one whose
+// event has completed.  Only events tell: a stream may be gone, and its handle must not be
+// asked.  With one stream there is no event, which costs the next launch 1 to 3 us (16 x 65536
+// reward_to_go 8.1 -> 10.9 on its packet, 11.9 recorded behind it); the last use before a second
+// stream came keeps its region until its stream uses it again.
 // ptr is null when there is none, and the caller takes a path that needs none: for more than
 // kMaxScratchBytes, while the stream is capturing (a graph may be replayed beside other work),
-// for hipStreamPerThread (one handle, many streams), when kMaxScratchStreams other streams have
-// work in flight, or when memory is short.
+// for hipStreamPerThread (one handle, many streams), when kMaxScratchStreams other streams hold
+// theirs, or when memory is short.
 // Not cleared, except for kScratchCounters arrival counters, which start at zero and which
 // every launch leaves at zero.  Grown by doubling; replaced memory is kept until the process
 // exits, so a region holds at most 2 kMaxScratchBytes.
+struct StreamRegion;
 struct StreamScratch {
   StreamScratch(size_t bytes, hipStream_t stream);
-  std::unique_lock<std::mutex> lock;
+  void ended();  // the last launch, with `done` as its stop event, was enqueued
   unsigned* counters = nullptr;
   void* ptr = nullptr;
+  hipEvent_t done = nullptr;  // null: this use needs no event
+
+ private:
+  std::unique_lock<std::mutex> lock_;
+  StreamRegion* region_ = nullptr;
 };
 constexpr int kScratchCounters = 1024;
 constexpr int kMaxScratchStreams = 8;

@@ -1,4 +1,6 @@
 // Host side of efficient_kan's direct fp32 path (efficient_kan_direct.hpp).
+#include <hip/hip_ext.h>
+
 #include <algorithm>
 #include <optional>
 
@@ -75,14 +77,22 @@ hipError_t launch(const float* x, const float* grid, const float* wb, const floa
   nsplit = plan.nsplit;
   if (nsplit > kMaxArrivals || tiles > kScratchCounters) counters = nullptr;
   const int64_t pairs = (int64_t)ctiles * nsplit, span = std::min<int64_t>(8, pairs), padded = (pairs + span - 1) / span * span;
-  hipLaunchKernelGGL((kan_direct::kan_direct<kNQ, kR>), dim3((unsigned)(padded * mtiles)), dim3(kThreads), plan.lds, stream,
-                     x, grid, wb, ws, sc, order, L, C, B, I, O, mtiles, ctiles, nsplit, plan.cper, partial,
-                     counters, out);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess || nsplit == 1 || counters != nullptr) return e;
-  hipLaunchKernelGGL(kan_direct_sum<kR>, dim3((unsigned)(tiles * 4 * kR)), dim3(kThreads), 0, stream,
-                     static_cast<const float*>(partial), B, O, mtiles, ctiles, nsplit, out);
-  return hipGetLastError();
+  auto enqueue = [&](bool last, auto kernel, dim3 groups, size_t lds, auto... args) {
+    const hipEvent_t done = last && scratch && scratch->ptr != nullptr ? scratch->done : nullptr;
+    if (done != nullptr)
+      hipExtLaunchKernelGGL(kernel, groups, dim3(kThreads), (unsigned)lds, stream, nullptr, done, 0, args...);
+    else
+      hipLaunchKernelGGL(kernel, groups, dim3(kThreads), lds, stream, args...);
+    const hipError_t e = hipGetLastError();
+    if (done != nullptr && e == hipSuccess) scratch->ended();
+    return e;
+  };
+  const bool one = nsplit == 1 || counters != nullptr;
+  const hipError_t e = enqueue(one, kan_direct::kan_direct<kNQ, kR>, dim3((unsigned)(padded * mtiles)), plan.lds, x, grid,
+                               wb, ws, sc, order, L, C, B, I, O, mtiles, ctiles, nsplit, plan.cper, partial, counters, out);
+  if (e != hipSuccess || one) return e;
+  return enqueue(true, kan_direct_sum<kR>, dim3((unsigned)(tiles * 4 * kR)), (size_t)0,
+                 static_cast<const float*>(partial), B, O, mtiles, ctiles, nsplit, out);
 }
 
 template <int kNQ>

@@ -5,6 +5,16 @@
 #include "common.hpp"
 
 namespace taskops {
+
+struct StreamRegion {
+  hipStream_t stream = nullptr;
+  void* ptr = nullptr;
+  size_t bytes = 0;
+  hipEvent_t event = nullptr;
+  bool ended = false;  // the last use has its event
+  uint64_t used = 0;   // g_scratch_uses at the last use
+};
+
 namespace {
 
 constexpr int kMaxDevices = 64;
@@ -12,13 +22,6 @@ constexpr int kMaxDevices = 64;
 struct Region {
   void* ptr = nullptr;
   size_t bytes = 0;
-};
-
-struct StreamRegion {
-  hipStream_t stream = nullptr;
-  void* ptr = nullptr;
-  size_t bytes = 0;
-  uint64_t used = 0;  // g_scratch_uses at the last use
 };
 
 std::mutex g_mu;
@@ -131,20 +134,8 @@ hipError_t workspace_if_possible(WorkspaceSlot slot, size_t bytes, hipStream_t s
 
 namespace {
 
-// Whether a region's stream has completed everything enqueued on it, or no longer exists.  A
-// capturing stream is not asked, which would end its capture.
-bool at_rest(hipStream_t stream) {
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  hipError_t e = hipStreamIsCapturing(stream, &status);
-  if (e == hipSuccess && status == hipStreamCaptureStatusNone) e = hipStreamQuery(stream);
-  else if (e == hipSuccess) e = hipErrorNotReady;
-  if (e == hipSuccess) return true;
-  (void)hipGetLastError();
-  return e == hipErrorContextIsDestroyed || e == hipErrorInvalidHandle;
-}
-
-// The region of `stream`: its own, an unused one, or one whose stream is at rest; null when every
-// other stream with a region has work in flight (g_scratch_mu held).
+// The region of `stream`: its own, an unused one, or the least recently used one whose last use
+// is known to have completed; null when there is none (g_scratch_mu held).
 StreamRegion* region_for(hipStream_t stream, int dev) {
   for (StreamRegion& s : g_scratch[dev])
     if (s.ptr != nullptr && s.stream == stream) return &s;
@@ -152,8 +143,11 @@ StreamRegion* region_for(hipStream_t stream, int dev) {
     if (s.ptr == nullptr) return &s;
   StreamRegion* r = nullptr;
   const RelaxedCapture relaxed;
-  for (StreamRegion& s : g_scratch[dev])
-    if ((r == nullptr || s.used < r->used) && at_rest(s.stream)) r = &s;
+  for (StreamRegion& s : g_scratch[dev]) {
+    if (!s.ended || (r != nullptr && s.used > r->used)) continue;
+    if (hipEventQuery(s.event) == hipSuccess) r = &s;
+    else (void)hipGetLastError();
+  }
   return r;
 }
 
@@ -169,7 +163,7 @@ StreamScratch::StreamScratch(size_t bytes, hipStream_t stream) {
     return;
   }
   if (status != hipStreamCaptureStatusNone) return;
-  lock = std::unique_lock<std::mutex>(g_scratch_mu);
+  lock_ = std::unique_lock<std::mutex>(g_scratch_mu);
   StreamRegion* r = region_for(stream, dev);
   if (r == nullptr) return;
   if (r->bytes < kHead + bytes) {
@@ -177,7 +171,8 @@ StreamScratch::StreamScratch(size_t bytes, hipStream_t stream) {
     while (want < kHead + bytes) want *= 2;
     void* p = nullptr;
     const RelaxedCapture relaxed;
-    if (hipMalloc(&p, want) != hipSuccess) {
+    if ((r->event == nullptr && hipEventCreateWithFlags(&r->event, hipEventDisableTiming) != hipSuccess) ||
+        hipMalloc(&p, want) != hipSuccess) {
       (void)hipGetLastError();
       return;
     }
@@ -195,9 +190,15 @@ StreamScratch::StreamScratch(size_t bytes, hipStream_t stream) {
   }
   r->stream = stream;
   r->used = ++g_scratch_uses;
+  r->ended = false;
+  for (const StreamRegion& s : g_scratch[dev])
+    if (s.ptr != nullptr && &s != r) done = r->event;
+  region_ = r;
   counters = static_cast<unsigned*>(r->ptr);
   ptr = static_cast<char*>(r->ptr) + kHead;
 }
+
+void StreamScratch::ended() { region_->ended = done != nullptr; }
 
 int device_cu_count() {
   int dev = 0;

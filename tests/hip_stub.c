@@ -18,12 +18,12 @@
 static int s_capturing[64];      /* by stream handle */
 static int s_global_capture;     /* another stream captures in global mode: see unsafe() */
 static int s_malloc_fails;
-static int s_state[64];          /* by stream handle: 0 at rest, 1 work in flight, 2 destroyed */
+static int s_busy[64];           /* by stream handle: events on it have not completed */
 
 void stub_set_capturing(int stream, int on) { s_capturing[stream] = on; }
 void stub_set_global_capture(int on) { s_global_capture = on; }
 void stub_set_malloc_fails(int on) { s_malloc_fails = on; }
-void stub_set_stream_state(int stream, int state) { s_state[stream] = state; }
+void stub_set_busy(int stream, int on) { s_busy[stream] = on; }
 
 /* ---- the record: one line per call of interest ---- */
 static char* g_log;
@@ -74,7 +74,6 @@ hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) {
 }
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* st) {
   if (s == NULL && s_global_capture) return hipErrorStreamCaptureImplicit;
-  if (s_state[(size_t)s % 64] == 2) return hipErrorContextIsDestroyed;
   *st = s_capturing[(size_t)s % 64] ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
   return hipSuccess;
 }
@@ -105,12 +104,17 @@ hipError_t hipMalloc(void** p, size_t n) {
 }
 hipError_t hipFree(void* p) { NOTE("free %p", p); free(p); return hipSuccess; }
 
-/* ---- streams ---- */
-hipError_t hipStreamQuery(hipStream_t s) {
-  if (s_capturing[(size_t)s % 64]) NOTE("capture_broken hipStreamQuery");
-  if (unsafe("hipStreamQuery")) return hipErrorStreamCaptureUnsupported;
-  NOTE("query stream %zu", (size_t)s);
-  return s_state[(size_t)s % 64] == 2 ? hipErrorContextIsDestroyed : s_state[(size_t)s % 64] ? hipErrorNotReady : hipSuccess;
+/* ---- events: each stands for the stream of its last record ---- */
+static size_t g_event_stream[1024];
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned f) {
+  static size_t n;
+  (void)f;
+  *e = (hipEvent_t)(++n);
+  return hipSuccess;
+}
+hipError_t hipEventQuery(hipEvent_t e) {
+  if (unsafe("hipEventQuery")) return hipErrorStreamCaptureUnsupported;
+  return s_busy[g_event_stream[(size_t)e]] ? hipErrorNotReady : hipSuccess;
 }
 
 /* ---- launches ---- */
@@ -123,8 +127,7 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t*
   *g = t_cfg.g; *b = t_cfg.b; *lds = t_cfg.lds; *s = t_cfg.s;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** a, size_t lds, hipStream_t s) {
-  (void)a;
+static hipError_t launch(const void* f, dim3 g, dim3 b, size_t lds, hipStream_t s, hipEvent_t stop) {
   const char* name = "?";
   for (int i = 0; i < g_nfn; ++i)
     if (g_fn[i].host == f) name = g_fn[i].name;
@@ -132,6 +135,16 @@ hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** a, size_t lds, 
     NOTE("refused %s", name);
     return hipErrorInvalidConfiguration;
   }
-  NOTE("launch %s grid %u %u block %u lds %zu stream %zu", name, g.x, g.y, b.x, lds, (size_t)s);
+  if (stop) g_event_stream[(size_t)stop] = (size_t)s % 64;
+  NOTE("launch %s grid %u %u block %u lds %zu stream %zu%s", name, g.x, g.y, b.x, lds, (size_t)s, stop ? " event" : "");
   return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** a, size_t lds, hipStream_t s) {
+  (void)a;
+  return launch(f, g, b, lds, s, NULL);
+}
+hipError_t hipExtLaunchKernel(const void* f, dim3 g, dim3 b, void** a, size_t lds, hipStream_t s, hipEvent_t e0,
+                              hipEvent_t e1, int flags) {
+  (void)a; (void)e0; (void)flags;
+  return launch(f, g, b, lds, s, e1);
 }

@@ -124,47 +124,43 @@ def test_kan_routes(host):
     assert kan_kernel(host, *KAN_FAST) == ["fast"] * len(KAN_FAST)
 
 
+def fine(stream):
+    return call("efficient_kan", stream=stream, **FINE_KNOTS)
+
+
 def split(step):
-    """Whether a FEW_LONG_ROWS call ran split over workgroups (two launches)."""
+    """Whether a FINE_KNOTS call ran with its features split over workgroups (128 tiles)."""
     assert step["rc"] == 0
-    return len([k for k in kernels(step) if "reward_to_go" in k]) == 2
+    line, = [line for line in step["log"] if "kan_directI" in line]
+    return int(line.split("grid ")[1].split()[0]) > 128
 
 
-def test_streams_at_rest_give_their_scratch_back(host):
-    """Ten streams one after another, each idle when the next one calls: all of them split."""
-    out = host([call("reward_to_go", stream=s, **FEW_LONG_ROWS) for s in range(3, 13)])
+def test_one_streams_calls_carry_no_event(host):
+    out = host([fine(3), fine(3)])
+    assert all(split(s) and not any(line.endswith("event") for line in s["log"]) for s in out)
+
+
+def test_streams_give_their_scratch_back(host):
+    """Twelve streams, each done when the next one calls: all of them split, on eight regions.
+    The first one's only use had no event, so its region stays its own."""
+    out = host([fine(s) for s in range(3, 15)] + [fine(3)])
     assert all(split(s) for s in out)
-    assert sum(line.startswith("malloc") for s in out for line in s["log"]) == 8
+    assert sum(line.startswith("malloc") for s in out for line in s["log"]) <= 16  # regions and one growth each
+    assert not any(line.startswith("malloc") for s in out[8:] for line in s["log"])
+    assert all(s["log"][-1].endswith("event") for s in out[1:])
 
 
-def test_destroyed_streams_give_their_scratch_back(host):
-    first = [call("reward_to_go", stream=s, **FEW_LONG_ROWS) for s in range(3, 11)]
-    busy = [put("stream_state", s, 1) for s in range(3, 11)]
-    out = host(first + busy + [call("reward_to_go", stream=20, **FEW_LONG_ROWS), put("stream_state", 6, 2),
-                               call("reward_to_go", stream=20, **FEW_LONG_ROWS)])
-    assert not split(out[16]) and split(out[18])
-
-
-def test_busy_and_capturing_streams_keep_their_scratch(host):
-    """No region is taken from a stream with work in flight or one that captures, whose capture
-    stays whole; the owners still have theirs afterwards."""
-    first = [call("reward_to_go", stream=s, **FEW_LONG_ROWS) for s in range(3, 11)]
-    busy = [put("stream_state", s, 1) for s in range(3, 10)] + [put("capturing", 10, 1), put("global_capture", 1)]
-    out = host(first + busy + [call("reward_to_go", stream=20, **FEW_LONG_ROWS), call("reward_to_go", stream=5, **FEW_LONG_ROWS)])
+def test_busy_streams_keep_their_scratch(host):
+    """No region is taken from a stream whose last call has not completed, and asking about
+    them leaves another stream's capture whole; the owners still have theirs afterwards."""
+    busy = [put("busy", s, 1) for s in range(3, 11)] + [put("capturing", 30, 1), put("global_capture", 1)]
+    out = host([fine(s) for s in range(3, 11)] + busy + [fine(20), fine(5)])
     assert not split(out[-2]) and split(out[-1])
     assert not any(line.startswith("capture_broken") for line in out[-2]["log"]), out[-2]["log"]
 
 
 def test_the_least_recently_used_scratch_goes_first(host):
     order = [3, 4, 5, 6, 7, 8, 9, 10, 3, 4]  # 5 is the oldest use
-    steps = [call("reward_to_go", stream=s, **FEW_LONG_ROWS) for s in order]
-    steps += [put("stream_state", s, 1) for s in range(3, 11)] + [put("stream_state", 5, 0), put("stream_state", 9, 0)]
-    out = host(steps + [call("reward_to_go", stream=20, **FEW_LONG_ROWS), call("reward_to_go", stream=9, **FEW_LONG_ROWS),
-                        put("stream_state", 9, 1), put("stream_state", 20, 1), call("reward_to_go", stream=5, **FEW_LONG_ROWS)])
+    steps = [fine(s) for s in order] + [put("busy", s, 1) for s in range(3, 11) if s not in (5, 9)]
+    out = host(steps + [fine(20), fine(9), put("busy", 9, 1), put("busy", 20, 1), fine(5)])
     assert split(out[-5]) and split(out[-4]) and not split(out[-1])
-
-
-def test_scratch_is_bounded(host):
-    """Maps for 2^31 steps, more than a region may hold: unsplit, and nothing is allocated."""
-    out = host([call("reward_to_go", stream=3, gamma=0.99, B=256, T=1 << 27)])[0]
-    assert not split(out) and not any(line.startswith("malloc") for line in out["log"])

@@ -3,6 +3,7 @@ row blocks, column tiles, feature chunks and basis groups at their edges, agains
 oracle at the task tolerance (atol = rtol = 1e-5: the path's fp32 sums of at most a few
 hundred terms of size below one round to about 1e-6).  The fast path's ragged tiles are
 covered at batches large enough to take it."""
+import ctypes
 import subprocess
 import sys
 from pathlib import Path
@@ -146,3 +147,34 @@ def test_direct_on_many_streams(lib):
     for inp, a in args:
         t = tally(a["out"].cpu().numpy(), exact.efficient_kan(inp)["out"], tasks.load_task("efficient_kan")["tolerance"])
         assert t["mismatched"] == 0, t
+
+
+def test_direct_on_streams_that_come_and_go(lib):
+    """Twelve streams one after another, each destroyed once its calls have completed, then the
+    default one: their scratch regions change hands."""
+    print("\n[kan_direct] streams that come and go", flush=True)
+    with open("/proc/self/maps") as f:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+    cases = []
+    for B, I, O in [(300, 40, 128), (20, 333, 131)]:
+        inp = inputs.make_inputs("efficient_kan", dict(name="d", seed=90 + B, B=B, I=I, O=O, grid_size=12, spline_order=3))
+        a = capi.device_args("efficient_kan", inp)
+        a["out"] = torch.zeros(B, O, device="cuda")
+        cases.append((a, exact.efficient_kan(inp)["out"]))
+    torch.cuda.synchronize()
+    for k in range(13):
+        s = ctypes.c_void_p()
+        if k < 12:
+            assert hip.hipStreamCreate(ctypes.byref(s)) == 0
+        for a, _ in cases:
+            a["out"].zero_()
+        torch.cuda.synchronize()
+        for _ in range(2):
+            for a, _ in cases:
+                capi.call(lib, "efficient_kan", a, s.value or 0)
+        assert hip.hipStreamSynchronize(s) == 0
+        if k < 12:
+            assert hip.hipStreamDestroy(s) == 0
+        for a, want in cases:
+            t = tally(a["out"].cpu().numpy(), want, tasks.load_task("efficient_kan")["tolerance"])
+            assert t["mismatched"] == 0, (k, t)
