@@ -170,8 +170,8 @@ hipError_t workspace_if_possible(WorkspaceSlot slot, size_t bytes, hipStream_t s
 // As soon as a second stream has a region, every use ends with an event (`done`) on its last
 // launch, and a stream that finds all regions taken gets the least recently used one whose
 // event has completed.  Only events tell: a stream may be gone, and its handle must not be
-// asked.  With one stream there is no event, which costs the next launch 1 to 3 us (16 x 65536
-// reward_to_go 8.1 -> 10.9 on its packet, 11.9 recorded behind it); the last use before a second
+// asked.  With one stream there is no event, which costs the next launch 1 to 3 us (a call of 8.1
+// us 10.9 with it on the kernel's packet, 11.9 recorded behind it); the last use before a second
 // stream came keeps its region until its stream uses it again.
 // ptr is null when there is none, and the caller takes a path that needs none: for more than
 // kMaxScratchBytes, while the stream is capturing (a graph may be replayed beside other work),

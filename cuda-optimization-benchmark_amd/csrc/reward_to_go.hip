@@ -9,6 +9,7 @@
 // of one 8-step-per-lane chunk (whose 16-byte accesses cover every other 16 bytes per
 // instruction, and which slows to 39 us with non-temporal stores).  Shorter rows use fewer
 // waves and chunks per wave, so no wave idles.
+#include <algorithm>
 #include <cmath>
 
 #include "reward_to_go.hpp"
@@ -45,35 +46,56 @@ void launch(const float* reward, const uint8_t* done, double g, int B, int T, fl
     const int nb = B - b0 < kRowsPerLaunch ? B - b0 : kRowsPerLaunch;
     const size_t off = (size_t)b0 * (size_t)T;  // T % 4 == 0 on the aligned path: alignment kept
     hipLaunchKernelGGL((reward_to_go_kernel<kWaves, kPerLane, kSeg, kAccess, policy<kAccess>()>), dim3(nb),
-                       dim3(kWaves * kWave), lds, stream, reward + off, done + off, g, nb, T, out + off, 1, 0,
-                       static_cast<RtgMap*>(nullptr));
+                       dim3(kWaves * kWave), lds, stream, reward + off, done + off, g, nb, T, out + off, 1, 0);
   }
 }
 
 // Few long rows.  A workgroup walks its row one segment of 4096 steps after another, about 2.2
 // us each, so such rows are split into parts over workgroups: one launch composes each part's
 // map, a second scans each part from the maps after it, reading the rewards again (from the
-// caches).  Whole row against split, us per call: 16 x 65536 33-39 / 8.5, 1 x 131072 71 / 7.9,
-// 6 x 18592 12.4 / 7.8, 33 x 109969 75.6 / 13.6, 128 x 131072 82.7 / 38.9, 256 x 65536 46.2 / 39.1.
+// caches).  Whole row against split, us per call: 16 x 65536 33-39 / 7.6, 1 x 131072 71 / 6.9,
+// 6 x 18592 12.4 / 6.5, 33 x 109969 75-140 / 14.0, 128 x 131072 82.7 / 40.8, 256 x 65536 46.2 / 39.8, 1 x
+// 1048576 600 / 14.7, 256 x 1048576 689 / 689.
 // Rows of at most 12288 steps (three segments) or more than 256 of them keep the whole-row
 // form: 1 x 8000 5.7 / 8.0, 229 x 9751 11.5 / 11.6, 256 x 16384 13.3 / 13.3, 512 x 8192 9.5 / 13.3.
 constexpr int kSplitMaxRows = 256, kSplitMinChunks = 48;
-// Up to this many chunks in all, parts of 4 chunks (up to 1024 workgroups), else of 16: 64 x
-// 16384 8.5 against 8.7 us, 33 x 109969 17.8 against 13.6.
-constexpr int kSmallPartChunks = 4096;
+// Chunks in all up to which parts have 4 chunks and 8, one and two per wave; beyond, four per wave
+// in 16 or more: at 4, 8 and 16 16 x 65536 8.5, 7.6 and 8.3 us, 64 x 16384 8.1, 7.4 and 8.2, 8 x 65536
+// 7.1, 7.2 and 8.1, 4 x 65536 6.5 and 6.7.  More parts would not find room for their maps either.
+constexpr int kPart4Chunks = 1024, kPart8Chunks = 4096;
+static_assert(kPart4Chunks / 4 <= 4 * kRtgMapsPerChunk && kPart8Chunks / 8 <= 8 * kRtgMapsPerChunk, "room for the maps");
+// Chunks per part of a call in parts of 16 or more: more where a part's outputs have no room for
+// the maps after it (rows past 4.2 M steps), and beyond what fills the chip where the maps'
+// copies, one to each earlier part, add up: 8 x 2097152 71.6 us in 512 parts a row, 47.3 in 256.
+int long_part(int B, int nchunks) {
+  const int64_t nseg = ((int64_t)nchunks + 15) / 16;
+  int64_t m = std::max<int64_t>((nseg + 16 * kRtgMapsPerChunk - 1) / (16 * kRtgMapsPerChunk), B * nseg / 4096);
+  for (m = std::max<int64_t>(m, 1);; ++m) {
+    const int64_t n = (nseg + m - 1) / m;  // parts of a row
+    if (B * n <= 1024 || (B * n <= 4096 && n <= 128 * m)) return (int)(16 * m);
+  }
+}
 
 template <int kSeg, RtgAccess kAccess>
 hipError_t launch_split(const float* reward, const uint8_t* done, double g, int B, int T, float* out, int nparts,
-                        int cpart, RtgMap* maps, hipStream_t stream) {
+                        int cpart, hipStream_t stream) {
   constexpr int kWaves = 4;
   // Ordinary loads in the first pass, so that the second finds the rewards in the caches.
   hipLaunchKernelGGL((reward_to_go_kernel<kWaves, kPerLane, kSeg, kAccess, 0, kMaps>), dim3(B * nparts),
-                     dim3(kWaves * kWave), 0, stream, reward, done, g, B, T, out, nparts, cpart, maps);
+                     dim3(kWaves * kWave), 0, stream, reward, done, g, B, T, out, nparts, cpart);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((reward_to_go_kernel<kWaves, kPerLane, kSeg, kAccess, policy<kAccess>(), kApply>), dim3(B * nparts),
-                     dim3(kWaves * kWave), 0, stream, reward, done, g, B, T, out, nparts, cpart, maps);
+                     dim3(kWaves * kWave), 0, stream, reward, done, g, B, T, out, nparts, cpart);
   return hipGetLastError();
+}
+
+// Whether a call's output shares memory with an input (each workgroup reads its rewards before
+// it writes there, so the whole-row form allows that; the maps of split rows do not).
+bool overlaps(const float* reward, const uint8_t* done, int B, int T, const float* out) {
+  const uintptr_t n = (uintptr_t)B * (uintptr_t)T, o = reinterpret_cast<uintptr_t>(out);
+  auto with = [&](uintptr_t p, uintptr_t bytes) { return p < o + 4 * n && o < p + bytes; };
+  return with(reinterpret_cast<uintptr_t>(reward), 4 * n) || with(reinterpret_cast<uintptr_t>(done), n);
 }
 
 template <RtgAccess kAccess>
@@ -82,13 +104,12 @@ hipError_t run(const float* reward, const uint8_t* done, double g, int B, int T,
   if constexpr (kAccess != kElements) {
     // |g| <= 1: a part's a = g^steps cannot overflow (inf * 0 would make the carry NaN).
     if (B <= kSplitMaxRows && nchunks > kSplitMinChunks && std::fabs(g) <= 1.0) {
-      const bool big = (int64_t)B * nchunks > kSmallPartChunks;
-      const int cpart = big ? 16 : 4, nparts = (nchunks + cpart - 1) / cpart;
-      StreamScratch scratch((size_t)B * nparts * sizeof(RtgMap), stream);
-      if (scratch.ptr != nullptr) {
-        auto* maps = static_cast<RtgMap*>(scratch.ptr);
-        return big ? launch_split<4, kAccess>(reward, done, g, B, T, out, nparts, cpart, maps, stream)
-                   : launch_split<1, kAccess>(reward, done, g, B, T, out, nparts, cpart, maps, stream);
+      const int64_t all = (int64_t)B * nchunks;
+      const int cpart = all <= kPart4Chunks ? 4 : (all <= kPart8Chunks ? 8 : long_part(B, nchunks));
+      const int nparts = (nchunks + cpart - 1) / cpart;
+      if (!overlaps(reward, done, B, T, out)) {
+        auto split = cpart == 4 ? launch_split<1, kAccess> : (cpart == 8 ? launch_split<2, kAccess> : launch_split<4, kAccess>);
+        return split(reward, done, g, B, T, out, nparts, cpart, stream);
       }
     }
   }

@@ -84,31 +84,60 @@ enum RtgAccess : int { kElements = 0, kAligned = 1, kUnaligned = 2 };
 // What a workgroup does with its span of the row: kWhole, the whole row; for a row split over
 // workgroups, kMaps writes its part's composed map and kApply, in a second launch, composes
 // the maps of the parts after its own and scans its part from that value.
+//
+// The maps pass from one launch to the other in `out`: kMaps writes its part's map once into the
+// span of every earlier part of the row, at the slot of its distance, and kApply reads the maps
+// after its part from its own span, one contiguous run, before it writes its outputs over them.
+// So no memory but the caller's is used, and a call takes the same path, with the same bits, on
+// any number of streams and threads and under graph capture.
 enum RtgMode : int { kWhole = 0, kMaps = 1, kApply = 2 };
 
 // A part's map v -> r + a v.
 struct RtgMap {
   double r, a;
 };
+// Maps that the outputs of one chunk (256 floats) have room for.
+constexpr int kRtgMapsPerChunk = 64;
 
 namespace rtg_detail {
-// The maps first .. n - 1 of a row's parts composed and applied to 0, the same in every lane:
-// lane l of each batch of 64 takes one part, a suffix scan composes the batch, and batches are
-// composed from the row's end, always in this order, so the bits do not depend on timing.
-__device__ __forceinline__ double compose_after(const RtgMap* __restrict__ maps, int first, int n, int lane) {
+// Its 16 bytes at a float's alignment.
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 __attribute__((aligned(4))) u32x4u;
+__device__ __forceinline__ u32x4 pack_map(RtgMap m) {
+  const unsigned long long r = (unsigned long long)__double_as_longlong(m.r), a = (unsigned long long)__double_as_longlong(m.a);
+  return u32x4{(unsigned)r, (unsigned)(r >> 32), (unsigned)a, (unsigned)(a >> 32)};
+}
+__device__ __forceinline__ RtgMap unpack_map(u32x4 v) {
+  return RtgMap{__longlong_as_double((long long)(((unsigned long long)v.y << 32) | v.x)),
+                __longlong_as_double((long long)(((unsigned long long)v.w << 32) | v.z))};
+}
+
+// The factor of two composed maps.  Where it is too small for a double it stays the smallest one,
+// not zero: only a done step makes a factor zero, and 0 * inf would turn the infinity that an
+// infinite reward sends up its row into NaN.
+__device__ __forceinline__ double factor(double a, double b) {
+  const double p = a * b;
+  return p == 0.0 && a != 0.0 && b != 0.0 ? 0x1p-1074 : p;
+}
+
+// n maps of consecutive parts composed and applied to 0, the same in every lane: lane l of
+// each batch of 64 takes one part, a suffix scan composes the batch, and batches are composed
+// from the row's end, always in this order, so the bits do not depend on timing.
+__device__ __forceinline__ double compose_after(const u32x4u* maps, int n, int lane) {
   double v = 0.0;
-  for (int p0 = first + (n - 1 - first) / kWave * kWave; p0 >= first && first < n; p0 -= kWave) {
+  for (int p0 = (n - 1) / kWave * kWave; p0 >= 0 && n > 0; p0 -= kWave) {
     double r = 0.0, a = 1.0;
     if (p0 + lane < n) {
-      r = maps[p0 + lane].r;
-      a = maps[p0 + lane].a;
+      const RtgMap m = unpack_map(maps[p0 + lane]);
+      r = m.r;
+      a = m.a;
     }
 #pragma unroll
     for (int off = 1; off < kWave; off <<= 1) {  // (r, a): the map of lanes lane .. lane + 2 off - 1
       const double rn = __shfl_down(r, off, kWave), an = __shfl_down(a, off, kWave);
       if (lane + off < kWave) {
         r = fma(a, rn, r);
-        a *= an;
+        a = factor(a, an);
       }
     }
     v = fma(uniform(__shfl(a, 0, kWave)), v, uniform(__shfl(r, 0, kWave)));
@@ -119,12 +148,12 @@ __device__ __forceinline__ double compose_after(const RtgMap* __restrict__ maps,
 
 // kNT: bit 0 = non-temporal loads; bits 1-2 = the cache policy of buffer output stores
 // (store_row16), 0 = plain stores.  Split rows (kMode != kWhole): workgroup (row, part) =
-// (blockIdx.x / nparts, blockIdx.x % nparts) owns chunks part * cpart .. + cpart - 1 and
-// maps[row * nparts + part].
+// (blockIdx.x / nparts, blockIdx.x % nparts) owns chunks part * cpart .. + cpart - 1, at least
+// (nparts - 1) / 64 of them (a part's room for the later maps).
 template <int kWaves, int kPerLane, int kSeg, RtgAccess kAccess, int kNT, RtgMode kMode = kWhole>
 __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
     const float* __restrict__ reward, const uint8_t* __restrict__ done, double g, int B, int T,
-    float* __restrict__ out, int nparts = 1, int cpart = 0, RtgMap* __restrict__ maps = nullptr) {
+    float* __restrict__ out, int nparts = 1, int cpart = 0) {
   using namespace rtg_detail;
   static_assert(kPerLane == 4, "a lane owns one 16-byte reward vector per chunk");
   constexpr int kChunk = kWave * kPerLane;
@@ -163,7 +192,6 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
   const uint8_t* dd = done + base;
   float* oo = out + base;
   double carry = 0.0, span = 1.0;  // span: kMaps, the a of the part's chunks so far
-  if constexpr (kMode == kApply) carry = compose_after(maps + (size_t)row * nparts, part + 1, nparts, lane);
   for (int hi = end; hi > first; hi -= kWaves * kSeg) {
     const int lo = hi - first > kWaves * kSeg ? hi - kWaves * kSeg : first;
     const int c0 = lo + wave * kSeg;
@@ -204,6 +232,12 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
         }
       }
     }
+
+    // The value entering this part, while the rewards are on their way; the outputs that take the
+    // maps' place are written past the barrier below.
+    if constexpr (kMode == kApply)
+      if (hi == end)
+        carry = compose_after(reinterpret_cast<const u32x4u*>(oo + (size_t)first * kChunk), nparts - 1 - part, lane);
 
     // Lane maps and wave suffix scans.  A map is (R, A): v -> R + A*v.  A lane's A over its
     // 4 steps is 0 if one of them is a done step, else g^4; in the suffix scan every
@@ -265,8 +299,8 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
     if constexpr (kMode == kMaps) {
       double a = 1.0;
 #pragma unroll
-      for (int v = 0; v < kWaves; ++v) a *= span_a[v];
-      span *= a;
+      for (int v = 0; v < kWaves; ++v) a = factor(a, span_a[v]);
+      span = factor(span, a);
       carry = next_carry;
       __syncthreads();
       continue;
@@ -314,8 +348,11 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
     carry = next_carry;
     __syncthreads();  // span_* are rewritten by the next segment
   }
-  if constexpr (kMode == kMaps)
-    if (threadIdx.x == 0) maps[(size_t)row * nparts + part] = RtgMap{carry, span};
+  if constexpr (kMode == kMaps) {
+    const u32x4 m = pack_map(RtgMap{carry, span});
+    for (int p = (int)threadIdx.x; p < part; p += kWaves * kWave)
+      reinterpret_cast<u32x4u*>(oo + (size_t)p * cpart * kChunk)[part - p - 1] = m;
+  }
 }
 
 }  // namespace taskops

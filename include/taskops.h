@@ -19,13 +19,13 @@
  * results or derived weight contents between calls.  Calls are asynchronous: no host synchronisation and no
  * device-to-host copy happens inside a call.  Calls that share a device and overlap in
  * time on different streams race on that workspace (as the reference's statics do);
- * calls on one stream are safe.  reward_to_go, leaky and fp8_linear, and efficient_kan where
- * it does not pack weights (other spline orders than 3, more than 16 knots), hold no such
- * shared memory and may overlap: what scratch they use belongs to the stream.  Up to 8 streams
- * per device have some at a time, at most 64 MB each; a stream whose work has completed gives
- * its own to another that needs it.  Further busy streams, hipStreamPerThread, captures and
- * calls that would need more run without.  Destroy a stream only once the calls on it have
- * completed.
+ * calls on one stream are safe.  reward_to_go, leaky and fp8_linear hold no memory and may
+ * overlap (reward_to_go keeps intermediate values in `output` until it writes its results).
+ * So may efficient_kan where it does not pack weights (other spline orders than 3, more than 16
+ * knots): what scratch it uses belongs to the stream.  Up to 8 streams per device have some at
+ * a time, at most 64 MB each; a stream whose work has completed gives its own to another that
+ * needs it.  Further busy streams, hipStreamPerThread and captures run without.  Destroy a
+ * stream only once the calls on it have completed.
  *
  * Raw-bit types are used at the boundary for the two non-C element types:
  *   e4m3 (OCP FP8, 1 byte)  -> uint8_t   (the reference uses __nv_fp8_e4m3)

@@ -56,8 +56,7 @@ FINE_KNOTS = dict(grid_size=16, spline_order=3, B=1024, I=256, O=512)
 SMALL_BATCH = dict(grid_size=5, spline_order=3, B=8, I=1024, O=1024)
 
 
-@pytest.mark.parametrize("op,args", [("reward_to_go", FEW_LONG_ROWS), ("efficient_kan", FINE_KNOTS),
-                                     ("efficient_kan", SMALL_BATCH)])
+@pytest.mark.parametrize("op,args", [("efficient_kan", FINE_KNOTS), ("efficient_kan", SMALL_BATCH)])
 def test_allocating_leaves_another_streams_capture_alone(host, op, args):
     """A first call on stream 3 allocates while stream 4 captures (the stub, like the runtime,
     breaks the capture for an allocation in the default capture mode)."""
@@ -72,6 +71,18 @@ def test_allocating_leaves_another_streams_capture_alone(host, op, args):
 def test_a_capturing_stream_allocates_nothing(host, op, args):
     out = host([put("capturing", 4, 1), put("global_capture", 1), call(op, stream=4, **args)])[-1]
     assert out["rc"] == 0 and not any(line.startswith(("malloc", "capture_broken")) for line in out["log"]), out["log"]
+
+
+@pytest.mark.parametrize("capturing", [0, 1])
+def test_split_rows_use_no_memory_of_the_library(host, capturing):
+    """Few long rows take two launches on any stream, under capture too, and allocate nothing;
+    an output that shares memory with an input takes the whole-row form."""
+    out = host([put("capturing", 4, capturing)] + [call("reward_to_go", stream=s, **FEW_LONG_ROWS) for s in (4, 0, 2)]
+               + [call("reward_to_go", stream=4, reward=1 << 41, output=(1 << 41) + 64, **FEW_LONG_ROWS),
+                  call("reward_to_go", stream=4, done=(1 << 41) + 4 * 16 * 65536 - 4, output=1 << 41, **FEW_LONG_ROWS),
+                  call("reward_to_go", stream=4, done=(1 << 41) + 4 * 16 * 65536, output=1 << 41, **FEW_LONG_ROWS)])
+    assert [len(kernels(s)) for s in out[1:]] == [2, 2, 2, 1, 1, 2]
+    assert not any(line.startswith("malloc") for s in out for line in s["log"])
 
 
 def fp8_kernel(host, *sizes, x=0):

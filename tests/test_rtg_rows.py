@@ -2,8 +2,6 @@
 chunk edges, odd row lengths, offset pointers, streams and captures, against the fp64 oracle
 at the task tolerance (atol = rtol = 1e-5; the fp32 steps from fp64 carries measure at most
 0.25 of it at these discounts)."""
-import ctypes
-
 import numpy as np
 import pytest
 import torch
@@ -40,7 +38,7 @@ def test_rows(lib, B, T):
 
 @pytest.mark.parametrize("gamma,done_p", [(1.0, 0.01), (0.0, 0.1), (-0.9, 0.01), (1.25, 0.2), (0.999, 0.0)])
 def test_split_discounts(lib, gamma, done_p):
-    """Discounts above 1 in size (whole rows only), zero, negative and slow ones."""
+    """Discounts above 1 in size, zero, negative and slow ones."""
     print(f"\n[rtg] gamma {gamma} done {done_p}", flush=True)
     inp = _case(2, 20001, gamma, done_p)
     t = tally(capi.run_op(lib, "reward_to_go", inp)["output"].cpu(), exact.reward_to_go(inp)["output"], TOL)
@@ -66,7 +64,7 @@ def test_offset_pointers(lib, B, T, off):
 
 
 def test_split_on_many_streams(lib):
-    """Ten streams at once, more than hold scratch memory: every call's result is its own."""
+    """Ten streams at once: every call's result is its own."""
     print("\n[rtg] ten streams", flush=True)
     streams = [torch.cuda.Stream() for _ in range(10)]
     args = []
@@ -85,30 +83,52 @@ def test_split_on_many_streams(lib):
         assert t["mismatched"] == 0, t
 
 
-def test_split_on_streams_that_come_and_go(lib):
-    """Twelve streams one after another, each destroyed once its call has completed."""
-    print("\n[rtg] streams that come and go", flush=True)
-    with open("/proc/self/maps") as f:
-        hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
-    inp = _case(4, 50_000)
-    a = capi.device_args("reward_to_go", inp)
-    out = a["output"] = torch.zeros(4, 50_000, device="cuda")
+# Parts of 4 chunks, up to the 256 that their outputs have room for, of 16 and of more; last
+# parts of one step and whole ones, unaligned rows.
+PART_SHAPES = [(1, 12289), (2, 12544), (5, 20480), (2, 28673), (16, 65536), (1, 262144), (1, 262145), (3, 261889),
+               (40, 28673), (256, 12290), (3, 1 << 20), (1, (1 << 22) + 257), (1, 9_000_001), (250, 300_001)]
+
+
+@pytest.mark.parametrize("B,T", PART_SHAPES)
+@pytest.mark.parametrize("gamma", [0.99, -1.0])
+def test_split_rows_against_whole_rows(lib, B, T, gamma):
+    """An output on top of the rewards takes the whole-row form: the same values within the
+    task's bound, and every element written."""
+    print(f"\n[rtg] parts B{B} T{T} gamma {gamma}", flush=True)
+    g = torch.Generator("cuda").manual_seed(B + T)
+    r = torch.rand(B, T, device="cuda", generator=g) * 2 - 1
+    d = torch.rand(B, T, device="cuda", generator=g) < 2e-4
+    out = torch.full((B, T), float("nan"), device="cuda")
+    a = dict(reward=r, done=d, gamma=gamma, B=B, T=T, output=out)
+    capi.call(lib, "reward_to_go", a)
+    capi.call(lib, "reward_to_go", dict(a, output=r))
     torch.cuda.synchronize()
-    want = exact.reward_to_go(inp)["output"]
-    for _ in range(12):
-        s = ctypes.c_void_p()
-        assert hip.hipStreamCreate(ctypes.byref(s)) == 0
-        out.zero_()
+    assert bool(((out - r).abs() <= 1e-5 + 1e-5 * r.abs()).all())
+
+
+@pytest.mark.parametrize("T,gamma", [(40_000, 0.99), (300_000, 0.9), (2_000_000, 0.9)])
+def test_split_rows_with_infinities(lib, T, gamma):
+    """An infinite or NaN reward reaches the same outputs split or not, also past the steps
+    after which the discount is too small for a double."""
+    print(f"\n[rtg] infinities T{T}", flush=True)
+    for v in (float("inf"), float("nan")):
+        r = torch.rand(2, T, device="cuda")
+        r[0, T - 9] = v
+        r[1, 77] = v
+        d = torch.rand(2, T, device="cuda") < 1e-4
+        d[0] = False
+        out = torch.zeros(2, T, device="cuda")
+        a = dict(reward=r, done=d, gamma=gamma, B=2, T=T, output=out)
+        capi.call(lib, "reward_to_go", a)
+        capi.call(lib, "reward_to_go", dict(a, output=r))
         torch.cuda.synchronize()
-        for _ in range(2):
-            capi.call(lib, "reward_to_go", a, s.value)
-        assert hip.hipStreamSynchronize(s) == 0
-        assert hip.hipStreamDestroy(s) == 0
-        assert tally(out.cpu(), want, TOL)["mismatched"] == 0
+        assert bool((out[0, :T - 8] == v).all()) or bool(out[0, :T - 8].isnan().all() and v != v)
+        assert torch.equal(out.isnan(), r.isnan())
+        assert torch.allclose(out, r, rtol=1e-5, atol=1e-5, equal_nan=True)
 
 
 def test_split_under_capture(lib):
-    """A captured call takes the whole-row form, which holds no scratch memory, and replays."""
+    """A captured call replays on new values with the bits of an eager one."""
     print("\n[rtg] capture", flush=True)
     inp = _case(3, 30_000)
     a = capi.device_args("reward_to_go", inp)
@@ -125,3 +145,4 @@ def test_split_under_capture(lib):
         torch.cuda.synchronize()
         t = tally(out.cpu(), exact.reward_to_go(new)["output"], TOL)
         assert t["mismatched"] == 0, t
+        assert torch.equal(out, capi.run_op(lib, "reward_to_go", new)["output"])
