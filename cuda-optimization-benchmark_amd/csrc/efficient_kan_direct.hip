@@ -56,7 +56,7 @@ hipError_t launch(const float* x, const float* grid, const float* wb, const floa
   const int mtiles = plan.mtiles, ctiles = plan.ctiles;
   const int64_t tiles = (int64_t)mtiles * ctiles;
   const size_t per_split = (size_t)tiles * 16 * kR * kCols * sizeof(float);
-  int nsplit = plan.nsplit;
+  const int nsplit = plan.nsplit;
   unsigned* counters = nullptr;
   float* partial = nullptr;
   std::optional<StreamScratch> scratch;
@@ -65,18 +65,15 @@ hipError_t launch(const float* x, const float* grid, const float* wb, const floa
     size_t have = 0;
     const hipError_t e = workspace_if_possible(kSlotKan, std::max(shared_bytes, nsplit * per_split), stream, &p, &have);
     if (e != hipSuccess) return e;
-    nsplit = (int)std::min<size_t>(nsplit, std::max<size_t>(have / per_split, 1));
-    partial = static_cast<float*>(p);
+    if (have >= nsplit * per_split) partial = static_cast<float*>(p);
   } else if (nsplit > 1) {
     scratch.emplace(nsplit * per_split, stream);
     counters = scratch->counters;
     partial = static_cast<float*>(scratch->ptr);
   }
-  if (partial == nullptr) nsplit = 1;
-  plan.split(nsplit);
-  nsplit = plan.nsplit;
-  if (nsplit > kMaxArrivals || tiles > kScratchCounters) counters = nullptr;
-  const int64_t pairs = (int64_t)ctiles * nsplit, span = std::min<int64_t>(8, pairs), padded = (pairs + span - 1) / span * span;
+  const int shares = partial != nullptr ? nsplit : 1;  // workgroups of one tile
+  if (shares > kMaxArrivals || tiles > kScratchCounters) counters = nullptr;
+  const int64_t pairs = (int64_t)ctiles * shares, span = std::min<int64_t>(8, pairs), padded = (pairs + span - 1) / span * span;
   auto enqueue = [&](bool last, auto kernel, dim3 groups, size_t lds, auto... args) {
     const hipEvent_t done = last && scratch && scratch->ptr != nullptr ? scratch->done : nullptr;
     if (done != nullptr)
@@ -87,9 +84,10 @@ hipError_t launch(const float* x, const float* grid, const float* wb, const floa
     if (done != nullptr && e == hipSuccess) scratch->ended();
     return e;
   };
-  const bool one = nsplit == 1 || counters != nullptr;
-  const hipError_t e = enqueue(one, kan_direct::kan_direct<kNQ, kR>, dim3((unsigned)(padded * mtiles)), plan.lds, x, grid,
-                               wb, ws, sc, order, L, C, B, I, O, mtiles, ctiles, nsplit, plan.cper, partial, counters, out);
+  const bool one = shares == 1 || counters != nullptr;
+  auto kernel = shares < nsplit ? kan_direct::kan_direct<kNQ, kR, true> : kan_direct::kan_direct<kNQ, kR, false>;
+  const hipError_t e = enqueue(one, kernel, dim3((unsigned)(padded * mtiles)), plan.lds, x, grid, wb, ws, sc, order, L, C, B,
+                               I, O, mtiles, ctiles, nsplit, plan.cper, partial, counters, out);
   if (e != hipSuccess || one) return e;
   return enqueue(true, kan_direct_sum<kR>, dim3((unsigned)(tiles * 4 * kR)), (size_t)0,
                  static_cast<const float*>(partial), B, O, mtiles, ctiles, nsplit, out);
@@ -110,7 +108,7 @@ hipError_t launch_rows(const float* x, const float* grid, const float* wb, const
 // Orders 1 .. 4 (the triangular scheme's instantiations), four or more bases (a feature's
 // bases are read 16 bytes at a time), 32-bit offsets for one workgroup's rows and columns,
 // and a grid one launch covers (2^32 - 1 work-items; the split never takes the grid past
-// three workgroups per CU).
+// four workgroups per CU).
 bool kan_direct_fits(int order, int C, int B, int I, int O) {
   const int64_t lim = 0x7fffffff;
   if (order < 1 || order > 4 || C < 4 || I < 1) return false;
@@ -141,8 +139,8 @@ double kan_direct_us(int C, int B, int I, int O) {
 }
 
 // shared_bytes: 0 for calls with no workspace of their own (the splits' sums then go to the
-// stream's scratch memory, and stay unsplit where there is none); else the size to which the
-// shared workspace is grown, which holds them.  The arrival counters are the scratch memory's
+// stream's scratch memory); else the size to which the shared workspace is grown, which holds
+// them.  Where there is no room a tile's one workgroup takes all splits, with the same bits.  The arrival counters are the scratch memory's
 // alone: two streams' calls at once could leave shared ones wrong for every later call.
 hipError_t kan_direct_launch(const float* x, const float* grid, const float* wb, const float* ws, const float* sc,
                              int order, int L, int C, int B, int I, int O, float* out, size_t shared_bytes,

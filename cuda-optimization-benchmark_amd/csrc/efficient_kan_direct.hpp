@@ -148,9 +148,13 @@ __device__ __forceinline__ void write_bases(float x, const float* kn, int L, int
 // kNQ: 16-byte groups of a feature's C bases, 4 (kNQ - 1) < C <= 4 kNQ.  The last group is
 // read at C - 4, inside the feature's own floats, so its first 4 kNQ - C ("dup") elements
 // repeat the group before it: they have no slot and no MFMA.  kR: row blocks of 16.
-// nsplit > 1: partial holds a tile of sums per (split, row tile, column tile), counters (or
-// null) one arrival counter per tile, zero between launches.
-template <int kNQ, int kR>
+// nsplit > 1: the features' sums are taken in nsplit parts and added in order.  partial: a tile
+// of sums per (split, row tile, column tile), a workgroup per part; counters: null or one
+// arrival counter per tile, zero between launches.  kAlone, for calls without that memory: a
+// tile's one workgroup takes the parts one after another and keeps their sum in `out`, in the
+// same order, so the same bits.  (The loop around the parts costs 27 registers and with them a
+// quarter of the waves, so it is a form of its own.)
+template <int kNQ, int kR, bool kAlone>
 __global__ __launch_bounds__(kThreads) void kan_direct(
     const float* __restrict__ x, const float* __restrict__ grid, const float* __restrict__ wb,
     const float* __restrict__ ws, const float* __restrict__ sc, int order, int L, int C, int B, int I, int O,
@@ -170,13 +174,15 @@ __global__ __launch_bounds__(kThreads) void kan_direct(
 
   // The row tiles of one (column tile, split) read the same weights: they go to one XCD
   // (workgroups are dispatched round-robin over 8) one after another, and share its L2.
-  const int span = min(8, ctiles * nsplit), seq = (int)blockIdx.x / span;
+  const int shares = kAlone ? 1 : nsplit;  // workgroups of one tile
+  const int span = min(8, ctiles * shares), seq = (int)blockIdx.x / span;
   const int pair = seq / mtiles * span + (int)blockIdx.x % span, mt = seq % mtiles;
-  if (pair >= ctiles * nsplit) return;
-  const int ct = pair % ctiles, split = pair / ctiles;
+  if (pair >= ctiles * shares) return;
+  const int ct = pair % ctiles;
+  int split = pair / ctiles;
   const int m0 = mt * kRows, n0 = ct * kCols;
   const int nchunks = (I + kFeat - 1) / kFeat;
-  const int c0 = split * cper, c1 = min(nchunks, c0 + cper);
+  int c0, c1;
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
 
   // This lane's column and feature quarter of the MFMA operands.
@@ -315,8 +321,6 @@ __global__ __launch_bounds__(kThreads) void kan_direct(
   };
 
   f32x4 acc[kR];
-#pragma unroll
-  for (int r = 0; r < kR; ++r) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // Step s of chunk c: the lane's weights scaled into their own registers (direct: the raw
   // ones reload for chunk c + 1), then 1 + C MFMAs per row block.
@@ -362,40 +366,60 @@ __global__ __launch_bounds__(kThreads) void kan_direct(
     for (int r = 0; r < kR; ++r) acc[r] += part[r];
   };
 
-  // The activations' loads go out before the weights', whose arrival nothing before the first
-  // MFMA waits for (loads return in order).
-  load_knots(c0);
-  float xv = load_x(c0);
-  const float x1 = load_x(c0 + 1);
-  write_knots(0);
-  load_knots(c0 + 1);
-  if constexpr (kFlat) {
-    load_flat(c0);
-  } else {
+  for (;;) {
+    c0 = split * cper;
+    c1 = min(nchunks, c0 + cper);
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) load_step(c0, s);
-  }
-  barrier_no_vm_drain();
-  expand(c0, xv);
-  write_knots(1);
-  xv = x1;
-  load_knots(c0 + 2);
-  for (int c = c0; c < c1; ++c) {
-    // Chunk c's runs and chunk c + 1's knots are written; every wave is done with the stage
-    // chunk c + 1 expands into and with chunk c's knots.
+    for (int r = 0; r < kR; ++r) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // The activations' loads go out before the weights', whose arrival nothing before the first
+    // MFMA waits for (loads return in order).
+    load_knots(c0);
+    float xv = load_x(c0);
+    const float x1 = load_x(c0 + 1);
+    write_knots(0);
+    load_knots(c0 + 1);
+    if constexpr (kFlat) {
+      load_flat(c0);
+    } else {
+#pragma unroll
+      for (int s = 0; s < kSteps; ++s) load_step(c0, s);
+    }
     barrier_no_vm_drain();
-    if (c + 1 < c1) {
-      expand(c + 1, xv);
-      write_knots((c - c0) & 1);
-      xv = load_x(c + 2);
-      load_knots(c + 3);
-    }
-    if constexpr (kFlat) {  // the wave's own LDS: its reads of the last chunk came before
-      stage_flat();
-      load_flat(c + 1);
-    }
+    expand(c0, xv);
+    write_knots(1);
+    xv = x1;
+    load_knots(c0 + 2);
+    for (int c = c0; c < c1; ++c) {
+      // Chunk c's runs and chunk c + 1's knots are written; every wave is done with the stage
+      // chunk c + 1 expands into and with chunk c's knots.
+      barrier_no_vm_drain();
+      if (c + 1 < c1) {
+        expand(c + 1, xv);
+        write_knots((c - c0) & 1);
+        xv = load_x(c + 2);
+        load_knots(c + 3);
+      }
+      if constexpr (kFlat) {  // the wave's own LDS: its reads of the last chunk came before
+        stage_flat();
+        load_flat(c + 1);
+      }
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) step(c, s);
+      for (int s = 0; s < kSteps; ++s) step(c, s);
+    }
+    if constexpr (!kAlone) break;
+    // This part's sum on top of the parts' before it.
+    if (col < O) {
+#pragma unroll
+      for (int r = 0; r < kR; ++r)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int row = m0 + 16 * r + 4 * fq + e;
+          float* at = out + (size_t)row * O + col;
+          if (row < B) *at = (split > 0 ? *at : 0.f) + acc[r][e];
+        }
+    }
+    if (++split == nsplit) return;
+    __syncthreads();  // the stages are free
   }
 
   if (nsplit > 1) {

@@ -81,12 +81,13 @@ import __graft_entry__; __graft_entry__.load_package()
 import torch
 from cob_amd import capi, inputs
 lib = capi.load()
-inp = inputs.make_inputs("efficient_kan", dict(name="c", seed=3, B=100, I=64, O=96, grid_size=7, spline_order=2))
+B, I, O, G, K = {shape}
+inp = inputs.make_inputs("efficient_kan", dict(name="c", seed=3, B=B, I=I, O=O, grid_size=G, spline_order=K))
 args = capi.device_args("efficient_kan", inp)
-out = args["out"] = torch.zeros(100, 96, device="cuda")
+out = args["out"] = torch.zeros(B, O, device="cuda")
 g = torch.cuda.CUDAGraph()
 with torch.cuda.graph(g):
-    capi.call(lib, "efficient_kan", args)   # the process's first call: nothing to split with
+    capi.call(lib, "efficient_kan", args)   # the process's first call: no memory to split with
 got = []
 for _ in range(3):
     out.zero_()
@@ -96,7 +97,7 @@ for _ in range(3):
 capi.call(lib, "efficient_kan", args)       # eager: allocates, splits
 torch.cuda.synchronize()
 assert all(torch.equal(t, got[0]) for t in got)
-assert torch.allclose(got[0], out, rtol=1e-5, atol=1e-5)
+assert torch.equal(got[0], out)
 g.replay()
 torch.cuda.synchronize()
 assert torch.equal(out, got[0])
@@ -104,11 +105,16 @@ print("captured")
 """
 
 
-def test_direct_first_call_in_a_capture(lib):
-    """A capture may allocate nothing: the path then runs unsplit, in a process of its own
-    where no earlier call has grown the workspace."""
-    print("\n[kan_direct] first call under capture", flush=True)
-    r = subprocess.run([sys.executable, "-c", CAPTURE.format(root=str(ROOT))], capture_output=True, text=True, timeout=110)
+# Other spline orders and finer knots (one, two and four row blocks; few splits and many), and
+# small batches of a shape that the packed path also takes.
+@pytest.mark.parametrize("shape", [(100, 64, 96, 7, 2), (16, 100, 70, 12, 3), (32, 333, 130, 20, 3), (9, 50, 33, 1, 4),
+                                   (8, 256, 256, 5, 3), (130, 96, 100, 8, 3)])
+def test_direct_first_call_in_a_capture(lib, shape):
+    """A capture may allocate nothing: a tile's one workgroup then takes all splits, in a process
+    of its own where no earlier call has grown the memory, and gives the eager call's bits."""
+    print(f"\n[kan_direct] first call under capture {shape}", flush=True)
+    r = subprocess.run([sys.executable, "-c", CAPTURE.format(root=str(ROOT), shape=shape)], capture_output=True, text=True,
+                       timeout=110)
     assert r.returncode == 0 and "captured" in r.stdout, (r.stdout[-500:], r.stderr[-2000:])
 
 
@@ -145,6 +151,7 @@ def test_direct_on_many_streams(lib):
             capi.call(lib, "efficient_kan", a, s.cuda_stream)
     torch.cuda.synchronize()
     for inp, a in args:
+        assert torch.equal(a["out"], capi.run_op(lib, "efficient_kan", inp)["out"])
         t = tally(a["out"].cpu().numpy(), exact.efficient_kan(inp)["out"], tasks.load_task("efficient_kan")["tolerance"])
         assert t["mismatched"] == 0, t
 
