@@ -185,3 +185,18 @@ def test_direct_on_streams_that_come_and_go(lib):
         for a, want in cases:
             t = tally(a["out"].cpu().numpy(), want, tasks.load_task("efficient_kan")["tolerance"])
             assert t["mismatched"] == 0, (k, t)
+
+
+def test_small_batch_with_repeated_knots(lib):
+    """The packed path leaves out an empty interval's terms; a small batch of its shape, which
+    takes the direct path, gives the same values as the packed path's rows."""
+    print("\n[kan_direct] repeated knots of a packed shape", flush=True)
+    inp = inputs.make_inputs("efficient_kan", dict(name="d", seed=6, B=4096, I=70, O=300, grid_size=5, spline_order=3))
+    inp["grid"] = inp["grid"].clone()
+    inp["grid"][:, :4] = inp["grid"][:, 3:4]    # clamped ends
+    inp["grid"][:, -4:] = inp["grid"][:, -4:-3]
+    packed = capi.run_op(lib, "efficient_kan", inp)["out"].cpu().numpy()
+    few = dict(inp, x=inp["x"][:9].contiguous(), B=9)
+    got = capi.run_op(lib, "efficient_kan", few)["out"].cpu().numpy()
+    t = tally(got, packed[:9].astype(np.float64), tasks.load_task("efficient_kan")["tolerance"])
+    assert t["mismatched"] == 0 and np.isfinite(got).all(), t
