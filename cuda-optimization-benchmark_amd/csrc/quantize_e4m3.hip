@@ -29,9 +29,10 @@
 // through a grid barrier, and each converts the chunks it holds, so x is read once.  The
 // barrier is a plain launch sized by the occupancy API (a cooperative launch, which guarantees
 // residency, costs about 100 us per launch on this stack).  Residency is not guaranteed
-// (another stream's kernels can hold CUs), so the wait is bounded: a workgroup that times out
-// reads all of x for the max itself.  The max is exact and order-free, so both paths give
-// identical bits, every wave exits, and no result depends on the timing.
+// (another stream's kernels can hold CUs), so the wait is bounded: workgroups that have waited
+// long enough find the max of x among themselves (qz_grid_max), or in the end each by itself.  The
+// max is exact and order-free, so all ways give identical bits, every wave exits, and no
+// result depends on the timing.
 #include "common.hpp"
 
 namespace taskops {
@@ -244,11 +245,35 @@ __global__ __launch_bounds__(kThreads) void qz_cast_any(const float* __restrict_
 // and a captured graph replays correctly.
 constexpr int kQzGroups = 16;
 constexpr int kQzLine = 16;  // unsigned per 64-byte line
-enum QzWord : int { kQzGroupCount = 0, kQzGroupMax = kQzGroups, kQzTopCount = 2 * kQzGroups, kQzSetWords };
+//
+// A workgroup that has polled kQzPatience times assumes that others wait for CUs that it may be
+// holding, and helps: the workgroups that run share out pieces of x among themselves, each takes
+// the next one (kQzHelpNext), folds its max into kQzHelpMax and counts it done (kQzHelpDone).
+// When all are done the max of x is known without the workgroups that have not started; those
+// find it so when they have arrived.  x is read once more by whoever runs, and no one waits for
+// work that is not running: a piece's workgroup computes it without waiting for anything.
+enum QzWord : int {
+  kQzGroupCount = 0,
+  kQzGroupMax = kQzGroups,
+  kQzTopCount = 2 * kQzGroups,
+  kQzHelpNext,
+  kQzHelpDone,
+  kQzHelpMax,
+  kQzSetWords
+};
 constexpr int kQzParity = 2 * kQzSetWords;  // after both sets
 constexpr int kQzWords = kQzParity + 1;
 static_assert(kQzSetWords <= kWave, "the grid's last arrival clears a set with one store per lane of a wave");
-constexpr unsigned kQzSpinDefault = 1u << 14;  // polls of the parity (~0.5-1 us each) before the fallback
+constexpr int64_t kQzPiece = 4 * kChunk;  // elements
+// Polls (0.5 to 1 us each) before a workgroup helps, more for larger tensors, whose workgroups
+// arrive further apart, and for the last helpers' pieces, after which it finds the max by itself.
+// With a stream of elementwise kernels holding the CUs 16.8 M elements took 9 ms when each
+// workgroup that gave up, after 2^14 polls, read all of x, and 0.25 helping; 33.5 M, 67 M and 134 M,
+// whose workgroups all found room in time, 0.26, 0.31 and 0.42 ms then and 0.31, 0.34 and 0.45 now.
+constexpr unsigned kQzPatience = 128, kQzHelpWait = 1u << 14;
+struct QzLimits {
+  unsigned patience, help_wait;
+};
 
 __device__ __forceinline__ unsigned* qz_word(unsigned* bar, unsigned set, int w, int i = 0) {
   return bar + ((int)set * kQzSetWords + w + i) * kQzLine;
@@ -270,15 +295,47 @@ __device__ __forceinline__ unsigned qz_add(unsigned* p) {
 // The barrier's words in LDS.
 struct QzShared {
   unsigned lds[kThreads / kWave];
-  unsigned gmax, fallback;
+  unsigned gmax, piece, parity;
+  bool done;
 };
+
+// Lane 0 of wave 0: polls until the barrier is complete (1) or the helpers have all of x (2), at
+// most `polls` times (0: neither).
+__device__ __forceinline__ int qz_poll(unsigned* bar, unsigned parity, unsigned pieces, unsigned polls) {
+  const unsigned set = parity & 1u;
+  for (unsigned i = 0; i < polls; ++i) {
+    const unsigned now = qz_load(qz_parity(bar)), helped = qz_load(qz_word(bar, set, kQzHelpDone));
+    if (now != parity) return 1;
+    if (helped == pieces) return 2;
+    __builtin_amdgcn_s_sleep(2);
+  }
+  return 0;
+}
+
+// Wave 0: polls, and leaves in LDS whether the max bits of x are known, and them.
+__device__ __forceinline__ void qz_settle(unsigned* bar, unsigned parity, unsigned pieces, unsigned polls, QzShared* sh) {
+  const unsigned set = parity & 1u, lane = threadIdx.x;
+  const unsigned groups = gridDim.x < kQzGroups ? gridDim.x : kQzGroups;
+  int how = 0;
+  if (lane == 0) how = qz_poll(bar, parity, pieces, polls);
+  how = __builtin_amdgcn_readfirstlane(how);
+  unsigned gm = 0u;
+  if (how == 1) gm = wave_max_u32(lane < groups ? qz_load(qz_word(bar, set, kQzGroupMax, (int)lane)) : 0u);
+  if (how == 2) gm = qz_load(qz_word(bar, set, kQzHelpMax));
+  if (lane == 0) {
+    sh->done = how != 0;
+    sh->gmax = gm;
+    sh->parity = parity;
+  }
+}
 
 // The max bits of all of x, from this workgroup's `m` (called by every thread; parity: thread
 // 0's read of the parity word).  Thread 0 of each workgroup runs the barrier; every RMW's
 // returned value is used before the next one is issued, which orders them at the coherence
 // point.
-__device__ __forceinline__ unsigned qz_grid_max(unsigned m, unsigned parity, unsigned* bar, unsigned spin_limit,
+__device__ __forceinline__ unsigned qz_grid_max(unsigned m, unsigned parity, unsigned* bar, QzLimits limits,
                                                 const float* __restrict__ x, int64_t n, QzShared* sh) {
+  const unsigned pieces = (unsigned)((n + kQzPiece - 1) / kQzPiece);
   m = block_max_u32(m, sh->lds);
   if (threadIdx.x < kWave) {  // wave 0 runs the barrier; lane 0 makes the RMWs
     const int lane = threadIdx.x;
@@ -298,37 +355,46 @@ __device__ __forceinline__ unsigned qz_grid_max(unsigned m, unsigned parity, uns
       if (lane < kQzSetWords) qz_store(qz_word(bar, set ^ 1u, 0, lane), 0u);
       if (lane == 0) qz_store(qz_parity(bar), parity ^ 1u);
     }
-    bool done = false;
-    if (lane == 0) {
-      for (unsigned i = 0; i < spin_limit; ++i) {
-        if (qz_load(qz_parity(bar)) != parity) {
-          done = true;
-          break;
-        }
-        __builtin_amdgcn_s_sleep(2);
-      }
-    }
-    done = __builtin_amdgcn_ballot_w64(done) != 0ull;
-    unsigned gm = 0u;
-    if (done) gm = wave_max_u32((unsigned)lane < groups ? qz_load(qz_word(bar, set, kQzGroupMax, lane)) : 0u);
-    if (lane == 0) {
-      sh->fallback = done ? 0u : 1u;
-      sh->gmax = gm;
-    }
+    qz_settle(bar, parity, pieces, limits.patience, sh);
   }
   __syncthreads();
-  unsigned gm = sh->gmax;
-  if (sh->fallback) {  // the barrier did not complete in time: this workgroup finds the max itself
-    unsigned mm = 0u;    // (one 16-byte load at a time: the held chunks stay in registers)
-    const int64_t n4 = n & ~(int64_t)3;
-    for (int64_t i = 4 * (int64_t)threadIdx.x; i < n4; i += 4 * kThreads) {
-      const f32x4 w = *reinterpret_cast<const f32x4*>(x + i);
-      mm = max(max(mm, max(abs_bits(w.x), abs_bits(w.y))), max(abs_bits(w.z), abs_bits(w.w)));
+  if (sh->done) return sh->gmax;
+
+  // Help; in the end, alone, piece after piece.  One 16-byte load at a time and every uniform
+  // value in scalar registers: the held chunks stay in registers.
+  const unsigned par = (unsigned)__builtin_amdgcn_readfirstlane((int)sh->parity), set = par & 1u;
+  bool alone = false;
+  unsigned next = 0u, all = 0u;
+  for (;;) {
+    if (threadIdx.x == 0 && !alone)
+      sh->piece = qz_load(qz_parity(bar)) != par ? pieces : qz_add(qz_word(bar, set, kQzHelpNext));
+    __syncthreads();
+    const unsigned piece = alone ? next++ : (unsigned)__builtin_amdgcn_readfirstlane((int)sh->piece);
+    if (piece < pieces) {
+      const int64_t from = (int64_t)piece * kQzPiece;
+      const int len = (int)(n - from < kQzPiece ? n - from : kQzPiece);
+      unsigned mm = 0u;
+      for (int i = 4 * (int)threadIdx.x; i < (len & ~3); i += 4 * kThreads) {
+        const f32x4 w = *reinterpret_cast<const f32x4*>(x + from + i);
+        mm = max(max(mm, max(abs_bits(w.x), abs_bits(w.y))), max(abs_bits(w.z), abs_bits(w.w)));
+      }
+      if ((int)threadIdx.x < (len & 3)) mm = max(mm, abs_bits(x[from + (len & ~3) + threadIdx.x]));
+      all = max(all, (unsigned)__builtin_amdgcn_readfirstlane((int)block_max_u32(mm, sh->lds)));
+      if (threadIdx.x == 0 && !alone) {
+        const unsigned r = qz_max(qz_word(bar, set, kQzHelpMax), all);
+        asm volatile("" ::"v"(r));
+        const unsigned d = qz_add(qz_word(bar, set, kQzHelpDone));
+        asm volatile("" ::"v"(d));
+      }
+      continue;
     }
-    if ((int64_t)threadIdx.x < n - n4) mm = max(mm, abs_bits(x[n4 + threadIdx.x]));
-    gm = block_max_u32(mm, sh->lds);
+    if (alone) return all;
+    if (threadIdx.x < kWave) qz_settle(bar, par, pieces, limits.help_wait, sh);
+    __syncthreads();
+    if (sh->done) return sh->gmax;
+    alone = true;
+    all = 0u;
   }
-  return gm;
 }
 
 // Requires x 16-byte and q 4-byte aligned and gridDim.x = ceil(n / kChunk).  8 waves per SIMD
@@ -336,7 +402,7 @@ __device__ __forceinline__ unsigned qz_grid_max(unsigned m, unsigned parity, uns
 // operand's chunks.
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) void qz_fused(
     const float* __restrict__ x, int64_t n, uint8_t* __restrict__ q, float* __restrict__ scale_out,
-    unsigned* __restrict__ bar, unsigned spin_limit) {
+    unsigned* __restrict__ bar, QzLimits limits) {
   __shared__ QzShared sh;
   const int64_t base = (int64_t)blockIdx.x * kChunk;
   f32x4 v[kVecs];
@@ -345,7 +411,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) v
   // workgroup arrives.
   unsigned parity = 0u;
   if (threadIdx.x == 0) parity = qz_load(qz_parity(bar));
-  const float scale = scale_from(qz_grid_max(chunk_max(v, 0u), parity, bar, spin_limit, x, n, &sh));
+  const float scale = scale_from(qz_grid_max(chunk_max(v, 0u), parity, bar, limits, x, n, &sh));
   if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = scale;
   store_chunk(q, n, base, v, scale);
 }
@@ -369,7 +435,7 @@ __device__ __forceinline__ void finish_loads(unsigned& m) {  // nothing loaded l
 }
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void qz_hold(
     const float* __restrict__ x, int64_t n, uint8_t* __restrict__ q, float* __restrict__ scale_out,
-    unsigned* __restrict__ bar, unsigned spin_limit) {
+    unsigned* __restrict__ bar, QzLimits limits) {
   __shared__ QzShared sh;
   extern __shared__ __attribute__((aligned(16))) f32x4 held[];  // [kVecs][kThreads]
   const int64_t stride = (int64_t)gridDim.x * kChunk, first = (int64_t)blockIdx.x * kChunk;
@@ -410,7 +476,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
   }
   unsigned parity = 0u;
   if (threadIdx.x == 0) parity = qz_load(qz_parity(bar));
-  const float scale = scale_from(qz_grid_max(m, parity, bar, spin_limit, x, n, &sh));
+  const float scale = scale_from(qz_grid_max(m, parity, bar, limits, x, n, &sh));
   if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = scale;
 #pragma unroll
   for (int c = 0; c < kHeldRegs; ++c) {
@@ -439,7 +505,12 @@ constexpr size_t kHeldLds = (size_t)kChunk * sizeof(float);
 constexpr int kHoldMost = 16;
 
 
-unsigned g_qz_spin_limit = kQzSpinDefault;
+QzLimits g_qz_limits = {kQzPatience, kQzHelpWait};
+QzLimits limits_for(int64_t n) {
+  QzLimits l = g_qz_limits;
+  if (l.patience > 0) l.patience += (unsigned)(n / (2 * kQzPiece));
+  return l;
+}
 int g_qz_capacity[2][64];  // resident qz_fused, qz_hold workgroups per device (0: not yet known, -1: none)
 
 int resident(int which, const void* kernel, size_t lds) {
@@ -488,13 +559,13 @@ extern "C" hipError_t taskops_quantize_e4m3(const float* x, int64_t n, uint8_t* 
   const int64_t chunks = (n + kChunk - 1) / kChunk;
   if (vx && vq && chunks <= fused_capacity()) {
     hipLaunchKernelGGL(qz_fused, dim3((unsigned)chunks), dim3(kThreads), 0, stream, x, n, q, scale,
-                       partial + kMaxPartials, g_qz_spin_limit);
+                       partial + kMaxPartials, limits_for(n));
     return hipGetLastError();
   }
   const int hold = vx && vq ? hold_capacity() : 0;
   if (hold > 0 && chunks <= (int64_t)kHoldMost * hold) {
     hipLaunchKernelGGL(qz_hold, dim3((unsigned)(chunks < hold ? chunks : hold)), dim3(kThreads), kHeldLds, stream, x, n, q,
-                       scale, partial + kMaxPartials, g_qz_spin_limit);
+                       scale, partial + kMaxPartials, limits_for(n));
     return hipGetLastError();
   }
   if (vx && vq) {
@@ -517,7 +588,8 @@ extern "C" hipError_t taskops_quantize_e4m3(const float* x, int64_t n, uint8_t* 
   return hipGetLastError();
 }
 
-// Test hook: the polls of the fused kernel's bounded wait before a workgroup falls back to
-// finding the max itself (0 sends every workgroup to the fallback).  Not thread-safe; for
-// tests that check both paths give the same bits.
-extern "C" void taskops_testing_quantize_spin_limit(unsigned polls) { g_qz_spin_limit = polls; }
+// Test hooks: the polls after which a workgroup helps (0 makes every workgroup help), and those
+// for the last helpers' pieces (0, with the first at 0 too, makes workgroups find the max
+// themselves).  Not thread-safe; for tests that check that all ways give the same bits.
+extern "C" void taskops_testing_quantize_spin_limit(unsigned polls) { g_qz_limits.patience = polls; }
+extern "C" void taskops_testing_quantize_help_limit(unsigned polls) { g_qz_limits.help_wait = polls; }

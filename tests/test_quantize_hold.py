@@ -88,3 +88,60 @@ def test_graph_replay(lib):
         torch.cuda.synchronize()
         qw, sw = _want(x)
         assert s[0] == sw and torch.equal(q, qw)
+
+
+@pytest.mark.parametrize("n", [3, 16385, 5 * CHUNK + 1, 1024 * CHUNK, 1100 * CHUNK + 9, 2100 * CHUNK + 2, 4096 * CHUNK + 1])
+def test_helping_and_alone(lib, n):
+    """With no polls allowed the workgroups share out x among themselves; with none for the last
+    pieces either, each may end up finding the max by itself.  Same bits, launch after launch,
+    as the barrier's, with the largest magnitude in turn in the first and the last element."""
+    print(f"\n[quantize] helping n={n}", flush=True)
+    x = torch.randn(n, device="cuda", generator=torch.Generator("cuda").manual_seed(4))
+    spin, wait = lib.taskops_testing_quantize_spin_limit, lib.taskops_testing_quantize_help_limit
+    spin.argtypes = wait.argtypes = [ctypes.c_uint]
+    try:
+        for limits in [(0, 1 << 14), (0, 0), (1, 1 << 14), (0, 1 << 14)]:
+            spin(limits[0])
+            wait(limits[1])
+            for at in (0, n - 1):
+                x[at] = 9.0 + at % 3
+                for _ in range(2):
+                    q, s = _run(lib, x, n)
+                    qw, sw = _want(x)
+                    assert s == sw and torch.equal(q, qw), (limits, at)
+                x[at] = 0.5
+    finally:
+        spin(128)
+        wait(1 << 14)
+    q, s = _run(lib, x, n)
+    qw, sw = _want(x)
+    assert s == sw and torch.equal(q, qw)
+
+
+def test_beside_work_that_holds_the_chip(lib):
+    """Elementwise kernels on another stream hold the CUs while tensors of every route are
+    quantised: right codes, and no wait for a workgroup that is not running (16.8 M elements took
+    9 ms when each waiting workgroup gave up on its own)."""
+    print("\n[quantize] beside other work", flush=True)
+    big = torch.randn(1 << 28, device="cuda")
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    for n in (1 << 24, 1 << 25, 1 << 26):
+        x = torch.randn(n, device="cuda")
+        qw, sw = _want(x)
+        q = torch.zeros(n, dtype=torch.uint8, device="cuda")
+        s = torch.zeros(1, device="cuda")
+        torch.cuda.synchronize()
+        took = []
+        for _ in range(3):
+            with torch.cuda.stream(s2):
+                for _ in range(6):
+                    big.mul_(1.0001)
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record(s1)
+            capi.call(lib, "quantize_e4m3", dict(x=x, n=n, q=q, scale=s), s1.cuda_stream)
+            b.record(s1)
+            torch.cuda.synchronize()
+            took.append(a.elapsed_time(b))
+            assert s[0] == sw and torch.equal(q, qw)
+        print(f"[quantize] n={n} {min(took):.3f} ms", flush=True)
+        assert min(took) < 5.0
