@@ -1,4 +1,6 @@
 // Launches of fp8_linear's middle kernel (fp8_linear_mid.hpp).
+#include <algorithm>
+
 #include "fp8_linear_mid.hpp"
 
 namespace taskops {
@@ -11,12 +13,19 @@ template <int kXI, int kWJ, int kStages, bool kDirect>
 hipError_t launch(const uint8_t* x, const uint8_t* w, int M, int N, int K, float inv, const uint16_t* bias,
                   uint16_t* out, hipStream_t stream) {
   using S = Shape<kXI, kWJ>;
-  const dim3 grid((unsigned)((M + S::kRows - 1) / S::kRows) * (unsigned)((N + S::kCols - 1) / S::kCols));
   const bool rows16 = N % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0 && (int64_t)S::kRows * N * 2 <= 0x7fffffff;
   auto kernel = rows16 ? mid::fp8_gemm_mid<kXI, kWJ, kStages, kDirect, 2> : mid::fp8_gemm_mid<kXI, kWJ, kStages, kDirect, 0>;
-  hipLaunchKernelGGL(kernel, grid, dim3(mid::kThreads), S::lds_bytes(kDirect ? kStages : 2), stream, x, w, M, N, K, inv,
-                     bias, out);
-  return hipGetLastError();
+  // A launch covers at most 2^32 - 1 work-items: whole rows of tiles at a time.
+  const int64_t tn = (N + S::kCols - 1) / S::kCols, most = (int64_t)0xffffffff / mid::kThreads / tn * S::kRows;
+  for (int64_t m0 = 0; m0 < M; m0 += most) {
+    const int rows = (int)std::min<int64_t>(most, M - m0);
+    const unsigned tiles = (unsigned)((rows + (int64_t)S::kRows - 1) / S::kRows * tn);
+    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(mid::kThreads), S::lds_bytes(kDirect ? kStages : 2), stream,
+                       x + m0 * K, w, rows, N, K, inv, bias, out + m0 * N);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 template <int kXI, int kWJ, int kStages>

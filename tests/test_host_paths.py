@@ -175,3 +175,11 @@ def test_the_least_recently_used_scratch_goes_first(host):
     steps = [fine(s) for s in order] + [put("busy", s, 1) for s in range(3, 11) if s not in (5, 9)]
     out = host(steps + [fine(20), fine(9), put("busy", 9, 1), put("busy", 20, 1), fine(5)])
     assert split(out[-5]) and split(out[-4]) and not split(out[-1])
+
+
+def test_fp8_more_tiles_than_one_launch_takes(host):
+    """8.75 M tiles of 128 x 128 by 512 threads (an output of 280 GB): launches of at most 2^32 - 1
+    work-items, together all of the tiles."""
+    out = host([call("fp8_linear", M=70_000_000, K=1, N=2000, scale_x=1.0, scale_w=1.0)])[0]
+    grids = [int(line.split("grid ")[1].split()[0]) for line in out["log"] if line.startswith("launch")]
+    assert out["rc"] == 0 and max(grids) * 512 < 2 ** 32 and sum(grids) == 546_875 * 16, out
