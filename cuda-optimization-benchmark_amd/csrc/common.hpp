@@ -202,6 +202,10 @@ int device_cu_count();
 // LDS bytes per compute unit of the current device (cached per device).
 int device_lds_per_cu();
 
+// Between a wave's LDS writes and its other lanes' reads of them: a wave's LDS operations run in
+// order, so only the compiler has to keep theirs.
+__device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local"); }
+
 // Workgroup barrier without __syncthreads()'s release fence: that fence waits for every
 // outstanding vector memory operation (vmcnt(0)), which would drain the copy ring at each
 // step.  Callers account for their copies with explicit vmcnt waits; LDS reads issued

@@ -400,7 +400,9 @@ __global__ __launch_bounds__(kThreads) void kan_direct(
         load_knots(c + 3);
       }
       if constexpr (kFlat) {  // the wave's own LDS: its reads of the last chunk came before
+        wave_lds_fence();
         stage_flat();
+        wave_lds_fence();
         load_flat(c + 1);
       }
 #pragma unroll

@@ -147,13 +147,16 @@ __device__ __forceinline__ void run_rows(const float* __restrict__ x, const floa
   float m = mem0[n];
   bool fired = m >= th;
 
-  // (T + 4) * N * 4 bytes fit 31 bits (the launch checks), so no row of a block wraps.
+  // (T + 4) * N * 4 bytes fit 31 bits (the launch checks), so no row of a block that is computed
+  // wraps.
   const unsigned bytes = (unsigned)T * (unsigned)N * 4u;
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), (short)0, (int)bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(spikes, (short)0, (int)bytes, 0x00020000);
   constexpr int kNT = 2;  // non-temporal
-  // Offsets of the next block's load and store, one addition per block: rows past T lie past
-  // the descriptors' end (and before the first row, by wrapping, the store of block -1).
+  // Offsets of the next block's load and store, one addition per block.  A store's rows past T
+  // lie past the descriptor's end (and so, by wrapping, does the store of block -1).  The loads run
+  // up to kRing + 1 blocks ahead: past T they read zero, or, where the offset wraps in a layer of
+  // more than 32 M neurons, some row of the input; nothing uses either.
   unsigned lat = ((unsigned)r * (unsigned)N + (unsigned)(n0 + g)) * 4u;
   const unsigned step4 = 16u * (unsigned)N;
   auto load = [&]() {
@@ -188,6 +191,9 @@ __device__ __forceinline__ void run_rows(const float* __restrict__ x, const floa
   };
   float* xin = lds;              // [2][4][64]
   float* sout = lds + 8 * kWave;  // [2][4][64]
+  // A wave's LDS operations run in order, and the compiler keeps this order because it cannot tell
+  // the addresses apart.  A fence that says so changed its schedule: N = 17000, T = 160 8.5 -> 8.4 us,
+  // but N = 800,199, T = 60 106 -> 109 and N = 2,096,640, T = 20 59 -> 61.
   auto stage_in = [&](int blk, f32x4 q, float (&xv)[4]) {
     float* st = xin + (blk & 1) * 4 * kWave;
     *reinterpret_cast<f32x4*>(st + r * kWave + g) = q;
