@@ -97,17 +97,18 @@ def test_baseline_efficient_kan_full(lib):
     print(f"[parity] worst error {worst:.4f} of the tolerance", flush=True)
 
 
-# (B, I, O, grid_size, spline_order, x_range, knots).  Order 3 with at most 16 knots per
-# feature runs the fused fp16x3 MFMA kernel (C = 4, 7, 8, 11, 12 cover both padded basis
-# widths); the others run the row-wise fp32 kernel.  Ragged B, I and O exercise every tile
-# tail; x_range > 1 puts inputs outside the knot span.  Knots: "uniform" (the task's grid:
-# the kernel's direct interval lookup), "random" (sorted random knots: the knot count),
-# "jitter" (uniform plus noise of 1e-4 h: still the direct lookup, which must agree with
-# the exact bases of the jittered knots), "mixed" (even features the task's grid, odd ones
-# jittered by 1e-4 h: the kernel then reads every row's per-interval cubics, and the even
-# rows' come from the cardinal closed form) and "mixed_edge" (even features jittered by
-# 4e-7 h, still within the 5e-7 h of the closed form, so its cubics meet knots that are
-# not exactly uniform).
+# (B, I, O, grid_size, spline_order, x_range, knots), by the path that takes them at 256 CUs;
+# test_host_paths.py pins that.  Ragged B, I and O exercise every tile tail; x_range > 1 puts
+# inputs outside the knot span.  Knots: "uniform" (the task's grid: the packed path's direct
+# interval lookup), "random" (sorted random knots: the knot count), "jitter" (uniform plus noise
+# of 1e-4 h: still the direct lookup, which must agree with the exact bases of the jittered
+# knots), "mixed" (even features the task's grid, odd ones jittered by 1e-4 h: the kernel then
+# reads every row's per-interval cubics, and the even rows' come from the cardinal closed form)
+# and "mixed_edge" (even features jittered by 4e-7 h, still within the 5e-7 h of the closed
+# form, so its cubics meet knots that are not exactly uniform).
+#
+# kan_direct: small batches, other spline orders and finer knots, batches of more rows than a
+# grid's y dimension takes (65,536) and than 2^23, and rows of more than 1024 features.
 KAN_SHAPES = [
     (130, 45, 70, 5, 3, 1.5, "uniform"),
     (67, 33, 258, 9, 3, 1.0, "random"),
@@ -120,22 +121,47 @@ KAN_SHAPES = [
     (64, 96, 40, 8, 3, 1.0, "mixed_edge"),
     (21, 40, 50, 6, 2, 1.2, "random"),
     (16, 12, 8, 13, 1, 1.0, "uniform"),
-    # Row-wise path with more batch rows than a grid's y dimension takes (65,536), and with
-    # more than one launch's 2^23 rows.
     (70001, 3, 5, 4, 2, 1.0, "uniform"),
     ((1 << 23) + 5, 1, 3, 3, 2, 1.0, "uniform"),
+    (24, 1100, 40, 5, 3, 1.0, "uniform"),
+    (20, 1030, 33, 10, 3, 1.0, "random"),
+]
+# kan_pack and kan_fused: order 3, at most 16 knots (C = 4, 7, 8, 11 and 12 cover both padded
+# basis widths), enough work to pay for the packing.
+KAN_PACKED_SHAPES = [
     # Split-K (fewer output tiles than CUs): 64 tiles and 5 feature groups split 2+2+1;
     # 96 tiles, ragged O and 3 groups split 2+1.
     (4096, 160, 512, 8, 3, 1.0, "uniform"),
     (4096, 90, 600, 5, 3, 1.0, "random"),
+    (2050, 60, 701, 5, 3, 1.2, "jitter"),
+    (2049, 64, 700, 5, 3, 1.2, "mixed"),
+    (2600, 96, 513, 8, 3, 1.0, "mixed_edge"),
+    (4001, 45, 602, 4, 3, 1.3, "random"),
+    (2000, 30, 1500, 1, 3, 1.0, "uniform"),
+    (5000, 70, 700, 9, 3, 1.5, "uniform"),
+    (5003, 70, 699, 9, 3, 1.0, "mixed"),
     # More than 1024 features: the weight packing reads each column twice instead of
     # keeping one batch of runs in registers (both padded basis widths).
-    (24, 1100, 40, 5, 3, 1.0, "uniform"),
-    (20, 1030, 33, 10, 3, 1.0, "random"),
+    (1201, 1100, 140, 5, 3, 1.0, "uniform"),
+    (1500, 1030, 701, 9, 3, 1.0, "random"),
+]
+# kan_rowwise: order 0 or above 4, or fewer than four bases; more rows than one launch's 2^23.
+KAN_ROWWISE_SHAPES = [
+    (70, 45, 300, 5, 0, 1.2, "uniform"),
+    (33, 130, 40, 9, 0, 1.2, "random"),
+    (65, 40, 70, 3, 5, 1.3, "uniform"),
+    (9, 129, 257, 6, 6, 1.0, "random"),
+    (130, 30, 20, 1, 1, 1.2, "uniform"),
+    (21, 17, 256, 2, 1, 1.2, "random"),
+    (40, 257, 33, 1, 2, 1.2, "uniform"),
+    ((1 << 23) + 5, 1, 3, 1, 2, 1.0, "uniform"),
 ]
 
 
-@pytest.mark.parametrize("shape", KAN_SHAPES, ids=[f"B{s[0]}_I{s[1]}_O{s[2]}_G{s[3]}_K{s[4]}_{s[6]}" for s in KAN_SHAPES])
+KAN_ALL = KAN_SHAPES + KAN_PACKED_SHAPES + KAN_ROWWISE_SHAPES
+
+
+@pytest.mark.parametrize("shape", KAN_ALL, ids=[f"B{s[0]}_I{s[1]}_O{s[2]}_G{s[3]}_K{s[4]}_{s[6]}" for s in KAN_ALL])
 def test_efficient_kan_shapes(lib, shape):
     B, I, O, G, K, xr, knots = shape
     print(f"\n[parity] efficient_kan {shape}", flush=True)
@@ -165,11 +191,16 @@ def test_efficient_kan_shapes(lib, shape):
 # dominates) and BASELINE's: knot rows jittered by 4.5e-7 h stay on the cardinal pieces
 # (uniform to 5e-7 h), which then differ from the exact bases by about 1e-6 of a basis
 # value; rows jittered by 9e-6 h take the table's exact per-interval cubics.
+# 256 rows run the direct path, which has no such limit.
+JITTER_ROWS = [256, 640]
+
+
+@pytest.mark.parametrize("B", JITTER_ROWS)
 @pytest.mark.parametrize("jitter", [4.5e-7, 9e-6])
 @pytest.mark.parametrize("weights", ["reference", "baseline"])
-def test_efficient_kan_knot_jitter_full_width(lib, jitter, weights):
-    print(f"\n[parity] efficient_kan B256 I1024 O1024 G5, knots jittered by {jitter:g} h, {weights} weights", flush=True)
-    case = dict(name="kj", seed=4620, B=256, I=1024, O=1024, grid_size=5, spline_order=3, x_range=1.0)
+def test_efficient_kan_knot_jitter_full_width(lib, jitter, weights, B):
+    print(f"\n[parity] efficient_kan B{B} I1024 O1024 G5, knots jittered by {jitter:g} h, {weights} weights", flush=True)
+    case = dict(name="kj", seed=4620, B=B, I=1024, O=1024, grid_size=5, spline_order=3, x_range=1.0)
     if weights == "baseline":
         case["kind"] = "baseline"
     inp = inputs.make_inputs("efficient_kan", case)
@@ -215,25 +246,24 @@ def test_efficient_kan_spline_weights_past_2gib(lib):
     assert t["mismatched"] == 0, t
 
 
-# (M, K, N, output offset in bf16 elements).  K % 16 == 0 with 16-byte aligned operands
-# runs the wide kernel: its three epilogues (N % 8 == 0 and a 16-byte aligned output; N % 4
-# == 0 and 8-byte aligned; otherwise), M and N tile tails, K not a multiple of its 128-wide
-# step.  Up to 128 tiles of 256x256 (half the 256 CUs) it runs in its 128x256-tile form
-# (fp8_gemm_half): every wide shape below up to the reference's timed M=2048 K=1024 N=4096;
-# the M=2200 shapes (9 x 16 tiles) run the 256x256 form with the same tails.  K % 16 != 0
-# runs the tiled kernel; M <= 64 the skinny (flat loads through LDS when K % 16 == 0, loads
-# in the MFMA layout otherwise).
+# (M, K, N, output offset in bf16 elements), by the kernel that takes them at 256 CUs
+# (test_host_paths.py pins that): the wide kernel (256x256 tiles and fp8_gemm_half, its 128x256
+# form) with its three epilogues (N % 8 == 0 and a 16-byte aligned output; N % 4 == 0 and 8-byte
+# aligned; otherwise), M and N tile tails, K not a multiple of its 128-wide step; the middle
+# kernel (few tiles, other K and alignments: test_fp8_mid.py has more); and the skinny one.
 FP8_SHAPES = [
     (2048, 1024, 4096, 0),
     (2200, 144, 4000, 0),
     (2200, 144, 4004, 4),
     (2200, 176, 3999, 0),
+    # middle kernel
     (300, 192, 264, 0),
     (300, 192, 264, 4),
     (257, 48, 260, 0),
     (130, 16, 257, 0),
     (333, 1000, 300, 0),
     (65, 40, 33, 1),
+    # skinny, one row block more than three
     (64, 4096, 96, 0),
     # skinny, flat 16-byte path: one to four row blocks (K slices of 512, 256, 256 and 128
     # bytes), K past the last whole slice, N past the last 16-column block
@@ -270,11 +300,11 @@ def test_fp8_linear_shapes(lib, shape):
     assert torch.isnan(buf[:off].float()).all() and torch.isnan(buf[off + M * N:].float()).all()
 
 
-def test_fp8_linear_k0(lib):
-    """K == 0: the product is empty, so every output row is the bias (the wide kernel's
-    copies are all out of range and zero-fill)."""
-    M, N = 70, 72
-    print("\n[parity] fp8_linear K=0", flush=True)
+@pytest.mark.parametrize("M,N", [(70, 72), (2200, 4000), (2000, 4000), (16, 40)])
+def test_fp8_linear_k0(lib, M, N):
+    """K == 0: the product is empty, so every output row is the bias (the kernels' copies are
+    all out of range and zero-fill); on the middle, wide, half and skinny kernels."""
+    print(f"\n[parity] fp8_linear K=0 M={M} N={N}", flush=True)
     bias = (torch.randn(N, generator=torch.Generator().manual_seed(3)) * 0.05).to(torch.bfloat16)
     args = dict(M=M, K=0, N=N, x_fp8=torch.empty(M, 0, dtype=torch.uint8, device="cuda"), scale_x=1.0,
                 w_fp8=torch.empty(N, 0, dtype=torch.uint8, device="cuda"), scale_w=1.0,

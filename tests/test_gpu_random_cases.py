@@ -7,7 +7,8 @@ test_gpu_parity.py sit on each kernel's boundaries (tile tails, chunk counts, la
 these cases draw shapes between and across them, with the distribution parameters the input
 builders take (scale, mem0, beta range, gamma, done rate, clip epsilon, knot count and
 spline order, x range).  fp8_linear's K includes values off a multiple of 16, which take the
-register-staged and byte-wise kernels.  The draws are fixed by the seed below, so a failure
+register-staged and byte-wise loads.  efficient_kan's draws are small and take its direct path;
+a second set has the batches and widths of the packed one (test_host_paths.py pins that).  The draws are fixed by the seed below, so a failure
 names a reproducible case.
 """
 import random
@@ -55,7 +56,17 @@ def _cases():
     return [(op, _draw(op, rng, i)) for op in tasks.OPS for i in range(PER_OP)]
 
 
-CASES = _cases()
+def _packed_cases(n=8):
+    """efficient_kan cases of the packed path: order 3, at most 16 knots."""
+    rng = random.Random(SEED + 1)
+    return [("efficient_kan", {"name": f"packed{i}", "seed": 97_000 + 31 * i, "small": False, "timed": False,
+                               "B": rng.randint(3000, 6000), "I": rng.randint(64, 200), "O": rng.randint(513, 768),
+                               "grid_size": rng.randint(1, 9), "spline_order": 3, "x_range": rng.uniform(0.5, 1.5)})
+            for i in range(n)]
+
+
+PACKED_CASES = _packed_cases()
+CASES = _cases() + PACKED_CASES
 
 
 def _label(c: dict) -> str:

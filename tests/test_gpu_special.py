@@ -10,7 +10,8 @@ exists, against a closed form of the op (the closed forms named for each op's or
 - efficient_kan: zero spline weights (silu(x) @ Wb^T only), zero base weights (spline
   term only), x outside the knot span (spline term zero);
 - fp8_linear: zero x (out = bias), e4m3 NaN codes in x (their rows NaN), +-448 codes; on the
-  skinny, wide and tiled kernels.
+  skinny, middle (direct and staged copies), half and wide kernels.
+test_host_paths.py pins which path takes each shape.
 """
 import math
 
@@ -150,14 +151,18 @@ def test_pow_identical_inputs(lib):
 
 # ---- efficient_kan ------------------------------------------------------------------------
 
-def _kan_inputs(seed):
-    return inputs.make_inputs("efficient_kan", dict(name="s", seed=seed, B=70, I=45, O=60, grid_size=5,
-                                                    spline_order=3))
+KAN_PATHS = {"direct": (70, 45, 60, 5, 3), "fast": (2050, 60, 701, 5, 3), "rowwise": (70, 45, 60, 5, 0)}
 
 
-def test_kan_zero_spline_weights(lib):
-    print("\n[special] efficient_kan Ws = 0", flush=True)
-    inp = _kan_inputs(4900)
+def _kan_inputs(seed, path):
+    B, I, O, G, K = KAN_PATHS[path]
+    return inputs.make_inputs("efficient_kan", dict(name="s", seed=seed, B=B, I=I, O=O, grid_size=G, spline_order=K))
+
+
+@pytest.mark.parametrize("path", list(KAN_PATHS))
+def test_kan_zero_spline_weights(lib, path):
+    print(f"\n[special] efficient_kan Ws = 0, {path}", flush=True)
+    inp = _kan_inputs(4900, path)
     inp["spline_weight"] = torch.zeros_like(inp["spline_weight"])
     got = capi.run_op(lib, "efficient_kan", inp)["out"].cpu().numpy()
     _agree("efficient_kan", got, exact.efficient_kan(inp)["out"])
@@ -166,17 +171,19 @@ def test_kan_zero_spline_weights(lib):
     _agree("efficient_kan", got, silu @ inp["base_weight"].double().numpy().T)
 
 
-def test_kan_zero_base_weights(lib):
-    print("\n[special] efficient_kan Wb = 0", flush=True)
-    inp = _kan_inputs(4910)
+@pytest.mark.parametrize("path", list(KAN_PATHS))
+def test_kan_zero_base_weights(lib, path):
+    print(f"\n[special] efficient_kan Wb = 0, {path}", flush=True)
+    inp = _kan_inputs(4910, path)
     inp["base_weight"] = torch.zeros_like(inp["base_weight"])
     got = capi.run_op(lib, "efficient_kan", inp)["out"].cpu().numpy()
     _agree("efficient_kan", got, exact.efficient_kan(inp)["out"])
 
 
-def test_kan_inputs_outside_the_knots(lib):
-    print("\n[special] efficient_kan x outside the knot span", flush=True)
-    inp = _kan_inputs(4920)
+@pytest.mark.parametrize("path", list(KAN_PATHS))
+def test_kan_inputs_outside_the_knots(lib, path):
+    print(f"\n[special] efficient_kan x outside the knot span, {path}", flush=True)
+    inp = _kan_inputs(4920, path)
     span = float(inp["grid"].abs().max())
     sign = torch.where(torch.rand(inp["x"].shape, generator=torch.Generator().manual_seed(4920)) < 0.5, -1.0, 1.0)
     inp["x"] = (sign * (span + 0.5 + inp["x"].abs())).contiguous()
@@ -188,14 +195,15 @@ def test_kan_inputs_outside_the_knots(lib):
 
 # ---- fp8_linear ---------------------------------------------------------------------------
 
-FP8_KERNELS = [(16, 256, 96), (300, 256, 264), (130, 40, 70)]  # skinny, wide, tiled
+FP8_KERNELS = {"skinny": (16, 256, 96), "mid_direct": (300, 256, 264), "mid_staged": (130, 40, 70),
+               "half": (2000, 144, 4000), "wide": (2200, 144, 4000)}
 
 
 def _fp8_inputs(M, K, N, seed):
     return inputs.make_inputs("fp8_linear", dict(name="s", seed=seed, M=M, K=K, N=N))
 
 
-@pytest.mark.parametrize("shape", FP8_KERNELS, ids=["skinny", "wide", "tiled"])
+@pytest.mark.parametrize("shape", list(FP8_KERNELS.values()), ids=list(FP8_KERNELS))
 def test_fp8_zero_x_gives_the_bias(lib, shape):
     M, K, N = shape
     print(f"\n[special] fp8_linear zero x {shape}", flush=True)
@@ -205,7 +213,7 @@ def test_fp8_zero_x_gives_the_bias(lib, shape):
     assert torch.equal(got, inp["bias"].reshape(1, N).expand(M, N))
 
 
-@pytest.mark.parametrize("shape", FP8_KERNELS, ids=["skinny", "wide", "tiled"])
+@pytest.mark.parametrize("shape", list(FP8_KERNELS.values()), ids=list(FP8_KERNELS))
 def test_fp8_nan_and_extreme_codes(lib, shape):
     M, K, N = shape
     print(f"\n[special] fp8_linear NaN and +-448 codes {shape}", flush=True)

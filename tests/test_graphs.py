@@ -33,10 +33,17 @@ def _bind(op, inp):
     return args, outs
 
 
-@pytest.mark.parametrize("op", list(SMALL))
-def test_graph_replay_matches_eager(lib, op):
-    print(f"\n[graph] {op}", flush=True)
-    case = SMALL[op]
+# efficient_kan's packed path, and fp8_linear's wide kernel (test_host_paths.py pins that).
+LARGE = {
+    "efficient_kan": dict(name="g", seed=5, B=2050, I=60, O=701),
+    "fp8_linear": dict(name="g", seed=6, M=2200, K=144, N=4000),
+}
+
+
+@pytest.mark.parametrize("op,size", [(op, "small") for op in SMALL] + [(op, "large") for op in LARGE])
+def test_graph_replay_matches_eager(lib, op, size):
+    print(f"\n[graph] {op} {size}", flush=True)
+    case = (SMALL if size == "small" else LARGE)[op]
     args, outs = _bind(op, inputs.make_inputs(op, case))
     capi.call(lib, op, args)           # eager call first: the workspace is allocated here
     torch.cuda.synchronize()

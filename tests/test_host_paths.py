@@ -183,3 +183,35 @@ def test_fp8_more_tiles_than_one_launch_takes(host):
     out = host([call("fp8_linear", M=70_000_000, K=1, N=2000, scale_x=1.0, scale_w=1.0)])[0]
     grids = [int(line.split("grid ")[1].split()[0]) for line in out["log"] if line.startswith("launch")]
     assert out["rc"] == 0 and max(grids) * 512 < 2 ** 32 and sum(grids) == 546_875 * 16, out
+
+
+def test_gpu_tests_reach_the_paths_they_name(host):
+    """The shape lists of the GPU tests, by path: a change of the rules shows here."""
+    import test_gpu_parity as parity
+    import test_gpu_random_cases as rand
+    import test_gpu_special as special
+    import test_graphs as graphs
+
+    def kan(cases):
+        return set(kan_kernel(host, *[tuple(c) for c in cases]))
+
+    def sizes(case):
+        return [case[k] for k in ("B", "I", "O")] + [case.get("grid_size", 5), case.get("spline_order", 3)]
+
+    assert kan(s[:5] for s in parity.KAN_SHAPES) == {"direct"}
+    assert kan(s[:5] for s in parity.KAN_PACKED_SHAPES) == {"fast"}
+    assert kan(s[:5] for s in parity.KAN_ROWWISE_SHAPES) == {"rowwise"}
+    assert kan_kernel(host, *[(B, 1024, 1024, 5) for B in parity.JITTER_ROWS]) == ["direct", "fast"]
+    assert kan(sizes(c) for _, c in rand.PACKED_CASES) == {"fast"}
+    assert kan([sizes(graphs.SMALL["efficient_kan"])]) == {"direct"} and kan([sizes(graphs.LARGE["efficient_kan"])]) == {"fast"}
+    assert kan_kernel(host, *special.KAN_PATHS.values()) == list(special.KAN_PATHS)
+
+    def fp8(*cases):
+        names = ["fp8_gemm_skinny_flat", "fp8_gemm_skinny", "fp8_gemm_mid", "fp8_gemm_half", "fp8_gemm_wide"]
+        return [next(n for n in names if n in k)[9:] for k in fp8_kernel(host, *[c[:3] for c in cases])]
+
+    assert fp8(*special.FP8_KERNELS.values()) == ["skinny_flat", "mid", "mid", "half", "wide"]
+    assert set(fp8(*parity.FP8_SHAPES)) == {"skinny_flat", "skinny", "mid", "half", "wide"}
+    assert fp8((70, 0, 72), (2200, 0, 4000), (2000, 0, 4000), (16, 0, 40)) == ["mid", "wide", "half", "skinny_flat"]
+    large = graphs.LARGE["fp8_linear"]
+    assert fp8((large["M"], large["K"], large["N"])) == ["wide"]
