@@ -89,7 +89,8 @@ EXPECTED_LAUNCHES = {
     "ppo_clip_entropy_noalloc": 1,  # its first call on a device adds the scratch clear
     "efficient_kan": 2,          # kan_pack + kan_fused, or kan_direct + kan_direct_sum
     "efficient_kan_direct": 1,   # kan_direct alone: features unsplit, or summed by the last arrival
-    "efficient_kan_rowwise": 1,  # kan_rowwise (spline order 0 or above 4)
+    "efficient_kan_rowwise": 1,  # kan_rowwise (spline order 0 or above 4, fewer than four bases)
+    "reward_to_go_split": 2,     # few long rows: each part's map, then the parts
     "fp8_linear": 1,
     "quantize_e4m3": 2,          # qz_amax + qz_cast (unaligned, or more than 134 M elements)
     "quantize_e4m3_fused": 1,    # qz_fused or qz_hold (aligned)
@@ -98,8 +99,8 @@ EXPECTED_LAUNCHES = {
 
 def workloads():
     """(name, entry point, expectation key, make_args) for every hidden and public case of
-    the six ops, the entropy variant of ppo_clip (allocating and not), efficient_kan's
-    other spline orders and the quantiser (aligned and unaligned)."""
+    the six ops, the entropy variant of ppo_clip (allocating and not), split reward_to_go rows,
+    efficient_kan's other spline orders and the quantiser (aligned and unaligned)."""
     import torch
     from cob_amd import capi, inputs, tasks
 
@@ -140,6 +141,10 @@ def workloads():
                             drop_in(op, case, entropy=True)))
                 out.append((f"ppo_clip_entropy_noalloc/{case['name']}", "ppo_clip_entropy_noalloc",
                             "ppo_clip_entropy_noalloc", drop_in(op, case, entropy=True)))
+    rows = dict(name="B16_T65536_split", seed=60, small=False, timed=False, B=16, T=65536, gamma=0.99, done_p=0.001)
+    out.append((f"reward_to_go/{rows['name']}", "reward_to_go", "reward_to_go_split", drop_in("reward_to_go", rows)))
+    sums = dict(name="B20_I333_O131_G10_sum", seed=61, small=False, timed=False, B=20, I=333, O=131, grid_size=10)
+    out.append((f"efficient_kan/{sums['name']}", "efficient_kan", "efficient_kan", drop_in("efficient_kan", sums)))
     for order in (1, 2, 5):
         case = dict(name=f"B64_I40_O24_order{order}", seed=70 + order, small=True, timed=False,
                     B=64, I=40, O=24, spline_order=order)

@@ -428,9 +428,9 @@ __global__ __launch_bounds__(kThreads) void kan_direct(
     // Every split stores its tile, 16 bytes per lane and row block.  Without counters
     // kan_direct_sum adds them.  With counters it then arrives on the tile's, and the last adds
     // the splits' tiles in split order, so the result does not depend on which one that is.
-    // The stores and the loads are system-scope (sc0 sc1): they go through
-    // to the coherence point, a store's completion (vmcnt) means it got there, and the arrival
-    // follows every wave's wait for that.  So no L2 needs writing back or invalidating: with
+    // Its stores and loads are system-scope (sc0 sc1) and go through to the coherence point: a
+    // store's completion (vmcnt) means that it got there, and the arrival follows every wave's
+    // wait for that.  So no L2 needs writing back or invalidating: with
     // agent-scope fences, one per workgroup, the write-backs queued up (B = 64, I = O = 1024
     // 55 us; a second launch for the sums 27.0).
     constexpr int kTile = kRows * kCols;

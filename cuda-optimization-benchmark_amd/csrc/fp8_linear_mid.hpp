@@ -183,8 +183,9 @@ __global__ __launch_bounds__(kThreads) void fp8_gemm_mid(
     load(0, v0);
     if (nk > 1) load(1, v1);
     // Stage kt % 2 is rewritten two steps on, past a barrier that follows its last read.  The
-    // fragments are read in their own step: the registers of a second set cost the second
-    // workgroup per CU that covers the reads (M = 2000, K = 1000, N = 3000: 17.4 against 21.6 us).
+    // fragments are read in their own step.  Read a step ahead, M = 2000, K = 1000, N = 3000 took 21.6
+    // us instead of 17.4; its 128 x 128 tiles fit one workgroup per CU either way (98,816 bytes of
+    // LDS), so the cause is another one, which was not found.
     for (int kt = 0; kt < nk; kt += 2) {
       write(0, v0);
       if (kt + 2 < nk) load(kt + 2, v0);
