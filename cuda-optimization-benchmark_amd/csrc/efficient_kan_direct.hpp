@@ -23,9 +23,9 @@
 //
 // Bound: for batches up to about 32 rows by the weight stream and two launches' latency (B = 8,
 // I = O = 1024, G = 5: 42 MB in 15.6 us, 71.4 with the fp16x3 path), above by the fp32 MFMAs
-// and the expansion beside them (fp32 MFMAs and VALU instructions do not overlap): B = 1024,
-// I = 256, O = 512, G = 16 takes 66.3 us, 35 of them MFMA time, against 11,050 for the row-wise
-// kernel; there the loads and LDS reads cost 3 us and the expansion about 14.
+// and the expansion beside them: B = 1024, I = 256, O = 512, G = 16 takes 66.3 us, against
+// 11,050 for the row-wise kernel; of its busy cycles the counters give 57 % to the MFMAs and
+// 30 % to the VALU, 17 % of them with the LDS in use.
 #pragma once
 
 #include "common.hpp"

@@ -13,9 +13,10 @@
 // two LDS stages; the row's last 16 bytes are loaded from K - 16 on and shifted, so no load
 // leaves the operand.
 //
-// Bound: the LDS, 16 KiB written and 32 KiB read per step of a 64 x 64 tile (384 cycles of the
-// 420 it takes), 24 + 48 of a 64 x 128 one (576 of 740); the MFMAs need 128 and 256.  Measured
-// (us, against the 128 x 256 form): M = 512, K = N = 4096 14.0 / 24.0, M = 256 9.3 / 24.0, M =
+// Bound: no unit by itself.  At M = 512, K = N = 4096 (64 x 128 tiles, one workgroup per CU) the
+// counters read the MFMAs busy 28 % of a CU's cycles, the LDS 25 % (2 % of that bank
+// conflicts) and the VALU 32 %: what is left is a step's chain of loads, barrier and LDS reads,
+// and the launch.  Measured (us, against the 128 x 256 form): M = 512, K = N = 4096 14.0 / 24.0, M = 256 9.3 / 24.0, M =
 // 1024 19.0 / 24.3; K = 8192, N = 1024, M = 512 13.8 / 41.1.  Against the register-staged 256 x
 // 256 kernel that took other K: M = 333, K = 1000, N = 3000 7.0 / 34.9, M = 1000, K = N = 1001
 // 6.7 / 138, M = 4096, K = 4088, N = 4096 97 / 103.
