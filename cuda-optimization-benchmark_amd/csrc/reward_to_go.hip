@@ -53,20 +53,20 @@ void launch(const float* reward, const uint8_t* done, double g, int B, int T, fl
 // Few long rows.  A workgroup walks its row one segment of 4096 steps after another, about 2.2
 // us each, so such rows are split into parts over workgroups: one launch composes each part's
 // map, a second scans each part from the maps after it, reading the rewards again (from the
-// caches).  Whole row against split, us per call: 16 x 65536 33-39 / 7.6, 1 x 131072 71 / 6.9,
-// 6 x 18592 12.4 / 6.5, 33 x 109969 75-140 / 14.0, 128 x 131072 82.7 / 40.8, 256 x 65536 46.2 / 39.8, 1 x
-// 1048576 600 / 14.7, 256 x 1048576 689 / 689.
+// caches).  Whole row against split, us per call: 16 x 65536 33-39 / 7.4, 1 x 131072 71 / 6.5,
+// 6 x 18592 12.4 / 5.8, 33 x 109969 75-140 / 13.4, 128 x 131072 82.7 / 39.5, 256 x 65536 46.2 / 38.7, 1 x
+// 1048576 600 / 12.9, 256 x 1048576 689 / 691.
 // Rows of at most 12288 steps (three segments) or more than 256 of them keep the whole-row
 // form: 1 x 8000 5.7 / 8.0, 229 x 9751 11.5 / 11.6, 256 x 16384 13.3 / 13.3, 512 x 8192 9.5 / 13.3.
 constexpr int kSplitMaxRows = 256, kSplitMinChunks = 48;
 // Chunks in all up to which parts have 4 chunks and 8, one and two per wave; beyond, four per wave
-// in 16 or more: at 4, 8 and 16 16 x 65536 8.5, 7.6 and 8.3 us, 64 x 16384 8.1, 7.4 and 8.2, 8 x 65536
-// 7.1, 7.2 and 8.1, 4 x 65536 6.5 and 6.7.  More parts would not find room for their maps either.
+// in 16 or more: at 4, 8 and 16 16 x 65536 7.8, 7.4 and 8.4 us, 64 x 16384 7.7, 7.3 and 8.4, 8 x 65536
+// 6.6, 6.7 and 8.1, 4 x 65536 6.0 and 6.5.  More parts would not find room for their maps either.
 constexpr int kPart4Chunks = 1024, kPart8Chunks = 4096;
 static_assert(kPart4Chunks / 4 <= 4 * kRtgMapsPerChunk && kPart8Chunks / 8 <= 8 * kRtgMapsPerChunk, "room for the maps");
 // Chunks per part of a call in parts of 16 or more: more where a part's outputs have no room for
 // the maps after it (rows past 4.2 M steps), and beyond what fills the chip where the maps'
-// copies, one to each earlier part, add up: 8 x 2097152 71.6 us in 512 parts a row, 47.3 in 256.
+// copies, one to each earlier part, add up: 8 x 2097152 71.6 us in 512 parts a row, 46.4 in 256.
 int long_part(int B, int nchunks) {
   const int64_t nseg = ((int64_t)nchunks + 15) / 16;
   int64_t m = std::max<int64_t>((nseg + 16 * kRtgMapsPerChunk - 1) / (16 * kRtgMapsPerChunk), B * nseg / 4096);
@@ -76,17 +76,31 @@ int long_part(int B, int nchunks) {
   }
 }
 
+// The factor of two composed maps.  Where it is too small for a double it stays the smallest one,
+// not zero: only a done step makes a factor zero, and 0 * inf would turn the infinity that an
+// infinite reward sends up its row into NaN.
+double rtg_factor(double a, double b) {
+  const double p = a * b;
+  return p == 0.0 && a != 0.0 && b != 0.0 ? 0x1p-1074 : p;
+}
+
 template <int kSeg, RtgAccess kAccess>
 hipError_t launch_split(const float* reward, const uint8_t* done, double g, int B, int T, float* out, int nparts,
                         int cpart, hipStream_t stream) {
   constexpr int kWaves = 4;
+  RtgPowers power;
+  double q = g;
+  power.p[0] = 1.0;
+  for (int e = kWave * kPerLane * cpart; e > 0; e >>= 1, q = rtg_factor(q, q))
+    if (e & 1) power.p[0] = rtg_factor(power.p[0], q);
+  for (int i = 1; i < 7; ++i) power.p[i] = rtg_factor(power.p[i - 1], power.p[i - 1]);
   // Ordinary loads in the first pass, so that the second finds the rewards in the caches.
   hipLaunchKernelGGL((reward_to_go_kernel<kWaves, kPerLane, kSeg, kAccess, 0, kMaps>), dim3(B * nparts),
-                     dim3(kWaves * kWave), 0, stream, reward, done, g, B, T, out, nparts, cpart);
+                     dim3(kWaves * kWave), 0, stream, reward, done, g, B, T, out, nparts, cpart, power);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((reward_to_go_kernel<kWaves, kPerLane, kSeg, kAccess, policy<kAccess>(), kApply>), dim3(B * nparts),
-                     dim3(kWaves * kWave), 0, stream, reward, done, g, B, T, out, nparts, cpart);
+                     dim3(kWaves * kWave), 0, stream, reward, done, g, B, T, out, nparts, cpart, power);
   return hipGetLastError();
 }
 

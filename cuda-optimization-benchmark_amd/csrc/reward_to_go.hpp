@@ -66,7 +66,7 @@ __device__ __forceinline__ float coef32(unsigned word, int byte, float g) {
 // they are the slowest (reward_to_go.hip).
 // The descriptor spans the row, so T * 4 bytes must fit its 32-bit size: the host takes
 // rows of 2^30 steps or more down the element path.
-template <int kStorePolicy>  // bit 0 sc0, bit 1 nt
+template <int kStorePolicy>  // bit 0 sc0, bit 1 nt, bit 4 sc1
 __device__ __forceinline__ void store_row16(float* row_base, int T, int t, f32x4 w) {
   const __amdgpu_buffer_rsrc_t rs =
       __builtin_amdgcn_make_buffer_rsrc(row_base, (short)0, (int)((unsigned)T * 4u), 0x00020000);
@@ -92,9 +92,15 @@ enum RtgAccess : int { kElements = 0, kAligned = 1, kUnaligned = 2 };
 // any number of streams and threads and under graph capture.
 enum RtgMode : int { kWhole = 0, kMaps = 1, kApply = 2 };
 
-// A part's map v -> r + a v.
+// A part's map v -> r + a v, a = 0 where a done step cuts it and else g^(steps), which all parts
+// but the row's last, after which nothing comes, have in common: it passes as r and a flag.
 struct RtgMap {
-  double r, a;
+  double r;
+  bool open;  // a != 0
+};
+// The factors of 1, 2, 4 .. 64 parts with no done step.
+struct RtgPowers {
+  double p[7];
 };
 // Maps that the outputs of one chunk (256 floats) have room for.
 constexpr int kRtgMapsPerChunk = 64;
@@ -104,43 +110,34 @@ namespace rtg_detail {
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef u32x4 __attribute__((aligned(4))) u32x4u;
 __device__ __forceinline__ u32x4 pack_map(RtgMap m) {
-  const unsigned long long r = (unsigned long long)__double_as_longlong(m.r), a = (unsigned long long)__double_as_longlong(m.a);
-  return u32x4{(unsigned)r, (unsigned)(r >> 32), (unsigned)a, (unsigned)(a >> 32)};
+  const unsigned long long r = (unsigned long long)__double_as_longlong(m.r);
+  return u32x4{(unsigned)r, (unsigned)(r >> 32), m.open ? 1u : 0u, 0u};
 }
 __device__ __forceinline__ RtgMap unpack_map(u32x4 v) {
-  return RtgMap{__longlong_as_double((long long)(((unsigned long long)v.y << 32) | v.x)),
-                __longlong_as_double((long long)(((unsigned long long)v.w << 32) | v.z))};
-}
-
-// The factor of two composed maps.  Where it is too small for a double it stays the smallest one,
-// not zero: only a done step makes a factor zero, and 0 * inf would turn the infinity that an
-// infinite reward sends up its row into NaN.
-__device__ __forceinline__ double factor(double a, double b) {
-  const double p = a * b;
-  return p == 0.0 && a != 0.0 && b != 0.0 ? 0x1p-1074 : p;
+  return RtgMap{__longlong_as_double((long long)(((unsigned long long)v.y << 32) | v.x)), v.z != 0u};
 }
 
 // n maps of consecutive parts composed and applied to 0, the same in every lane: lane l of
 // each batch of 64 takes one part, a suffix scan composes the batch, and batches are composed
-// from the row's end, always in this order, so the bits do not depend on timing.
-__device__ __forceinline__ double compose_after(const u32x4u* maps, int n, int lane) {
+// from the row's end, always in this order, so the bits do not depend on timing.  As in the lane
+// scan a span's factor is 0, by the mask, or the level's power: factors in the lanes, shuffled and
+// kept from underflow, cost 1 x 131072 0.5 us of 7.0, and leaving out the levels that n does not
+// need 0.7 (its branches wait for each power's load).
+__device__ __forceinline__ double compose_after(const u32x4u* maps, int n, int lane, const RtgPowers& power) {
   double v = 0.0;
   for (int p0 = (n - 1) / kWave * kWave; p0 >= 0 && n > 0; p0 -= kWave) {
-    double r = 0.0, a = 1.0;
-    if (p0 + lane < n) {
-      const RtgMap m = unpack_map(maps[p0 + lane]);
-      r = m.r;
-      a = m.a;
-    }
+    RtgMap m{0.0, true};
+    if (p0 + lane < n) m = unpack_map(maps[p0 + lane]);
+    unsigned long long mask = __ballot(!m.open);
+    double r = m.r;
 #pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {  // (r, a): the map of lanes lane .. lane + 2 off - 1
-      const double rn = __shfl_down(r, off, kWave), an = __shfl_down(a, off, kWave);
-      if (lane + off < kWave) {
-        r = fma(a, rn, r);
-        a = factor(a, an);
-      }
+    for (int lv = 0, off = 1; off < kWave; ++lv, off <<= 1) {  // r: of the map of lanes lane .. lane + 2 off - 1
+      const double rn = __shfl_down(r, off, kWave);
+      const double a = (mask >> lane) & 1ull ? 0.0 : power.p[lv];
+      if (lane + off < kWave) r = fma(a, rn, r);
+      mask |= mask >> off;
     }
-    v = fma(uniform(__shfl(a, 0, kWave)), v, uniform(__shfl(r, 0, kWave)));
+    v = fma(mask & 1ull ? 0.0 : power.p[6], v, uniform(__shfl(r, 0, kWave)));
   }
   return v;
 }
@@ -149,15 +146,16 @@ __device__ __forceinline__ double compose_after(const u32x4u* maps, int n, int l
 // kNT: bit 0 = non-temporal loads; bits 1-2 = the cache policy of buffer output stores
 // (store_row16), 0 = plain stores.  Split rows (kMode != kWhole): workgroup (row, part) =
 // (blockIdx.x / nparts, blockIdx.x % nparts) owns chunks part * cpart .. + cpart - 1, at least
-// (nparts - 1) / 64 of them (a part's room for the later maps).
+// (nparts - 1) / 64 of them (a part's room for the later maps); power
+// holds the powers of g^(256 cpart).
 template <int kWaves, int kPerLane, int kSeg, RtgAccess kAccess, int kNT, RtgMode kMode = kWhole>
 __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
     const float* __restrict__ reward, const uint8_t* __restrict__ done, double g, int B, int T,
-    float* __restrict__ out, int nparts = 1, int cpart = 0) {
+    float* __restrict__ out, int nparts = 1, int cpart = 0, RtgPowers power = {}) {
   using namespace rtg_detail;
   static_assert(kPerLane == 4, "a lane owns one 16-byte reward vector per chunk");
   constexpr int kChunk = kWave * kPerLane;
-  __shared__ double span_a[kWaves], span_r[kWaves];
+  __shared__ double span_a[kWaves], span_r[kWaves], later;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int nchunks = (T + kChunk - 1) / kChunk;
 
@@ -191,7 +189,8 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
   const float* rr = reward + base;
   const uint8_t* dd = done + base;
   float* oo = out + base;
-  double carry = 0.0, span = 1.0;  // span: kMaps, the a of the part's chunks so far
+  double carry = 0.0;
+  bool open = true;  // kMaps: no done step in the part's chunks so far
   for (int hi = end; hi > first; hi -= kWaves * kSeg) {
     const int lo = hi - first > kWaves * kSeg ? hi - kWaves * kSeg : first;
     const int c0 = lo + wave * kSeg;
@@ -234,10 +233,14 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
     }
 
     // The value entering this part, while the rewards are on their way; the outputs that take the
-    // maps' place are written past the barrier below.
+    // maps' place are written past the barrier below.  One wave composes it (every wave: 64 x 131072
+    // 21.4 us against 21.0, 128 x 131072 40.0 against 39.6).
     if constexpr (kMode == kApply)
-      if (hi == end)
-        carry = compose_after(reinterpret_cast<const u32x4u*>(oo + (size_t)first * kChunk), nparts - 1 - part, lane);
+      if (hi == end && wave == 0) {
+        const double v = compose_after(reinterpret_cast<const u32x4u*>(oo + (size_t)first * kChunk), nparts - 1 - part, lane,
+                                       power);
+        if (lane == 0) later = v;
+      }
 
     // Lane maps and wave suffix scans.  A map is (R, A): v -> R + A*v.  A lane's A over its
     // 4 steps is 0 if one of them is a done step, else g^4; in the suffix scan every
@@ -287,6 +290,8 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
       span_a[wave] = wa;
     }
     __syncthreads();
+    if constexpr (kMode == kApply)
+      if (hi == end) carry = later;
     // Compose the spans from the segment end: the value entering this wave's span, and the
     // value entering the segment (the next segment's carry).
     double x = carry, cin = carry;
@@ -297,10 +302,8 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
     }
     const double next_carry = x;
     if constexpr (kMode == kMaps) {
-      double a = 1.0;
 #pragma unroll
-      for (int v = 0; v < kWaves; ++v) a = factor(a, span_a[v]);
-      span = factor(span, a);
+      for (int v = 0; v < kWaves; ++v) open &= span_a[v] != 0.0;
       carry = next_carry;
       __syncthreads();
       continue;
@@ -349,9 +352,11 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
     __syncthreads();  // span_* are rewritten by the next segment
   }
   if constexpr (kMode == kMaps) {
-    const u32x4 m = pack_map(RtgMap{carry, span});
+    // Through the L2 (sc0 | sc1): ordinary stores leave a partial line dirty for each copy, which
+    // the end of the launch writes back: 64 x 131072 21.5 us, 21.1 with these, 22.9 with nt.
+    const f32x4 m = __builtin_bit_cast(f32x4, pack_map(RtgMap{carry, open}));
     for (int p = (int)threadIdx.x; p < part; p += kWaves * kWave)
-      reinterpret_cast<u32x4u*>(oo + (size_t)p * cpart * kChunk)[part - p - 1] = m;
+      store_row16<17>(oo, T, p * cpart * kChunk + 4 * (part - p - 1), m);
   }
 }
 
