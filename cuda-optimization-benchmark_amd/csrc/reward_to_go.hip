@@ -46,7 +46,7 @@ void launch(const float* reward, const uint8_t* done, double g, int B, int T, fl
     const int nb = B - b0 < kRowsPerLaunch ? B - b0 : kRowsPerLaunch;
     const size_t off = (size_t)b0 * (size_t)T;  // T % 4 == 0 on the aligned path: alignment kept
     hipLaunchKernelGGL((reward_to_go_kernel<kWaves, kPerLane, kSeg, kAccess, policy<kAccess>()>), dim3(nb),
-                       dim3(kWaves * kWave), lds, stream, reward + off, done + off, g, nb, T, out + off, 1, 0);
+                       dim3(kWaves * kWave), lds, stream, reward + off, done + off, g, nb, T, out + off, RtgArgs<kWhole>{});
   }
 }
 
@@ -88,19 +88,16 @@ template <int kSeg, RtgAccess kAccess>
 hipError_t launch_split(const float* reward, const uint8_t* done, double g, int B, int T, float* out, int nparts,
                         int cpart, hipStream_t stream) {
   constexpr int kWaves = 4;
-  RtgPowers power;
-  double q = g;
-  power.p[0] = 1.0;
-  for (int e = kWave * kPerLane * cpart; e > 0; e >>= 1, q = rtg_factor(q, q))
-    if (e & 1) power.p[0] = rtg_factor(power.p[0], q);
-  for (int i = 1; i < 7; ++i) power.p[i] = rtg_factor(power.p[i - 1], power.p[i - 1]);
+  double gpart = 1.0, power = g;  // g^(256 cpart)
+  for (int e = kWave * kPerLane * cpart; e > 0; e >>= 1, power = rtg_factor(power, power))
+    if (e & 1) gpart = rtg_factor(gpart, power);
   // Ordinary loads in the first pass, so that the second finds the rewards in the caches.
   hipLaunchKernelGGL((reward_to_go_kernel<kWaves, kPerLane, kSeg, kAccess, 0, kMaps>), dim3(B * nparts),
-                     dim3(kWaves * kWave), 0, stream, reward, done, g, B, T, out, nparts, cpart, power);
+                     dim3(kWaves * kWave), 0, stream, reward, done, g, B, T, out, RtgArgs<kMaps>{nparts, cpart});
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((reward_to_go_kernel<kWaves, kPerLane, kSeg, kAccess, policy<kAccess>(), kApply>), dim3(B * nparts),
-                     dim3(kWaves * kWave), 0, stream, reward, done, g, B, T, out, nparts, cpart, power);
+                     dim3(kWaves * kWave), 0, stream, reward, done, g, B, T, out, RtgArgs<kApply>{nparts, cpart, gpart});
   return hipGetLastError();
 }
 

@@ -98,9 +98,19 @@ struct RtgMap {
   double r;
   bool open;  // a != 0
 };
-// The factors of 1, 2, 4 .. 64 parts with no done step.
-struct RtgPowers {
-  double p[7];
+// The arguments that a mode adds: none for whole rows, and never more than 64 bytes in all (with 56
+// bytes more to pass a launch took the host 0.5 to 1 us longer, and small calls are all launch).
+// gpart: the factor of a part with no done step.
+template <RtgMode kMode>
+struct RtgArgs {};
+template <>
+struct RtgArgs<kMaps> {
+  int nparts, cpart;
+};
+template <>
+struct RtgArgs<kApply> {
+  int nparts, cpart;
+  double gpart;
 };
 // Maps that the outputs of one chunk (256 floats) have room for.
 constexpr int kRtgMapsPerChunk = 64;
@@ -120,24 +130,26 @@ __device__ __forceinline__ RtgMap unpack_map(u32x4 v) {
 // n maps of consecutive parts composed and applied to 0, the same in every lane: lane l of
 // each batch of 64 takes one part, a suffix scan composes the batch, and batches are composed
 // from the row's end, always in this order, so the bits do not depend on timing.  As in the lane
-// scan a span's factor is 0, by the mask, or the level's power: factors in the lanes, shuffled and
-// kept from underflow, cost 1 x 131072 0.5 us of 7.0, and leaving out the levels that n does not
-// need 0.7 (its branches wait for each power's load).
-__device__ __forceinline__ double compose_after(const u32x4u* maps, int n, int lane, const RtgPowers& power) {
+// scan a span's factor is 0, by the mask, or the level's power of gpart: factors in the lanes,
+// shuffled and kept from underflow, cost 1 x 131072 0.4 us of 6.9, and branches around the levels
+// that n does not need as much.
+__device__ __forceinline__ double compose_after(const u32x4u* maps, int n, int lane, double gpart) {
   double v = 0.0;
   for (int p0 = (n - 1) / kWave * kWave; p0 >= 0 && n > 0; p0 -= kWave) {
     RtgMap m{0.0, true};
     if (p0 + lane < n) m = unpack_map(maps[p0 + lane]);
     unsigned long long mask = __ballot(!m.open);
-    double r = m.r;
+    double r = m.r, power = gpart;
+    asm volatile("" : "+v"(power));  // the powers anew for each batch, not 14 registers of them
 #pragma unroll
-    for (int lv = 0, off = 1; off < kWave; ++lv, off <<= 1) {  // r: of the map of lanes lane .. lane + 2 off - 1
+    for (int off = 1; off < kWave; off <<= 1) {  // r: of the map of lanes lane .. lane + 2 off - 1
       const double rn = __shfl_down(r, off, kWave);
-      const double a = (mask >> lane) & 1ull ? 0.0 : power.p[lv];
+      const double a = (mask >> lane) & 1ull ? 0.0 : power;
       if (lane + off < kWave) r = fma(a, rn, r);
       mask |= mask >> off;
+      power = fmax(power * power, fmin(power, 0x1p-1074));  // kept from underflow, as gpart is
     }
-    v = fma(mask & 1ull ? 0.0 : power.p[6], v, uniform(__shfl(r, 0, kWave)));
+    v = fma(mask & 1ull ? 0.0 : power, v, uniform(__shfl(r, 0, kWave)));
   }
   return v;
 }
@@ -146,16 +158,21 @@ __device__ __forceinline__ double compose_after(const u32x4u* maps, int n, int l
 // kNT: bit 0 = non-temporal loads; bits 1-2 = the cache policy of buffer output stores
 // (store_row16), 0 = plain stores.  Split rows (kMode != kWhole): workgroup (row, part) =
 // (blockIdx.x / nparts, blockIdx.x % nparts) owns chunks part * cpart .. + cpart - 1, at least
-// (nparts - 1) / 64 of them (a part's room for the later maps); power
-// holds the powers of g^(256 cpart).
+// (nparts - 1) / 64 of them (a part's room for the later maps); gpart is
+// g^(256 cpart).
 template <int kWaves, int kPerLane, int kSeg, RtgAccess kAccess, int kNT, RtgMode kMode = kWhole>
 __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
     const float* __restrict__ reward, const uint8_t* __restrict__ done, double g, int B, int T,
-    float* __restrict__ out, int nparts = 1, int cpart = 0, RtgPowers power = {}) {
+    float* __restrict__ out, RtgArgs<kMode> args) {
   using namespace rtg_detail;
   static_assert(kPerLane == 4, "a lane owns one 16-byte reward vector per chunk");
   constexpr int kChunk = kWave * kPerLane;
   __shared__ double span_a[kWaves], span_r[kWaves], later;
+  int nparts = 1, cpart = 0;
+  if constexpr (kMode != kWhole) {
+    nparts = args.nparts;
+    cpart = args.cpart;
+  }
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int nchunks = (T + kChunk - 1) / kChunk;
 
@@ -235,12 +252,13 @@ __global__ __launch_bounds__(kWaves * 64) void reward_to_go_kernel(
     // The value entering this part, while the rewards are on their way; the outputs that take the
     // maps' place are written past the barrier below.  One wave composes it (every wave: 64 x 131072
     // 21.4 us against 21.0, 128 x 131072 40.0 against 39.6).
-    if constexpr (kMode == kApply)
+    if constexpr (kMode == kApply) {
       if (hi == end && wave == 0) {
         const double v = compose_after(reinterpret_cast<const u32x4u*>(oo + (size_t)first * kChunk), nparts - 1 - part, lane,
-                                       power);
+                                       args.gpart);
         if (lane == 0) later = v;
       }
+    }
 
     // Lane maps and wave suffix scans.  A map is (R, A): v -> R + A*v.  A lane's A over its
     // 4 steps is 0 if one of them is a done step, else g^4; in the suffix scan every
