@@ -47,6 +47,9 @@ bool offsets_fit(int64_t M, int64_t K, int64_t N) {
 //    with the weights in the L2s, and at N = 64, K = 4096 5.7 / 7.0.  Longer K from memory is too much for
 //    the few CUs that hold a tile: M = 39, K = 5536, N = 1568 (14.3 / 18.1), M = 48, K = 10352, N =
 //    1216 (26.6 / 36.6), although from the Infinity Cache the tiles would be faster.
+//  * 33 to 48 rows and short K: M = 42, K = 256, N = 1024 4.1 / 3.3 (4.7 / 3.3), M = 48, K = 768, N = 2048
+//    4.9 / 3.8 (5.0 / 4.4), K = 1280 5.1 / 4.4 (5.9 / 5.2); at K = 1536 5.2 / 4.6 (6.1 / 5.5) but 4.8 / 4.7 at
+//    N = 3360 and, with the weights in the L2s, 4.1 / 4.6; N = 512: K = 768 3.8 / 3.8, K = 1024 3.8 / 4.0.
 //  * 49 rows up at fewer columns: M = 64, K = 1024, N = 512 3.5 / 4.1, K = 2048, N = 4096 5.5 / 5.2 (6.0 /
 //    8.0), K = 7168, N = 1024 13.4 / 11.9 (13.7 / 19.3): the skinny kernel.
 //  * 33 rows up at less than two columns per CU, where the skinny kernel has few workgroups as well,
@@ -64,7 +67,8 @@ int mid_tile(int64_t M, int64_t K, int64_t N, int vec) {
     if (vec == 16) {
       if (rb == 1) tiles = N >= 28 * cus && (K <= 8192 || N > 32 * cus);
       else if (rb == 2) tiles = N >= 20 * cus;
-      else tiles = wide || (K > 4096 ? N < 2 * cus : rb == 3 && K > 2048 && N >= 2 * cus);
+      else if (rb == 3 && K <= 2048) tiles = wide || K <= 640 || (K <= 1280 && N >= 4 * cus);
+      else tiles = wide || (K > 4096 ? N < 2 * cus : rb == 3 && N >= 2 * cus);
     } else if (vec == 8) {
       tiles = wide && (rb == 4 || (rb == 3 && (K > 2048 || N >= 32 * cus)));
     }

@@ -271,6 +271,7 @@ FP8_SHAPES = [
     (17, 528, 100, 0),
     (40, 2064, 64, 2),
     (33, 48, 20, 0),
+    (33, 1312, 20, 0),
     (1, 16, 1, 0),
     (49, 400, 130, 0),
     # more than 32 column blocks, not a multiple of 32 (63 and 38): the XCD-aware block order

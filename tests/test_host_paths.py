@@ -96,11 +96,11 @@ def fp8_kernel(host, *sizes, x=0):
 
 # Sides of fp8_linear's rule for at most 64 rows: the skinny kernel where its workgroups fit the
 # CUs once (it was up to 25% faster there than the tiles), the tiles beyond.
-FP8_SKINNY = [(33, 2048, 64), (33, 4096, 64), (40, 1024, 4096), (48, 2048, 2048), (64, 1024, 512), (64, 2048, 1024),
+FP8_SKINNY = [(33, 2048, 64), (33, 4096, 64), (40, 2048, 4096), (40, 1536, 1024), (33, 1024, 512), (48, 2048, 2048), (64, 1024, 512), (64, 2048, 1024),
               (64, 4096, 4096), (64, 8192, 512), (64, 7168, 4096), (56, 704, 1600), (63, 3136, 576), (16, 16384, 4096),
               (32, 8192, 4096), (16, 16384, 8192), (8, 4096, 6144), (48, 8192, 520), (33, 4096, 448), (39, 5536, 1568),
               (16, 4088, 8200), (33, 1016, 4104), (33, 2040, 8000), (48, 4088, 4096), (64, 4088, 1024)]
-FP8_TILES = [(33, 4096, 1024), (48, 2064, 512), (48, 8192, 64), (64, 7168, 504), (33, 256, 4112), (64, 256, 4112), (64, 8192, 5120), (17, 256, 5120),
+FP8_TILES = [(40, 1024, 4096), (33, 256, 64), (48, 640, 512), (48, 1280, 1024), (33, 4096, 1024), (48, 2064, 512), (48, 8192, 64), (64, 7168, 504), (33, 256, 4112), (64, 256, 4112), (64, 8192, 5120), (17, 256, 5120),
              (32, 16384, 5120), (1, 256, 7168), (16, 8192, 8192), (16, 16384, 16384), (33, 4088, 4104), (48, 1016, 8200),
              (64, 1016, 4104), (1, 333, 300), (64, 4095, 64), (16, 63, 4096)]
 
@@ -212,6 +212,8 @@ def test_gpu_tests_reach_the_paths_they_name(host):
 
     assert fp8(*special.FP8_KERNELS.values()) == ["skinny_flat", "mid", "mid", "half", "wide"]
     assert set(fp8(*parity.FP8_SHAPES)) == {"skinny_flat", "skinny", "mid", "half", "wide"}
+    three = [c for c in parity.FP8_SHAPES if c[:3] in ((40, 2064, 64), (33, 1312, 20))]
+    assert len(three) == 2 and all("skinny_flatILi3E" in k for k in fp8_kernel(host, *[c[:3] for c in three]))
     assert fp8((70, 0, 72), (2200, 0, 4000), (2000, 0, 4000), (16, 0, 40)) == ["mid", "wide", "half", "skinny_flat"]
     large = graphs.LARGE["fp8_linear"]
     assert fp8((large["M"], large["K"], large["N"])) == ["wide"]
