@@ -14,8 +14,8 @@
 // leaves the operand.
 //
 // Bound: no unit by itself.  At M = 512, K = N = 4096 (64 x 128 tiles, one workgroup per CU) the
-// counters read the MFMAs busy 28 % of a CU's cycles, the LDS 25 % (2 % of that bank
-// conflicts) and the VALU 32 %: what is left is a step's chain of loads, barrier and LDS reads,
+// counters read the MFMAs busy 28 % of a CU's cycles, the LDS 24 % (2 % of that bank
+// conflicts) and the VALU 31 %: what is left is a step's chain of loads, barrier and LDS reads,
 // and the launch.  Measured (us, against the 128 x 256 form): M = 512, K = N = 4096 14.0 / 24.0, M = 256 9.3 / 24.0, M =
 // 1024 19.0 / 24.3; K = 8192, N = 1024, M = 512 13.8 / 41.1.  Against the register-staged 256 x
 // 256 kernel that took other K: M = 333, K = 1000, N = 3000 7.0 / 34.9, M = 1000, K = N = 1001
